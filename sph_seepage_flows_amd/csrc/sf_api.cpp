@@ -129,12 +129,12 @@ int ensure_sort_capacity(sf_system* h, size_t m) {
     if ((rc = h->hist.alloc(256 * nblocks))) return rc;
     if ((rc = h->wpre.alloc(c + 1)) || (rc = h->wpart.alloc((size_t)wprefix_blocks((int)c + 1) + 1)) ||
         (rc = h->plist.alloc(c)) || (rc = h->wflag.alloc(c)) || (rc = h->pph.alloc(c)) || (rc = h->ilist.alloc(c)) ||
-        (rc = h->icount.alloc(2)) || (rc = h->iface.alloc(c)) || (rc = h->wl.alloc(c)) || (rc = h->vq.alloc(c)) || (rc = h->wq.alloc(c)) ||
+        (rc = h->icount.alloc(2 * kCountStride)) || (rc = h->iface.alloc(c)) || (rc = h->wl.alloc(c)) || (rc = h->vq.alloc(c)) || (rc = h->wq.alloc(c)) ||
         (rc = h->xq.alloc(c)) || (rc = h->wbq.alloc(c)) || (rc = h->rec0.alloc(c)) || (rc = h->rec1.alloc(c)))
         return rc;
     // the interface counters start at zero (each step's water momentum pass
     // clears them for the next)
-    SF_HIP(hipMemsetAsync(h->icount.p, 0, 2 * sizeof(uint32_t), h->stream));
+    SF_HIP(hipMemsetAsync(h->icount.p, 0, h->icount.n * sizeof(uint32_t), h->stream));
     if ((rc = h->skeys[0].alloc(c)) || (rc = h->skeys[1].alloc(c)) || (rc = h->sperm.alloc(c)) ||
         (rc = h->slot.alloc(c)) || (rc = h->in_list.alloc(c)) || (rc = h->stay_pre.alloc(c + 1)))
         return rc;

@@ -154,6 +154,7 @@ int wprefix_blocks(int n);
 int vprefix2_partials(int n1, int n2);
 
 // ---- solver launchers (sf_solver.hip) ----
+constexpr int kCountStride = 64;  // words between the two interface counters (a cache line each)
 struct Fields {
     const float4* pm;
     const float4* vr;
@@ -188,7 +189,8 @@ struct Fields {
     // the sand ones pph[nw + s - wpre[s], nw + e - wpre[e])
     const float4* pph;
     // interface particles of the avg-flow / voidage-adhesion passes (phase
-    // indices t): water at ilist[0, icount[0]), sand at ilist[nw, nw + icount[1])
+    // indices t): water at ilist[0, icount[0]), sand at
+    // ilist[nw, nw + icount[kCountStride])
     uint32_t* ilist;
     uint32_t* icount;
     // iface[ts] = 1 when sand particle ts (index among the sand, plist[nw + ts])

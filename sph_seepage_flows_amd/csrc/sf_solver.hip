@@ -342,23 +342,33 @@ SF_DEV void write_no_interface(const Fields& f, int i, bool sand, float2 rpi, co
     }
 }
 // Appends phase index t of every listed lane to its phase's list (water at
-// ilist[0, nw), sand at ilist[nw, n)): one atomic per wave and phase, each
-// listed lane taking its rank among the wave's.  A list never grows past its
-// phase's size (that would take a missed clear of the counters).  Must be
-// called by all lanes of the wave.
+// ilist[0, nw), sand at ilist[nw, n)): one atomic per block and phase, each
+// listed lane taking its rank among the block's.  Atomics on one word pass one
+// after another, about 9 ns each: one per wave (23.4k for 500k + 500k
+// interpenetrating particles, both counters on one cache line) held the
+// density pass of that scene to 288 us, one per block on lines of their own
+// leaves it at 76 us (step 1.26 -> 1.05 ms).  A list never grows past its phase's size (that would
+// take a missed clear of the counters).  Must be called by all threads of the
+// block; `sand` is the same for all lanes of a wave.
+template <int NB>
 SF_DEV void list_interface(const Fields& f, bool listed, bool sand, uint32_t t, uint32_t nw, uint32_t n) {
-    const int lane = (int)(threadIdx.x & 63u);
-    for (int ph = 0; ph < 2; ++ph) {
-        const bool mine = listed && sand == (ph == 1);
-        const uint64_t m = __ballot(mine);
-        if (m == 0) continue;
-        const int leader = __builtin_ctzll(m);
-        uint32_t base = 0;
-        if (lane == leader) base = atomicAdd(f.icount + ph, (uint32_t)__popcll(m));
-        base = (uint32_t)__shfl((int)base, leader, 64);
-        const uint32_t q = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        if (mine && q < (ph ? n - nw : nw)) f.ilist[(ph ? nw : 0u) + q] = t;
+    constexpr int W = NB / 64;
+    __shared__ uint32_t cnt[2][W], base[2];  // listed lanes of each wave, by phase; the block's first entries
+    const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);
+    const uint64_t m = __ballot(listed);
+    if (lane < 2) cnt[lane][w] = (lane == 1) == sand ? (uint32_t)__popcll(m) : 0u;
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        uint32_t c = 0;
+        for (int q = 0; q < W; ++q) c += cnt[threadIdx.x][q];
+        base[threadIdx.x] = c ? atomicAdd(f.icount + threadIdx.x * kCountStride, c) : 0u;
     }
+    __syncthreads();
+    if (!listed) return;
+    const int ph = sand ? 1 : 0;
+    uint32_t q = base[ph] + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    for (int v = 0; v < w; ++v) q += cnt[ph][v];
+    if (q < (sand ? n - nw : nw)) f.ilist[(sand ? nw : 0u) + q] = t;
 }
 
 // ---------------------------------------------------------------------------
@@ -429,7 +439,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
             });
         }
         const bool listed = valid && other != 0u;
-        list_interface(f, listed, true, nw + t, nw, (uint32_t)n);
+        list_interface<NB>(f, listed, true, nw + t, nw, (uint32_t)n);
         if (valid) f.iface[t] = listed ? 1 : 0;
         if (valid) {  // every grain's velocity and saturation by phase index (P2 sets the listed ones' .w)
             const float4 v = ldo(f.vr, (uint32_t)i);
@@ -513,7 +523,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
         sb += __shfl_xor(sb, o);
     }
     const bool listed = water && lead && other != 0u;
-    list_interface(f, listed, false, t, nw, (uint32_t)n);
+    list_interface<NB>(f, listed, false, t, nw, (uint32_t)n);
     if (!water || !lead) return;
     f.wl[t] = listed ? 1 : 0;
     const float rho = pi.w * k.w0 + k.w_coef * (sf + k.rho0 * sb);
@@ -537,14 +547,17 @@ void launch_density(const SFConst& k, const Fields& f, int n, PassCfg c, hipStre
 // k_interface: the interface lists and the empty sums' results, as the
 // density pass leaves them, for a lone avg-flow run.
 __global__ void k_zero_counts(uint32_t* __restrict__ c) {
-    if (threadIdx.x < 2) c[threadIdx.x] = 0u;
+    if (threadIdx.x < 2) c[threadIdx.x * kCountStride] = 0u;
 }
 template <bool B>
 __global__ __launch_bounds__(kBlock) void k_interface(SFConst k, Fields f, int n) {
-    const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
-    const bool valid = t < (uint32_t)n;
-    const uint32_t nw = *f.nwater;
-    const bool sand_i = t >= nw;
+    const uint32_t nw = *f.nwater, ns = (uint32_t)n - nw;
+    const PhaseBlock pb = phase_block((nw + kBlock - 1) / kBlock, (ns + kBlock - 1) / kBlock);
+    if (pb.phase < 0) return;
+    const bool sand_i = pb.phase == 1;
+    const uint32_t u = pb.blk * kBlock + threadIdx.x;  // index within the phase
+    const uint32_t t = (sand_i ? nw : 0u) + u;
+    const bool valid = u < (sand_i ? ns : nw);
     int i = 0;
     uint32_t other = 0;
     float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -562,9 +575,9 @@ __global__ __launch_bounds__(kBlock) void k_interface(SFConst k, Fields f, int n
         });
     }
     const bool listed = valid && other != 0u;
-    list_interface(f, listed, sand_i, t, nw, (uint32_t)n);
-    if (valid && !sand_i) f.wl[t] = listed ? 1 : 0;
-    if (valid && sand_i) f.iface[t - nw] = listed ? 1 : 0;
+    list_interface<kBlock>(f, listed, sand_i, t, nw, (uint32_t)n);
+    if (valid && !sand_i) f.wl[u] = listed ? 1 : 0;
+    if (valid && sand_i) f.iface[u] = listed ? 1 : 0;
     if (valid && !listed) write_no_interface(f, i, sand_i, ldo(f.rp, (uint32_t)i), pi);
 }
 __global__ __launch_bounds__(kBlock) void k_fill_empty(SFConst k, Fields f, int n) {
@@ -582,8 +595,8 @@ void launch_fill_empty(const SFConst& k, const Fields& f, int n, hipStream_t s) 
 }
 void launch_zero_counts(const Fields& f, hipStream_t s) { k_zero_counts<<<1, 64, 0, s>>>(f.icount); }
 void launch_interface(const SFConst& k, const Fields& f, int n, hipStream_t s) {
-    if (f.scene) k_interface<true><<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, f, n);
-    else k_interface<false><<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, f, n);
+    if (f.scene) k_interface<true><<<phase_grid(n, kBlock), kBlock, 0, s>>>(k, f, n);
+    else k_interface<false><<<phase_grid(n, kBlock), kBlock, 0, s>>>(k, f, n);
 }
 
 template <int NB, int LP>
@@ -597,7 +610,7 @@ struct PhaseSlot {
 template <int NB, int LP>
 SF_DEV bool phase_slot(const Fields& f, uint32_t nw, PhaseSlot<NB, LP>& ps) {
     constexpr uint32_t PB = NB / LP;  // particles per block
-    const uint32_t cw = f.icount[0], cs = f.icount[1];
+    const uint32_t cw = f.icount[0], cs = f.icount[kCountStride];
     const PhaseBlock pb = phase_block((cw + PB - 1) / PB, (cs + PB - 1) / PB);
     if (pb.phase < 0) return false;
     ps.sand = pb.phase == 1;
@@ -1003,7 +1016,7 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     float4* stage = stage_lds + (threadIdx.x >> 6) * kWmStage;
     // P2 and P3 have read the interface lists: the next density pass lists
     // into counters that start at zero
-    if (blockIdx.x == 0 && threadIdx.x < 2) f.icount[threadIdx.x] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x < 2) f.icount[threadIdx.x * kCountStride] = 0u;
     constexpr uint32_t PB = NB / kWmL;  // water particles per block
     const uint32_t nw = *f.nwater;
     const PhaseBlock pb = phase_block((nw + PB - 1) / PB, 0u);
