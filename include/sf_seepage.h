@@ -467,7 +467,9 @@ int sf_set_sort_strategy(sf_handle h, int strategy);
 int sf_set_prefix_scan_threshold(int tiles);
 /* Launch shape of a neighbour pass (SF_PASS_DENSITY .. SF_PASS_WATER_MOMENTUM):
  * workgroup size nb in {64, 128, 256}; LDS candidate-list depth cap in {8, 16}
- * (sand / water momentum only).  Results do not depend on the shape. */
+ * (sand / water momentum only).  Results do not depend on the shape.  A pass
+ * whose shape was never set (nor tuned) reports (256, 16) and launches the
+ * workgroup size the library's own rule gives for the handle's particles. */
 int sf_set_launch_config(sf_handle h, int pass, int nb, int cap);
 int sf_get_launch_config(sf_handle h, int pass, int* nb, int* cap);
 /* Lanes per particle (1, 2 or 4; default 4) of the two interface passes

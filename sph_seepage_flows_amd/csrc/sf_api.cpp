@@ -1436,6 +1436,7 @@ int sf_set_launch_config(sf_handle h, int pass, int nb, int cap) {
     PassCfg& c = h->cfg[pass - SF_PASS_DENSITY];
     c.nb = nb;
     c.cap = cap;
+    c.chosen = true;
     h->drop_graph();
     return SF_OK;
 }
@@ -1486,11 +1487,11 @@ int sf_autotune(sf_handle h, int reps, float* best_ms, float* default_ms) {
     for (int q = 0; q < 5; ++q) {
         const bool lists = q >= 3;
         float best = 0.f, dflt = 0.f;
-        PassCfg pick{256, 16, h->cfg[q].lanes};
+        PassCfg pick{256, 16, h->cfg[q].lanes, true};
         for (int nb : kNbChoices)
             for (int cap : kCapChoices) {
                 if (!lists && cap != 16) continue;
-                const PassCfg c{nb, cap, h->cfg[q].lanes};
+                const PassCfg c{nb, cap, h->cfg[q].lanes, true};
                 launch_pass(h, q, c);  // warm-up
                 SF_HIP(hipEventRecord(h->ev0, h->stream));
                 for (int r = 0; r < reps; ++r) launch_pass(h, q, c);

@@ -241,6 +241,9 @@ struct PassCfg {
     int nb = 256;
     int cap = 16;
     int lanes = 4;  // lanes per particle (interface passes P2, P3)
+    // the shape was set (sf_set_launch_config, sf_autotune); a pass left alone
+    // launches the workgroup size its own rule gives
+    bool chosen = false;
 };
 constexpr int kNbChoices[3] = {64, 128, 256};
 constexpr int kCapChoices[2] = {8, 16};

@@ -76,18 +76,13 @@ SF_DEV void filter_push(NList<NB, CAP>& L, const float4* __restrict__ pm, uint32
     }
 }
 
-// Phase-index ranges of one phase over the 9 neighbour columns, in the order
-// of for_columns: a column's slot range [s, e) holds the water candidates
-// pph[wpre[s], wpre[e]) and the sand candidates pph[nw + s - wpre[s],
-// nw + e - wpre[e]), each in slot order (the cell table holds both ends).
-template <class F>
-SF_DEV void for_phase_ranges(const SFConst& k, const Fields& f, uint32_t cb, int cx, int cy, int cz, bool water,
-                             uint32_t nw, F&& fn) {
-    for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
-        const uint2 a = ldo(f.ct, cb + c0), b = ldo(f.ct, cb + c1);
-        const uint32_t t0 = water ? a.y : nw + (a.x - a.y), t1 = water ? b.y : nw + (b.x - b.y);
-        if (t0 < t1) fn(t0, t1);
-    });
+// Phase-index range of one phase in the cells [c0, c1) of a column: a slot
+// range [s, e) holds the water candidates pph[wpre[s], wpre[e]) and the sand
+// candidates pph[nw + s - wpre[s], nw + e - wpre[e]), each in slot order (the
+// cell table holds both ends).
+SF_DEV uint2 phase_range(const uint2* __restrict__ ct, uint32_t c0, uint32_t c1, bool water, uint32_t nw) {
+    const uint2 a = ldo(ct, c0), b = ldo(ct, c1);
+    return water ? make_uint2(a.y, b.y) : make_uint2(nw + (a.x - a.y), nw + (b.x - b.y));
 }
 
 SF_DEV float sq3(float d) { return d * d * d; }
@@ -156,8 +151,8 @@ SF_DEV void staged_walk(const SFConst& k, const Fields& f, float4* __restrict__ 
                 const uint32_t base = scb + (uint32_t)((x * k.gy + y) * k.gz);
                 uint2 a = make_uint2(0u, 0u), b = make_uint2(0u, 0u);
                 if (mine) {
-                    a = ldo(f.ct, base + (uint32_t)zlo);
-                    b = ldo(f.ct, base + (uint32_t)zhi + 1u);
+                    a = ldo(f.ct + base, (uint32_t)zlo);
+                    b = ldo(f.ct + base, (uint32_t)zhi + 1u);
                     range(a, b);
                 }
                 const uint32_t ax = Water ? a.y : a.x, bx = Water ? b.y : b.x;
@@ -189,23 +184,38 @@ SF_DEV void staged_walk(const SFConst& k, const Fields& f, float4* __restrict__ 
     }
 }
 
-// The filtered walk of the water momentum pass: every candidate j of the
-// particle's 9 column ranges with test(pm[j]) goes to the lane's list, lane
-// sub (of S per particle) taking j = s + sub + S m of each range [s, e) in
-// increasing j, exactly as filter_push over the ranges.  The filter is bound
-// by the texture address unit, which costs the same per wave load
+// The filtered walk of the passes: every candidate j of the particle's 9
+// column ranges with test(src[j]) goes to the lane's list, lane sub (of S per
+// particle) taking j = s + sub + S m of each range [s, e) in increasing j,
+// exactly as filter_push over the ranges.  range(b, c0, c1) gives an active
+// lane's [s, e) in src for the cells [b + c0, b + c1) of a column.  The filter is
+// bound by the texture address unit, which costs the same per wave load
 // instruction whatever it carries, so where the wave's ranges overlap it
-// loads them once: when every particle of the wave sits in one grid column
-// (most waves of an ordered region), the lanes walk the same 9 columns, and
-// a column whose union range (first lane's start to last lane's end) fits
-// KS candidates is staged in LDS with coalesced loads (one per lane up to
-// 64) and filtered from there.  Other columns, and waves spread over several columns, filter from
-// memory per lane.  Either way a lane's list gets the same entries in the
-// same order, so which way a column goes does not change the sums.  Must be
-// called by all lanes of the wave.
-template <uint32_t S, uint32_t KS, int NB, int CAP, class Test, class Fetch, class Apply>
-SF_DEV void column_filter(const SFConst& k, const Fields& f, float4* __restrict__ stage, bool active, uint32_t cb,
-                          int cx, int cy, int cz, NList<NB, CAP>& L, Test&& test, Fetch&& fetch, Apply&& apply) {
+// loads them once: when every particle of the wave sits in one grid column,
+// its lanes in cell order (most waves of an ordered region), the lanes walk
+// the same 9 columns, and a column whose union range (first lane's start to
+// last lane's end) fits KS candidates is staged in LDS with coalesced loads
+// (one per lane up to 64) and filtered from there.  Other columns, and waves
+// spread over several columns, filter from memory per lane.  Either way a
+// lane's list gets the same entries in the same order, so which way a column
+// goes does not change the sums.  Must be called by all lanes of the wave.
+// P2, P3 and P4's water walk stage the other phase's candidates (P2 216 ->
+// 200 us, P3 216 -> 203, P4 176 -> 155 at 500k + 500k interpenetrating; where
+// little is listed, the stage's LDS leaves fewer of the waves that find
+// nothing resident: 2 x 4 us of 1.12 ms at 4M).
+constexpr uint32_t kStageList = 64;  // longest union range staged per wave: P2, P3, P4's water
+// P5's candidates are both phases': 16 water particles span 2-3 cells, so the
+// union is 4-5 cells of 8 water particles, or of 16 particles where the
+// phases interpenetrate (64-80).  96 instead of 64: P5 255 -> 227 us at 500k +
+// 500k interpenetrating, 137 -> 138 us where they are apart.
+constexpr uint32_t kStageWm = 96;
+#define SF_STAGE(name, KS)                              \
+    __shared__ float4 name##_lds[(NB / 64) * (KS)];     \
+    float4* name = name##_lds + (threadIdx.x >> 6) * (KS)
+template <uint32_t S, uint32_t KS, int NB, int CAP, class Range, class Test, class Fetch, class Apply>
+SF_DEV void column_filter(const SFConst& k, const float4* __restrict__ src, float4* __restrict__ stage, bool active,
+                          uint32_t cb, int cx, int cy, int cz, NList<NB, CAP>& L, Range&& range, Test&& test,
+                          Fetch&& fetch, Apply&& apply) {
     static_assert(CAP >= 4, "a round pushes up to four candidates");
     static_assert(KS <= 128, "at most two staged candidates per lane");
     const int lane = (int)(threadIdx.x & 63u);
@@ -214,24 +224,46 @@ SF_DEV void column_filter(const SFConst& k, const Fields& f, float4* __restrict_
     if (!act) return;
     const int lead = __builtin_ctzll(act), last = 63 - __builtin_clzll(act);
     const uint32_t col = cb + (uint32_t)((cx * k.gy + cy) * k.gz);
-    const bool one = !__ballot(active && col != lane_value(col, lead));  // wave-uniform
-    if (!one && !active) return;
-    // lanes without a particle follow the lead's columns (with empty ranges)
-    const int wx = active ? cx : lane_value(cx, lead), wy = active ? cy : lane_value(cy, lead);
-    const int wz = active ? cz : lane_value(cz, lead);
-    for_columns(k, wx, wy, wz, [&](uint32_t c0, uint32_t c1) {
-        const uint32_t rs = active ? ldo(f.ct, cb + c0).x : 0u, re = active ? ldo(f.ct, cb + c1).x : 0u;
-        if (one) {
-            const uint32_t us = lane_value(rs, lead), ue = lane_value(re, last);
-            if (us >= ue) return;
+    const uint32_t zlo = (uint32_t)(cz > 0 ? cz - 1 : 0), zhi = (uint32_t)(cz + 1 < k.gz ? cz + 1 : k.gz - 1);
+    const bool one = !__ballot(active && (col != lane_value(col, lead) || cz < lane_value(cz, lead) ||
+                                          cz > lane_value(cz, last)));  // wave-uniform
+    if (!one) {
+        if (!active) return;
+        for (int dx = -1; dx <= 1; ++dx) {
+            const int x = cx + dx;
+            if (x < 0 || x >= k.gx) continue;
+            for (int dy = -1; dy <= 1; ++dy) {
+                const int y = cy + dy;
+                if (y < 0 || y >= k.gy) continue;
+                const uint2 r = range(0u, cb + (uint32_t)((x * k.gy + y) * k.gz) + zlo,
+                                      cb + (uint32_t)((x * k.gy + y) * k.gz) + zhi + 1u);
+                filter_push<S>(L, src, r.x + sub, r.y, test, fetch, apply);
+            }
+        }
+        return;
+    }
+    // one column: its coordinates, the bounds checks and the columns' first
+    // cells are the wave's (scalar registers and arithmetic)
+    const int sx = lane_value(cx, lead), sy = lane_value(cy, lead);
+    const uint32_t scb = lane_value(cb, lead);
+    for (int dx = -1; dx <= 1; ++dx) {
+        const int x = sx + dx;
+        if (x < 0 || x >= k.gx) continue;
+        for (int dy = -1; dy <= 1; ++dy) {
+            const int y = sy + dy;
+            if (y < 0 || y >= k.gy) continue;
+            uint2 r = make_uint2(0u, 0u);
+            if (active) r = range(scb + (uint32_t)((x * k.gy + y) * k.gz), zlo, zhi + 1u);
+            const uint32_t us = lane_value(r.x, lead), ue = lane_value(r.y, last);
+            if (us >= ue) continue;
             if (ue - us <= KS) {
-                for (uint32_t q = (uint32_t)lane; q < ue - us; q += 64u) stage[q] = ldo(f.pm, us + q);
+                for (uint32_t q = (uint32_t)lane; q < ue - us; q += 64u) stage[q] = ldo(src + us, q);
                 wave_sync();
-                uint32_t j = rs + sub;
-                for (; j + 3u * S < re; j += 4u * S) {
+                uint32_t j = r.x + sub;
+                for (; j + 3u * S < r.y; j += 4u * S) {
                     const float4 a = stage[j - us], b = stage[j + S - us], c = stage[j + 2u * S - us],
                                  d = stage[j + 3u * S - us];
-                    const bool ka = test(a), kb = test(b), kc = test(c), kd = test(d);
+                    const bool ka = test(j, a), kb = test(j + S, b), kc = test(j + 2u * S, c), kd = test(j + 3u * S, d);
                     if (__ballot(L.cnt >= CAP)) nl_flush2(L, fetch, apply);
                     L.slot[L.cnt * NB] = j;
                     L.cnt += ka ? 1 : 0;
@@ -242,14 +274,13 @@ SF_DEV void column_filter(const SFConst& k, const Fields& f, float4* __restrict_
                     L.slot[L.cnt * NB] = j + 3u * S;
                     L.cnt += kd ? 1 : 0;
                 }
-                for (; j < re; j += S) nl_push2(L, test(stage[j - us]), j, fetch, apply);
+                for (; j < r.y; j += S) nl_push2(L, test(j, stage[j - us]), j, fetch, apply);
                 wave_sync();
-                return;
+            } else if (active) {
+                filter_push<S>(L, src, r.x + sub, r.y, test, fetch, apply);
             }
         }
-        if (active)
-            filter_push<S>(L, f.pm, rs + sub, re, [&](uint32_t, const float4& pj) { return test(pj); }, fetch, apply);
-    });
+    }
 }
 
 // Lanes per particle of the interface passes (P2, P3), whose work sits at the
@@ -606,14 +637,17 @@ struct PhaseSlot {
     uint32_t sub;  // its lane among LP
     bool sand;
 };
-// The listed particle of this thread (false: none).
+// The listed particle of this thread (false: none; slot and phase index 0
+// then, the phase still the block's).
 template <int NB, int LP>
 SF_DEV bool phase_slot(const Fields& f, uint32_t nw, PhaseSlot<NB, LP>& ps) {
     constexpr uint32_t PB = NB / LP;  // particles per block
     const uint32_t cw = f.icount[0], cs = f.icount[kCountStride];
     const PhaseBlock pb = phase_block((cw + PB - 1) / PB, (cs + PB - 1) / PB);
-    if (pb.phase < 0) return false;
+    ps.i = 0;
+    ps.t = 0;
     ps.sand = pb.phase == 1;
+    if (pb.phase < 0) return false;
     const uint32_t q = pb.blk * PB + threadIdx.x / LP;
     ps.sub = threadIdx.x % LP;
     if (q >= (ps.sand ? cs : cw)) return false;
@@ -638,9 +672,11 @@ inline int phase_slot_grid(int n, int lanes, int nb) { return phase_grid(n * lan
 template <bool B, int NB, int CAP, int LP>
 __global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
     SF_NLIST(L);
+    SF_STAGE(stage, kStageList);
     const uint32_t nw = *f.nwater;
     PhaseSlot<NB, LP> ps;
-    if (!phase_slot(f, nw, ps)) return;
+    const bool active = phase_slot(f, nw, ps);
+    if (!__ballot(active)) return;  // the other lanes of a wave help to stage its candidates
     const int i = ps.i;
     const uint32_t sub = ps.sub;
     const bool sand_i = ps.sand;
@@ -673,10 +709,11 @@ __global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
         av += xyz(q.vj) * vw;
         vsum += vw;
     };
-    for_phase_ranges(k, f, cb, cx, cy, cz, sand_i, nw, [&](uint32_t t0, uint32_t t1) {
-        filter_push<LP>(L, f.pph, t0 + sub, t1, in_range, fetch, pair);
-    });
+    column_filter<LP, kStageList>(
+        k, f.pph, stage, active, cb, cx, cy, cz, L,
+        [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, sand_i, nw); }, in_range, fetch, pair);
     nl_flush2(L, fetch, pair);
+    if (!active) return;
     sandv = lane_sum<LP>(sandv);
     vsum = lane_sum<LP>(vsum);
     av = mk3(lane_sum<LP>(av.x), lane_sum<LP>(av.y), lane_sum<LP>(av.z));
@@ -711,9 +748,11 @@ void launch_avg_flow(const SFConst& k, const Fields& f, int n, PassCfg c, hipStr
 template <bool B, int NB, int CAP, int LP>
 __global__ __launch_bounds__(NB) void k_voidage_adhesion(SFConst k, Fields f, int n) {
     SF_NLIST(L);
+    SF_STAGE(stage, kStageList);
     const uint32_t nw = *f.nwater;
     PhaseSlot<NB, LP> ps;
-    if (!phase_slot(f, nw, ps)) return;
+    const bool active = phase_slot(f, nw, ps);
+    if (!__ballot(active)) return;
     const int i = ps.i;
     const uint32_t sub = ps.sub;
     const float4 pi = ldo(f.pm, (uint32_t)i);
@@ -745,10 +784,11 @@ __global__ __launch_bounds__(NB) void k_voidage_adhesion(SFConst k, Fields f, in
             num += q.x.y * vw;
             den += vw;
         };
-        for_phase_ranges(k, f, cb, cx, cy, cz, true, nw, [&](uint32_t t0, uint32_t t1) {
-            filter_push<LP>(L, f.pph, t0 + sub, t1, in_range, fetch, pair);
-        });
+        column_filter<LP, kStageList>(
+            k, f.pph, stage, active, cb, cx, cy, cz, L,
+            [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); }, in_range, fetch, pair);
         nl_flush2(L, fetch, pair);
+        if (!active) return;
         num = lane_sum<LP>(num);
         den = lane_sum<LP>(den);
         if (sub != 0) return;
@@ -774,10 +814,11 @@ __global__ __launch_bounds__(NB) void k_voidage_adhesion(SFConst k, Fields f, in
             F += dp * (G * mi * mj * A * frcp(fmaxf(kEps, l)));
         }
     };
-    for_phase_ranges(k, f, cb, cx, cy, cz, false, nw, [&](uint32_t t0, uint32_t t1) {
-        filter_push<LP>(L, f.pph, t0 + sub, t1, in_range, fetch, pair);
-    });
+    column_filter<LP, kStageList>(
+        k, f.pph, stage, active, cb, cx, cy, cz, L,
+        [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, false, nw); }, in_range, fetch, pair);
     nl_flush2(L, fetch, pair);
+    if (!active) return;
     vs = lane_sum<LP>(vs);
     F = mk3(lane_sum<LP>(F.x), lane_sum<LP>(F.y), lane_sum<LP>(F.z));
     if (sub != 0) return;
@@ -821,16 +862,19 @@ constexpr int kSmL = 2;  // lanes per sand particle (as in the water momentum pa
 template <bool B, int NB, int CAP>
 __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n) {
     SF_NLIST(L);
+    SF_STAGE(stage, kStageList);
     constexpr uint32_t PB = NB / kSmL;  // sand particles per block
     const uint32_t nw = *f.nwater, ns = (uint32_t)n - nw;
     const PhaseBlock pb = phase_block(0u, (ns + PB - 1) / PB);
     const uint32_t t = pb.blk * PB + threadIdx.x / kSmL;
     const uint32_t sub = threadIdx.x % kSmL;  // this lane's share of the particle's candidates
-    if (pb.phase < 0 || t >= ns) return;
-    const int i = (int)ldo(f.plist, nw + t);
+    if (pb.phase < 0) return;  // the whole block
+    // lanes past the last grain help to stage their wave's water candidates
+    const int i = t < ns ? (int)ldo(f.plist, nw + t) : 0;
     const uint32_t self = nw + t;  // this particle's phase index
     const float4 pi = ldo(f.pm, (uint32_t)i);
-    if (pi.w >= 0.f) return;
+    const bool active = t < ns && pi.w < 0.f;
+    if (!__ballot(active)) return;
     const uint32_t cb = scene_base<B>(k, f, i);
     if constexpr (B) {  // the scene's friction, capillary curve and drag coefficient
         const SceneConst sc = f.sct[ldo(f.scene, (uint32_t)i)];
@@ -872,7 +916,7 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
             if (H > 0.f && H < k.cap_srup) fsum += capillary(k, dji, dist, H, (sat_i + q.vj.w) * 0.5f);
         }
     };
-    {
+    if (active) {
         const float rcm = cap_r + 1e-3f * k.h;  // conservative against FP32 cell edges
         int xa, xb, ya, yb, za, zb;
         near_span(pi.x, k.lox, k.h, cx, k.gx, rcm, xa, xb);
@@ -915,16 +959,18 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
     };
     // a grain with no water in its 9 column ranges (the density pass flagged
     // the others) has nothing to walk
-    if (ldo(f.iface, t)) {
-        for_phase_ranges(k, f, cb, cx, cy, cz, true, nw, [&](uint32_t t0, uint32_t t1) {
-            filter_push<kSmL>(L, f.pph, t0 + sub, t1, [&](uint32_t, const float4& pj) {
-                const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-                const float r2 = dx * dx + dy * dy + dz * dz;
-                return r2 < k.h2;
-            }, fetch_water, water);
-        });
-    }
+    const bool wet = active && ldo(f.iface, t);
+    column_filter<kSmL, kStageList>(
+        k, f.pph, stage, wet, cb, cx, cy, cz, L,
+        [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); },
+        [&](uint32_t, const float4& pj) {
+            const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+            const float r2 = dx * dx + dy * dy + dz * dz;
+            return r2 < k.h2;
+        },
+        fetch_water, water);
     nl_flush2(L, fetch_water, water);
+    if (!active) return;
     if (k.blabel1 && ldo(f.bnear, cell_key(k, cx, cy, cz))) {  // ComputeSFUniRadiusDemBoundaryForces: label 1 only
         for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
             const uint32_t be = ldo(f.bcell, c1);
@@ -973,6 +1019,10 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
 }
 void launch_sand_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
     if (n <= 0) return;
+    // one wave per workgroup unless the shape was set: no wave's LDS and slot
+    // wait for the slowest of four (15.1 -> 13.6 us at 24k, 71 -> 69 at 1M
+    // apart, 158 -> 150 interpenetrating, 255 -> 255 at 4M)
+    if (!c.chosen) c.nb = 64;
     dispatch(f, c, [&](auto B, auto NB, auto CAP) {
         k_sand_momentum<decltype(B)::value, decltype(NB)::value, decltype(CAP)::value>
             <<<phase_grid(n * kSmL, NB), (int)NB, 0, s>>>(k, f, n);
@@ -986,7 +1036,6 @@ void launch_sand_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, h
 // its own list (column_filter, which stages the candidates in LDS where the
 // wave's ranges overlap), and the partial sums are combined with shuffles.
 constexpr int kWmL = 4;
-constexpr uint32_t kWmStage = 64;  // longest union range staged per wave
 // A neighbour's data in the water momentum pass: r0 = (position, w) with
 // w > 0 for water, w = -mass for sand.  WmRecords reads the two records
 // (Fields::rec0; every water particle has mass f.mw); WmSlots reads the
@@ -1012,8 +1061,7 @@ struct WmSlots {
 template <bool B, class Nbr, int NB, int CAP>
 __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int n) {
     SF_NLIST(L);
-    __shared__ float4 stage_lds[(NB / 64) * kWmStage];
-    float4* stage = stage_lds + (threadIdx.x >> 6) * kWmStage;
+    SF_STAGE(stage, kStageWm);
     // P2 and P3 have read the interface lists: the next density pass lists
     // into counters that start at zero
     if (blockIdx.x == 0 && threadIdx.x < 2) f.icount[threadIdx.x * kCountStride] = 0u;
@@ -1068,12 +1116,15 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     };
     // the particle's own slot passes too: d = 0 makes its term exactly zero
     // (the spiky factor is 0 below r = eps), and acc adds g afterwards
-    auto in_range = [&](const float4& pj) {
+    auto in_range = [&](uint32_t, const float4& pj) {
         const float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         const float r2 = dx * dx + dy * dy + dz * dz;
         return r2 < k.h2;
     };
-    column_filter<kWmL, kWmStage>(k, f, stage, active, cb, cx, cy, cz, L, in_range, fetch, pair);
+    column_filter<kWmL, kStageWm>(
+        k, f.pm, stage, active, cb, cx, cy, cz, L,
+        [&](uint32_t b, uint32_t c0, uint32_t c1) { return make_uint2(ldo(f.ct + b, c0).x, ldo(f.ct + b, c1).x); },
+        in_range, fetch, pair);
     nl_flush2(L, fetch, pair);
     if (!active) return;
     if (ldo(f.bnear, cell_key(k, cx, cy, cz))) {  // boundary particles within the 27 cells
@@ -1106,6 +1157,12 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
 }
 void launch_water_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
     if (n <= 0) return;
+    // one wave per workgroup, as in the sand momentum pass, up to kWmOneWave
+    // particles (24.7 -> 20.4 us at 24k, 134.5 -> 128 at 1M, 169 -> 168 at
+    // 2M); above, neighbouring waves on one CU share more of its L1 than they
+    // wait for each other (4M: 335 us with 256 threads, 354 with 64)
+    constexpr int kWmOneWave = 2 << 20;
+    if (!c.chosen && n <= kWmOneWave) c.nb = 64;
     dispatch(f, c, [&](auto B, auto NB, auto CAP) {
         constexpr bool b = decltype(B)::value;
         constexpr int nb = decltype(NB)::value, cap = decltype(CAP)::value;
