@@ -50,18 +50,17 @@ def pass_bytes(n_w: int, n_s: int, nb: int, cells: int, multi: bool, listed=(0, 
     aux = 24 if multi else 0
     lw, ls = listed
     return {
-        # stepping loop: the advect computes the next keys (below), the stable
-        # sort is the incremental one (change flags and both prefixes, the
-        # newcomer lists, the placement: keys, prefixes, permutation, sorted
-        # keys; per cell the newcomer counts and starts)
-        "sort": n * 44 + 12 * (cells + 1),
-        # perm, persistent state read by perm and written, water flag; the
-        # water prefix then reads the flags and writes prefix + phase list
-        "gather": n * (4 + 2 * (48 + aux) + 1) + n * (1 + 4 + 4),
-        # per cell: old start, stayer / newcomer prefixes, water prefix read,
-        # cellStart, (start, prefix) table and newcomer counter written; per
-        # particle: phase list + position read, position in phase order written
-        "cell_start": (cells + 1) * (16 + 16) + n * (4 + 16 + 16),
+        # stepping loop: the advect computes the next keys and counts the
+        # moves (below).  The prefixes read both keys and the water flag and
+        # write the packed stay prefix, per cell the newcomer counts; the
+        # placement reads the keys and the prefix, reads and writes the
+        # persistent state and writes permutation, keys, flag, phase list and
+        # the positions in phase order; per cell the old table, the newcomer
+        # prefix and the chain head are read, the new tables and the cleared
+        # counters written.
+        "sort": n * (4 + 4 + 1 + 8 + 4 + 4 + 8 + 2 * (48 + aux) + 4 + 4 + 1 + 4 + 16) + (cells + 1) * (8 + 8 + 8 + 8 + 4 + 24),
+        "gather": 0,  # within the placement, as the cell table
+        "cell_start": 0,
         # plist, own position (water: pm, sand: pph), water candidates' pph, rho/p (water);
         # sand: position record, velocity read and written in phase order;
         # unlisted water: velocity read, both records written; unlisted

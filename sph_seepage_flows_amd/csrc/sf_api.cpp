@@ -118,6 +118,12 @@ using namespace sf;
 
 namespace sf {
 
+template <class T>
+int zero(sf_system* h, DevBuf<T>& b) {
+    SF_HIP(hipMemsetAsync(b.p, 0, b.n * sizeof(T), h->stream));
+    return SF_OK;
+}
+
 int ensure_sort_capacity(sf_system* h, size_t m) {
     if (m <= h->sort_cap && h->kA.p) return SF_OK;
     size_t c = std::max<size_t>(m, 1);
@@ -136,7 +142,7 @@ int ensure_sort_capacity(sf_system* h, size_t m) {
     // clears them for the next)
     SF_HIP(hipMemsetAsync(h->icount.p, 0, h->icount.n * sizeof(uint32_t), h->stream));
     if ((rc = h->skeys[0].alloc(c)) || (rc = h->skeys[1].alloc(c)) || (rc = h->sperm.alloc(c)) ||
-        (rc = h->slot.alloc(c)) || (rc = h->in_list.alloc(c)) || (rc = h->stay_pre.alloc(c + 1)))
+        (rc = h->next.alloc(c)) || (rc = h->stay_pre.alloc(c + 1)))
         return rc;
     h->sort_cap = c;
     return ensure_cell_capacity(h);
@@ -148,18 +154,16 @@ int ensure_cell_capacity(sf_system* h) {
     const size_t C1 = (size_t)h->C + 1;
     int rc;
     if (h->in_count.n < C1) {
-        if ((rc = h->in_count.alloc(C1)) || (rc = h->in_start.alloc(C1))) return rc;
-        // zero before the first incremental sort; afterwards every cell-start pass clears it
-        SF_HIP(hipMemsetAsync(h->in_count.p, 0, C1 * sizeof(uint32_t), h->stream));
+        if ((rc = h->in_count.alloc(C1)) || (rc = h->in_start.alloc(C1)) || (rc = h->head[0].alloc(C1)) ||
+            (rc = h->head[1].alloc(C1)))
+            return rc;
+        // zero before the first incremental sort; afterwards every build clears them
+        if ((rc = zero(h, h->in_count)) || (rc = zero(h, h->head[0])) || (rc = zero(h, h->head[1]))) return rc;
     }
-    const size_t np = (size_t)vprefix2_partials((int)h->sort_cap, (int)h->C);
-    if (h->part2.n < np && (rc = h->part2.alloc(np))) return rc;
-    return SF_OK;
-}
-
-template <class T>
-int zero(sf_system* h, DevBuf<T>& b) {
-    SF_HIP(hipMemsetAsync(b.p, 0, b.n * sizeof(T), h->stream));
+    const size_t np = (size_t)inc_parts((int)h->sort_cap, h->C);
+    if (h->part2.n < np) {
+        if ((rc = h->part2.alloc(np)) || (rc = zero(h, h->part2))) return rc;
+    }
     return SF_OK;
 }
 
@@ -170,27 +174,12 @@ int zero(sf_system* h, DevBuf<T>& b) {
 int build_neighbors(sf_system* h, hipEvent_t* ev) {
     const int n = (int)h->n;
     hipStream_t s = h->stream;
-    const bool inc = h->sort_inc && h->built && h->sorted_keys;
-    const bool fused = inc && h->keys_fresh;  // the last advect hashed and flagged
+    const bool inc = h->sort_inc && h->built && h->sorted_keys && n > 0;
+    const bool fused = inc && h->keys_fresh;  // the last advect hashed and counted the moves
     h->keys_fresh = false;
     SF_MARK(ev, SF_PASS_HASH);
-    if (!fused) launch_hash(h->K, h->pm[h->cur].p, h->nscenes ? h->scene.p : nullptr, h->keys.p, n, s);
-    SortBuffers sb{h->kA.p, h->vA.p, h->kB.p, h->vB.p, h->hist.p};
-    SF_MARK(ev, SF_PASS_SORT);
-    if (inc) {
-        // the particles are in the last sort's order: rebuild the stable sort
-        // from the previous keys and cellStart
-        uint32_t* out = h->sorted_keys == h->skeys[0].p ? h->skeys[1].p : h->skeys[0].p;
-        IncSortBuffers ib{h->in_count.p, h->in_start.p, h->slot.p, h->in_list.p, h->stay_pre.p, h->part2.p};
-        launch_incremental_sort(h->keys.p, h->sorted_keys, h->cell.p, n, h->C, ib, h->sperm.p, out, fused, s);
-        h->sorted_keys = out;
-        h->perm = h->sperm.p;
-    } else {
-        int rc = radix_sort(h->keys.p, n, h->plan, sb, &h->sorted_keys, &h->perm, s);
-        if (rc) return rc;
-    }
+    if (!fused) launch_hash(h->K, h->pm[h->cur].p, h->nscenes ? h->scene.p : nullptr, h->keys.p, h->wflag.p, n, s);
     GatherArgs g;
-    g.perm = h->perm;
     g.pm_in = h->pm[h->cur].p;
     g.vr_in = h->vr[h->cur].p;
     g.cs_in = h->cs[h->cur_cs].p;
@@ -203,13 +192,51 @@ int build_neighbors(sf_system* h, hipEvent_t* ev) {
     g.amc_out = h->amc[h->cur_aux ^ 1].p;
     g.wflag = h->wflag.p;
     g.multi = h->K.multi;
-    SF_MARK(ev, SF_PASS_GATHER);
-    launch_gather_wprefix(g, n, h->wpart.p, h->wpre.p, h->plist.p, s);
-    SF_MARK(ev, SF_PASS_CELL_START);
-    launch_cell_start(h->sorted_keys, n, h->C, h->wpre.p, h->cell.p, h->ct.p, h->in_count.p,
-                      PhasePos{h->plist.p, g.pm_out, h->pph.p},
-                      // the incremental sort wrote stay_pre and in_start only for n > 0
-                      inc && n > 0 ? IncStart{h->stay_pre.p, h->in_start.p} : IncStart{nullptr, nullptr}, s);
+    SF_MARK(ev, SF_PASS_SORT);
+    if (inc) {
+        // the particles are in the last sort's order: rebuild the stable sort
+        // from the previous keys and cell table, and reorder
+        uint32_t* out = h->sorted_keys == h->skeys[0].p ? h->skeys[1].p : h->skeys[0].p;
+        PlaceArgs a;
+        a.g = g;
+        a.g.perm = nullptr;
+        a.key = h->keys.p;
+        a.old_key = h->sorted_keys;
+        a.wflag_in = h->wflag.p;
+        a.ct_old = h->ct[h->cur_ct].p;
+        a.stay_pre = h->stay_pre.p;
+        a.in_start = h->in_start.p;
+        a.in_count = h->in_count.p;
+        a.head = h->head[h->cur_ct].p;
+        a.next = h->next.p;
+        a.head_next = h->head[h->cur_ct ^ 1].p;
+        a.part = h->part2.p;
+        a.parts = inc_parts(n, h->C);
+        a.perm = h->sperm.p;
+        a.sorted_keys = out;
+        a.plist = h->plist.p;
+        a.pph = h->pph.p;
+        a.cell = h->cell.p;
+        a.ct = h->ct[h->cur_ct ^ 1].p;
+        a.nwater = h->wpre.p + n;
+        launch_incremental_sort(a, h->newcomers(), n, h->C, fused, s);
+        h->sorted_keys = out;
+        h->perm = h->sperm.p;
+        h->cur_ct ^= 1;
+        SF_MARK(ev, SF_PASS_GATHER);  // the placement reorders and writes the cell table too
+        SF_MARK(ev, SF_PASS_CELL_START);
+    } else {
+        SortBuffers sb{h->kA.p, h->vA.p, h->kB.p, h->vB.p, h->hist.p};
+        int rc = radix_sort(h->keys.p, n, h->plan, sb, &h->sorted_keys, &h->perm, s);
+        if (rc) return rc;
+        g.perm = h->perm;
+        SF_MARK(ev, SF_PASS_GATHER);
+        launch_gather_wprefix(g, n, h->wpart.p, h->wpre.p, h->plist.p, s);
+        SF_MARK(ev, SF_PASS_CELL_START);
+        launch_cell_start(h->sorted_keys, n, h->C, h->wpre.p, h->cell.p, h->ct[h->cur_ct].p,
+                          PhasePos{h->plist.p, g.pm_out, h->pph.p},
+                          IncClear{h->in_count.p, h->head[h->cur_ct].p, h->part2.p, inc_parts(n, h->C)}, s);
+    }
     h->cur ^= 1;
     h->cur_cs ^= 1;
     if (h->K.multi) h->cur_aux ^= 1;
@@ -257,8 +284,7 @@ int advect(sf_system* h, float dt, const CflOut* dt_dev, hipEvent_t* ev) {
     const bool fuse = h->sort_inc && h->built && h->sorted_keys && !h->pm_shared;
     a.keys_out = fuse ? h->keys.p : nullptr;
     a.old_keys = h->sorted_keys;
-    a.in_count = h->in_count.p;
-    a.slot = h->slot.p;
+    a.nc = h->newcomers();
     a.scene = h->nscenes ? h->scene.p : nullptr;
     launch_advect(h->K, a, (int)h->n, s);
     h->keys_fresh = fuse;
@@ -375,9 +401,10 @@ static ViewArgs view_args(sf_system* h, uint32_t bits) {
 
 int drop_fresh_keys(sf_system* h) {
     if (!h->keys_fresh) return SF_OK;
-    // the last advect hashed the next build's keys and took the newcomers'
-    // ranks in in_count; the next build hashes and ranks again from zero
-    SF_HIP(hipMemsetAsync(h->in_count.p, 0, h->in_count.n * sizeof(uint32_t), h->stream));
+    // the last advect hashed the next build's keys and counted the particles
+    // that change cell; the next build hashes and counts again from zero
+    int rc;
+    if ((rc = zero(h, h->in_count)) || (rc = zero(h, h->head[h->cur_ct])) || (rc = zero(h, h->part2))) return rc;
     h->keys_fresh = false;
     return SF_OK;
 }
@@ -545,7 +572,8 @@ int sf_create(const sf_params* p, const sf_boundary_params* b, const sf_solver_o
         (rc = h->xf.alloc(c)) || (rc = h->acc.alloc(c)))
         return bail(rc);
     if ((rc = h->cell.alloc((size_t)h->C + 1)) || (rc = h->bcell.alloc((size_t)h->local_cells() + 1)) ||
-        (rc = h->bnear.alloc((size_t)h->local_cells())) || (rc = h->ct.alloc((size_t)h->C + 1)))
+        (rc = h->bnear.alloc((size_t)h->local_cells())) || (rc = h->ct[0].alloc((size_t)h->C + 1)) ||
+        (rc = h->ct[1].alloc((size_t)h->C + 1)))
         return bail(rc);
     if ((rc = h->cfl_part.alloc(cfl_partials(0))) || (rc = h->cfl_out.alloc(1)) ||
         (rc = h->frame_dev.alloc(1)))
@@ -561,7 +589,7 @@ int sf_create(const sf_params* p, const sf_boundary_params* b, const sf_solver_o
     if ((rc = zero(h, h->rp)) || (rc = zero(h, h->es)) || (rc = zero(h, h->flow)) || (rc = zero(h, h->adh)) ||
         (rc = zero(h, h->xf)) || (rc = zero(h, h->acc)) || (rc = zero(h, h->cell)) || (rc = zero(h, h->bcell)) ||
         (rc = zero(h, h->bnear)) ||
-        (rc = zero(h, h->ct)) || (rc = zero(h, h->wt)) || (rc = zero(h, h->wpre)) || (rc = zero(h, h->plist)) ||
+        (rc = zero(h, h->ct[0])) || (rc = zero(h, h->ct[1])) || (rc = zero(h, h->wt)) || (rc = zero(h, h->wpre)) || (rc = zero(h, h->plist)) ||
         (rc = zero(h, h->keys)) || (rc = zero(h, h->bpv)))
         return bail(rc);
     {
@@ -704,8 +732,7 @@ int sf_upload_boundary(sf_handle h, size_t nb, const float* pos3, const uint64_t
     SortBuffers sb{h->kA.p, h->vA.p, h->kB.p, h->vB.p, h->hist.p};
     const uint32_t *sk = nullptr, *bperm = nullptr;
     if ((rc = radix_sort(h->keys.p, (int)nb, h->plan, sb, &sk, &bperm, h->stream))) return rc;
-    launch_cell_start(sk, (int)nb, h->local_cells(), nullptr, h->bcell.p, nullptr, nullptr, PhasePos{},
-                      IncStart{nullptr, nullptr}, h->stream);
+    launch_cell_start(sk, (int)nb, h->local_cells(), nullptr, h->bcell.p, nullptr, PhasePos{}, IncClear{}, h->stream);
     launch_boundary_gather(bperm, tmp.p, h->bpv.p, (int)nb, h->stream);
     launch_boundary_volume(h->K, h->bpv.p, h->bcell.p, (int)nb, h->stream);
     launch_boundary_near(h->K, h->bcell.p, h->bnear.p, h->stream);
@@ -1335,13 +1362,15 @@ int sf_batch_create(const sf_params* p, const sf_boundary_params* b, const sf_so
         sf_destroy(h);
         return code;
     };
-    if ((rc = h->cell.alloc((size_t)h->C + 1)) || (rc = h->ct.alloc((size_t)h->C + 1)) ||
+    if ((rc = h->cell.alloc((size_t)h->C + 1)) || (rc = h->ct[0].alloc((size_t)h->C + 1)) ||
+        (rc = h->ct[1].alloc((size_t)h->C + 1)) ||
         (rc = h->scene.alloc(sid.size())) || (rc = h->sct.alloc(n_scenes)) || (rc = ensure_cell_capacity(h)))
         return bail(rc);
     {
         hipError_t e;
         if ((e = hipMemsetAsync(h->cell.p, 0, h->cell.n * sizeof(uint32_t), h->stream)) != hipSuccess ||
-            (e = hipMemsetAsync(h->ct.p, 0, h->ct.n * sizeof(uint2), h->stream)) != hipSuccess ||
+            (e = hipMemsetAsync(h->ct[0].p, 0, h->ct[0].n * sizeof(uint2), h->stream)) != hipSuccess ||
+            (e = hipMemsetAsync(h->ct[1].p, 0, h->ct[1].n * sizeof(uint2), h->stream)) != hipSuccess ||
             (e = hipMemcpyAsync(h->scene.p, sid.data(), sid.size() * sizeof(uint16_t), hipMemcpyHostToDevice,
                                 h->stream)) != hipSuccess)
             return bail(hip_error(e, "batch buffers"));

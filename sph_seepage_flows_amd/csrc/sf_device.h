@@ -215,6 +215,61 @@ SF_DEV v3 world_walls(const SFConst& k, v3 p, v3 v) {
     return f;
 }
 
+// What the incremental sort needs to know of the particles that change cell,
+// counted by whoever writes the new keys.  Counts carry the number of water
+// particles in their upper half.
+//   in_count[c]  particles whose key changed to c
+//   head, next   those particles chained: head[c] and next[i] hold 1 + a slot
+//                (0: end), with the slot's water flag in the top bit
+//   part         per tile of kMoveTile slots (tiles of slots, then of cells
+//                from part + cell_part on): the slots whose key did not change,
+//                and the newcomers of the tile's cells
+struct Newcomers {
+    uint64_t* in_count;
+    uint32_t* head;
+    uint32_t* next;
+    uint64_t* part;
+    uint32_t cell_part;
+};
+constexpr int kMoveTile = 2048;
+constexpr uint32_t kChainIndex = 0x7fffffffu;
+// Must be called by all threads of a kBlock block (kMoveTile is a multiple of
+// it); slot i = the thread's, not `valid` past the last.
+SF_DEV void count_moves(bool valid, uint32_t key, uint32_t old, bool water, int i, const Newcomers& nc) {
+    __shared__ uint32_t stays[kBlock / 64], wets[kBlock / 64];
+    const bool move = valid && key != old;
+    if (move) {
+        atomicAdd((unsigned long long*)nc.in_count + key, water ? 0x100000001ull : 1ull);
+        nc.next[i] = atomicExch(nc.head + key, ((uint32_t)i + 1u) | (water ? ~kChainIndex : 0u));
+    }
+    // movers of a wave mostly go to cells of one tile: one atomic per tile
+    uint64_t todo = __ballot(move);
+    const uint64_t wet = __ballot(water);
+    while (todo) {
+        const int lead = __builtin_ctzll(todo);
+        const uint32_t tile = (uint32_t)__builtin_amdgcn_readlane((int)(key / (uint32_t)kMoveTile), lead);
+        const uint64_t mine = __ballot(move && key / (uint32_t)kMoveTile == tile);
+        if ((int)(threadIdx.x & 63u) == lead)
+            atomicAdd((unsigned long long*)nc.part + nc.cell_part + tile,
+                      ((unsigned long long)__popcll(mine & wet) << 32) + (unsigned long long)__popcll(mine));
+        todo &= ~mine;
+    }
+    const uint64_t stay = __ballot(valid && !move);
+    if ((threadIdx.x & 63u) == 0) {
+        stays[threadIdx.x >> 6] = (uint32_t)__popcll(stay);
+        wets[threadIdx.x >> 6] = (uint32_t)__popcll(stay & wet);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t a = 0, b = 0;
+        for (int q = 0; q < kBlock / 64; ++q) {
+            a += stays[q];
+            b += wets[q];
+        }
+        if (a) atomicAdd((unsigned long long*)nc.part + i / kMoveTile, ((unsigned long long)b << 32) + a);
+    }
+}
+
 // Block mapping of a pass over two phases of a slot list: na blocks of phase
 // 0, then nb blocks of phase 1.  Each XCD (hardware blocks b with b % 8 = x)
 // first runs its contiguous 1/8 share of the phase-0 blocks, then its share

@@ -97,7 +97,7 @@ int diff_step(sf_system* h, float dt, StepTapeBufs* tape) {
     CopyJobs before{{{h->pm[h->cur].p, T.pm.p, n * sizeof(float4)},
                      {h->vr[h->cur].p, T.vr.p, n * sizeof(float4)},
                      {h->perm, T.perm.p, n * sizeof(uint32_t)},
-                     {h->ct.p, T.ct.p, ((size_t)h->C + 1) * sizeof(uint2)}},
+                     {h->ct[h->cur_ct].p, T.ct.p, ((size_t)h->C + 1) * sizeof(uint2)}},
                     4};
     launch_copy_jobs(before, s);
     Fields f = h->fields();

@@ -87,7 +87,9 @@ int radix_sort(const uint32_t* keys, int n, const RadixPlan& plan, const SortBuf
 
 // ---- searcher launchers (sf_searcher.hip) ----
 // scene (batched handles): per-slot scene id, keys offset by scene * C; null for one scene
-void launch_hash(const SFConst& k, const float4* pm, const uint16_t* scene, uint32_t* keys, int n, hipStream_t s);
+// wflag (may be null): the slots' water flags, written along
+void launch_hash(const SFConst& k, const float4* pm, const uint16_t* scene, uint32_t* keys, uint8_t* wflag, int n,
+                 hipStream_t s);
 // Positions in phase order, written by the cell-start launch when pph is set:
 // pph[t] = pm[plist[t]] for t < n.
 struct PhasePos {
@@ -95,19 +97,19 @@ struct PhasePos {
     const float4* pm;
     float4* pph;
 };
-// After an incremental sort: cellStart[c] is then the stayers before c's old
-// start plus the newcomers of the cells before c.
-struct IncStart {
-    const uint32_t* stay_pre;  // n + 1
-    const uint32_t* in_start;  // C + 1
+// Counters of the next incremental sort, cleared by every build: newcomers
+// per cell (in_count, C + 1; null: none to clear), the chains' heads (C + 1)
+// and the tile sums (part[0, parts)).
+struct IncClear {
+    uint64_t* in_count;
+    uint32_t* head;
+    uint64_t* part;
+    uint32_t parts;
 };
-// cellStart[c] for c in [0, C] plus the cell table ct[c] = (cellStart[c], wpre[cellStart[c]]);
-// zero_c (may be null) is cleared over [0, C) (the incremental sort's newcomer counters).
-// With inc.stay_pre set, cell_start holds the previous sort's cellStart on
-// entry and each entry is updated in place from it; otherwise each cell's
-// start is found by binary search over sorted_keys.
+// cellStart[c] for c in [0, C] by binary search over sorted_keys, plus the
+// cell table ct[c] = (cellStart[c], wpre[cellStart[c]]).
 void launch_cell_start(const uint32_t* sorted_keys, int n, uint32_t C, const uint32_t* wpre, uint32_t* cell_start,
-                       uint2* ct, uint32_t* zero_c, PhasePos pp, IncStart inc, hipStream_t s);
+                       uint2* ct, PhasePos pp, IncClear z, hipStream_t s);
 struct GatherArgs {
     const uint32_t* perm;
     const float4 *pm_in, *vr_in, *cs_in, *cda_in;
@@ -134,24 +136,39 @@ void launch_boundary_near(const SFConst& k, const uint32_t* bcs, uint8_t* near, 
 void launch_nbr_count(const SFConst& k, const float4* pm, const uint16_t* scene, const uint32_t* cs, uint32_t* cnt,
                       uint32_t* cand, int n, hipStream_t s);
 void launch_hash_boundary(const SFConst& k, const float4* bp, uint32_t* keys, int nb, hipStream_t s);
-// Incremental stable sort (the particles are in the previous sort's order):
-// key / old_key per slot, old_start = the previous cellStart (C + 1).
-struct IncSortBuffers {
-    uint32_t* in_count;  // C + 1, zero on entry (launch_cell_start clears it)
-    uint32_t* in_start;  // C + 1
-    uint32_t* slot;      // n
-    uint32_t* in_list;   // n
-    uint32_t* stay_pre;  // n + 1
-    uint32_t* part;      // vprefix2_partials(n, C)
+// Where whoever writes the next build's keys (the advect, or k_inc_flag)
+// counts the particles that change cell: see count_moves (sf_device.h).
+// Incremental stable sort and reorder (the particles are in the previous
+// sort's order).  ct_old is the previous cell table; nwater receives the
+// water count, cell / ct the new cellStart and cell table (C + 1 entries).
+struct PlaceArgs {
+    GatherArgs g;  // perm unused
+    const uint32_t* key;
+    const uint32_t* old_key;
+    const uint8_t* wflag_in;  // water flags of the current slots
+    const uint2* ct_old;
+    uint64_t* stay_pre;  // n + 1
+    uint64_t* in_start;  // C + 1
+    uint64_t* in_count;  // C + 1, zero on entry of the counting, cleared here
+    const uint32_t* head;
+    const uint32_t* next;
+    uint32_t* head_next;  // the next sort's heads, cleared here
+    uint64_t* part;       // inc_parts(n, C) tile sums, cleared here
+    uint32_t parts;
+    uint32_t* perm;
+    uint32_t* sorted_keys;
+    uint32_t* plist;
+    float4* pph;
+    uint32_t* cell;
+    uint2* ct;
+    uint32_t* nwater;
 };
-// flags_done: the newcomer ranks (slot) and counts (in_count) were already
-// taken, by the advect that wrote key
-void launch_incremental_sort(const uint32_t* key, const uint32_t* old_key, const uint32_t* old_start, int n,
-                             uint32_t C, const IncSortBuffers& b, uint32_t* perm, uint32_t* sorted_keys,
-                             bool flags_done, hipStream_t s);
+// flags_done: the moves were already counted, by the advect that wrote key
+void launch_incremental_sort(const PlaceArgs& a, const Newcomers& nc, int n, uint32_t C, bool flags_done,
+                             hipStream_t s);
+uint32_t inc_parts(int n, uint32_t C);
 // partial-sum counts of the prefix kernels
 int wprefix_blocks(int n);
-int vprefix2_partials(int n1, int n2);
 
 // ---- solver launchers (sf_solver.hip) ----
 constexpr int kCountStride = 64;  // words between the two interface counters (a cache line each)
@@ -302,12 +319,11 @@ struct AdvectArgs {
     // The next neighbour build's hash and change flags, written here from the
     // new positions when keys_out is non-null (incremental sort): keys_out[i]
     // = cell key of the new position (offset by scene * C for batched
-    // handles), and where it differs from old_keys[i] (this step's sorted key
-    // of slot i) slot[i] = the newcomer rank taken from in_count.
+    // handles), and the slots whose key differs from old_keys[i] (this step's
+    // sorted key of slot i) counted in nc.
     uint32_t* keys_out;
     const uint32_t* old_keys;
-    uint32_t* in_count;
-    uint32_t* slot;
+    Newcomers nc;
     const uint16_t* scene;
 };
 void launch_advect(const SFConst& k, const AdvectArgs& a, int n, hipStream_t s);

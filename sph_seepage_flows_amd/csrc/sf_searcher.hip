@@ -14,7 +14,7 @@ namespace sf {
 template <bool kBatch>
 __global__ __launch_bounds__(kBlock) void k_hash(SFConst k, const float4* __restrict__ pm,
                                                  const uint16_t* __restrict__ scene, uint32_t* __restrict__ keys,
-                                                 int n) {
+                                                 uint8_t* __restrict__ wflag, int n) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const float4 p = pm[i];
@@ -23,16 +23,18 @@ __global__ __launch_bounds__(kBlock) void k_hash(SFConst k, const float4* __rest
     uint32_t key = cell_key(k, cx, cy, cz);
     if constexpr (kBatch) key += (uint32_t)scene[i] * k.C;
     keys[i] = key;
+    if (wflag) wflag[i] = p.w > 0.f ? 1 : 0;  // the caller may have changed labels too
 }
-void launch_hash(const SFConst& k, const float4* pm, const uint16_t* scene, uint32_t* keys, int n, hipStream_t s) {
+void launch_hash(const SFConst& k, const float4* pm, const uint16_t* scene, uint32_t* keys, uint8_t* wflag, int n,
+                 hipStream_t s) {
     if (n <= 0) return;
     if (scene)
-        k_hash<true><<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, pm, scene, keys, n);
+        k_hash<true><<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, pm, scene, keys, wflag, n);
     else
-        k_hash<false><<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, pm, nullptr, keys, n);
+        k_hash<false><<<(n + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, pm, nullptr, keys, wflag, n);
 }
 void launch_hash_boundary(const SFConst& k, const float4* bp, uint32_t* keys, int nb, hipStream_t s) {
-    launch_hash(k, bp, nullptr, keys, nb, s);
+    launch_hash(k, bp, nullptr, keys, nullptr, nb, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -95,42 +97,43 @@ __global__ __launch_bounds__(kRsThreads) void k_rs_upsweep(const uint32_t* __res
 
 // exclusive scan of hist[0, total) in place by one workgroup of 1024
 // threads; *total_out (if given) receives the sum
-SF_DEV void scan_range(uint32_t* __restrict__ hist, int total, uint32_t* __restrict__ total_out) {
-    __shared__ uint32_t wsum[16];
-    __shared__ uint32_t carry_s;
+template <class U>
+SF_DEV void scan_range(U* __restrict__ hist, int total, U* __restrict__ total_out) {
+    __shared__ U wsum[16];
+    __shared__ U carry_s;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     if (t == 0) carry_s = 0;
     __syncthreads();
     for (int base = 0; base < total; base += 1024 * 4) {
-        uint32_t v[4];
-        uint32_t s = 0;
+        U v[4];
+        U s = 0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int idx = base + t * 4 + q;
-            v[q] = idx < total ? hist[idx] : 0u;
+            v[q] = idx < total ? hist[idx] : (U)0;
             s += v[q];
         }
         // inclusive wave scan of s
-        uint32_t x = s;
+        U x = s;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            uint32_t y = __shfl_up(x, o, 64);
+            U y = __shfl_up(x, o, 64);
             if (lane >= o) x += y;
         }
         if (lane == 63) wsum[w] = x;
         __syncthreads();
         if (w == 0) {
-            uint32_t ws = lane < 16 ? wsum[lane] : 0u;
+            U ws = lane < 16 ? wsum[lane] : (U)0;
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) {
-                uint32_t y = __shfl_up(ws, o, 64);
+                U y = __shfl_up(ws, o, 64);
                 if (lane >= o) ws += y;
             }
             if (lane < 16) wsum[lane] = ws;  // inclusive over waves
         }
         __syncthreads();
-        const uint32_t carry = carry_s;
-        uint32_t run = carry + (w > 0 ? wsum[w - 1] : 0u) + x - s;
+        const U carry = carry_s;
+        U run = carry + (w > 0 ? wsum[w - 1] : (U)0) + x - s;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int idx = base + t * 4 + q;
@@ -145,13 +148,13 @@ SF_DEV void scan_range(uint32_t* __restrict__ hist, int total, uint32_t* __restr
     __syncthreads();
 }
 __global__ __launch_bounds__(1024) void k_rs_scan(uint32_t* __restrict__ hist, int total) {
-    scan_range(hist, total, nullptr);
+    scan_range<uint32_t>(hist, total, nullptr);
 }
 // two independent scans, [0, n1) and [n1, n1 + n2), in one launch
-__global__ __launch_bounds__(1024) void k_rs_scan2(uint32_t* __restrict__ part, int n1, int n2,
-                                                  uint32_t* __restrict__ total_out) {
-    scan_range(part, n1, total_out);
-    scan_range(part + n1, n2, nullptr);
+template <class U>
+__global__ __launch_bounds__(1024) void k_rs_scan2(U* __restrict__ part, int n1, int n2, U* __restrict__ total_out) {
+    scan_range<U>(part, n1, total_out);
+    scan_range<U>(part + n1, n2, nullptr);
 }
 
 // stable scatter: each wave ranks a contiguous chunk of 64*kRsItems keys
@@ -234,39 +237,36 @@ int radix_sort(const uint32_t* keys, int n, const RadixPlan& plan, const SortBuf
 
 // ---------------------------------------------------------------------------
 // cellStart[c] = number of particles with key < c, c in [0, C]
-// (CountingInCell_CUDA + exclusive_scan, cuda_neighbor_searcher.cu:45-47)
+// (CountingInCell_CUDA + exclusive_scan, cuda_neighbor_searcher.cu:45-47),
+// after a radix sort (the incremental sort's placement writes its own)
 __global__ __launch_bounds__(kBlock) void k_cell_start(const uint32_t* __restrict__ sk, int n, uint32_t C,
                                                        const uint32_t* __restrict__ wpre, uint32_t* __restrict__ cs,
-                                                       uint2* __restrict__ ct, uint32_t* __restrict__ zero_c,
-                                                       PhasePos pp, IncStart inc) {
+                                                       uint2* __restrict__ ct, PhasePos pp, IncClear z) {
     const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
     // pph[t] = pm[plist[t]]: coalesced stores, loads that walk each phase's
     // slots in increasing order
     if (pp.pph && c < (uint32_t)n) pp.pph[c] = ldo(pp.pm, ldo(pp.plist, c));
+    if (c < z.parts) z.part[c] = 0ull;
     if (c > C) return;
-    if (zero_c && c < C) zero_c[c] = 0u;  // the next incremental sort's newcomer counters
-    uint32_t lo = 0;
-    if (inc.stay_pre) {
-        // particles with a new key below c: the stayers (key unchanged) of the
-        // old cells below c and the newcomers of the cells below c
-        lo = inc.stay_pre[cs[c]] + inc.in_start[c];
-    } else {
-        uint32_t hi = (uint32_t)n;
-        while (lo < hi) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (sk[mid] < c) lo = mid + 1;
-            else hi = mid;
-        }
+    if (z.in_count) {
+        z.in_count[c] = 0ull;
+        z.head[c] = 0u;
+    }
+    uint32_t lo = 0, hi = (uint32_t)n;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (sk[mid] < c) lo = mid + 1;
+        else hi = mid;
     }
     cs[c] = lo;
     if (ct) ct[c] = make_uint2(lo, wpre ? wpre[lo] : 0u);
 }
 void launch_cell_start(const uint32_t* sorted_keys, int n, uint32_t C, const uint32_t* wpre, uint32_t* cell_start,
-                       uint2* ct, uint32_t* zero_c, PhasePos pp, IncStart inc, hipStream_t s) {
+                       uint2* ct, PhasePos pp, IncClear z, hipStream_t s) {
     uint32_t total = C + 1;
     if (pp.pph && (uint32_t)n > total) total = (uint32_t)n;
-    k_cell_start<<<(total + kBlock - 1) / kBlock, kBlock, 0, s>>>(sorted_keys, n, C, wpre, cell_start, ct, zero_c,
-                                                                  pp, inc);
+    if (z.parts > total) total = z.parts;
+    k_cell_start<<<(total + kBlock - 1) / kBlock, kBlock, 0, s>>>(sorted_keys, n, C, wpre, cell_start, ct, pp, z);
 }
 
 // ---------------------------------------------------------------------------
@@ -276,6 +276,7 @@ void launch_cell_start(const uint32_t* sorted_keys, int n, uint32_t C, const uin
 // tile's water count in wpart[block] for the prefix that follows.
 constexpr int kWpItems = 8;
 constexpr int kWpTile = kBlock * kWpItems;
+static_assert(kWpTile == kMoveTile, "the tiles whoever counts the moves sums over");
 __global__ __launch_bounds__(kBlock) void k_gather(GatherArgs a, int n, uint32_t* __restrict__ wpart) {
     __shared__ uint32_t ws[kBlock / 64];
     const int t = threadIdx.x;
@@ -374,29 +375,6 @@ void launch_boundary_near(const SFConst& k, const uint32_t* bcs, uint8_t* near, 
 // needs.  Two kernels around a tiny scan of per-block counts.
 int wprefix_blocks(int n) { return (n + kWpTile - 1) / kWpTile; }
 
-// Exclusive prefix of a per-slot value v(i), i in [0, n): block partial sums,
-// one-workgroup scan of the partials, then per-slot prefixes; slot n gets the
-// total.  Used for the water prefix and the incremental sort.
-template <class V>
-SF_DEV void tile_sum(V v, int n, int tile, uint32_t* __restrict__ part_out) {
-    __shared__ uint32_t ws[kBlock / 64];
-    const int t = threadIdx.x;
-    const int base = tile * kWpTile;
-    uint32_t c = 0;
-#pragma unroll
-    for (int q = 0; q < kWpItems; ++q) {
-        const int i = base + q * kBlock + t;
-        c += i < n ? v(i) : 0u;
-    }
-    for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o, 64);
-    if ((t & 63) == 0) ws[t >> 6] = c;
-    __syncthreads();
-    if (t == 0) {
-        uint32_t sum = 0;
-        for (int q = 0; q < kBlock / 64; ++q) sum += ws[q];
-        *part_out = sum;
-    }
-}
 // tile's slot prefixes from its scanned partial (thread t owns kWpItems
 // consecutive slots); slot n (one past the end) receives the total.
 // emit(i, prefix, value) is called for every slot i < n.
@@ -405,14 +383,14 @@ SF_DEV void tile_sum(V v, int n, int tile, uint32_t* __restrict__ part_out) {
 // over q in [lo, b) (before) and over [lo, hi) (all), by the whole block.
 constexpr int kDirectTiles = 4096;
 int g_direct_tiles = kDirectTiles;  // sf_set_prefix_scan_threshold
-SF_DEV void block_sums(const uint32_t* __restrict__ cnt, uint32_t lo, uint32_t b, uint32_t hi, uint32_t& before,
-                       uint32_t& all) {
-    __shared__ uint32_t red[2][kBlock / 64];
-    uint32_t a = 0, p = 0;
+template <class U>
+SF_DEV void block_sums(const U* __restrict__ cnt, uint32_t lo, uint32_t b, uint32_t hi, U& before, U& all) {
+    __shared__ U red[2][kBlock / 64];
+    U a = 0, p = 0;
     for (uint32_t q = lo + threadIdx.x; q < hi; q += kBlock) {
-        const uint32_t c = cnt[q];
+        const U c = cnt[q];
         a += c;
-        p += q < b ? c : 0u;
+        p += q < b ? c : (U)0;
     }
     for (int o = 32; o > 0; o >>= 1) {
         a += __shfl_down(a, o, 64);
@@ -431,30 +409,30 @@ SF_DEV void block_sums(const uint32_t* __restrict__ cnt, uint32_t lo, uint32_t b
     }
 }
 
-template <class V, class Emit>
-SF_DEV void tile_prefix(V v, int n, int tile, uint32_t part, uint32_t* __restrict__ out, Emit&& emit) {
-    __shared__ uint32_t wsum[kBlock / 64];
+template <class U, class V, class Emit>
+SF_DEV void tile_prefix(V v, int n, int tile, U part, U* __restrict__ out, Emit&& emit) {
+    __shared__ U wsum[kBlock / 64];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int base = tile * kWpTile + t * kWpItems;
-    uint32_t f[kWpItems];
-    uint32_t s = 0;
+    U f[kWpItems];
+    U s = 0;
     if (base + kWpItems <= n) {
         v.load8(base, f);  // whole run in range: vector loads
     } else {
 #pragma unroll
-        for (int q = 0; q < kWpItems; ++q) f[q] = base + q < n ? v(base + q) : 0u;
+        for (int q = 0; q < kWpItems; ++q) f[q] = base + q < n ? v(base + q) : (U)0;
     }
 #pragma unroll
     for (int q = 0; q < kWpItems; ++q) s += f[q];
-    uint32_t x = s;
+    U x = s;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-        uint32_t y = __shfl_up(x, o, 64);
+        U y = __shfl_up(x, o, 64);
         if (lane >= o) x += y;
     }
     if (lane == 63) wsum[w] = x;
     __syncthreads();
-    uint32_t run = part + x - s;
+    U run = part + x - s;
     for (int q = 0; q < w; ++q) run += wsum[q];
 #pragma unroll
     for (int q = 0; q < kWpItems; ++q) {
@@ -465,47 +443,32 @@ SF_DEV void tile_prefix(V v, int n, int tile, uint32_t part, uint32_t* __restric
     }
 }
 struct NoEmit {
-    SF_DEV void operator()(int, uint32_t, uint32_t) const {}
+    template <class U>
+    SF_DEV void operator()(int, U, U) const {}
 };
 
-// Exclusive prefixes of two per-slot values in three launches: v1 over
-// [0, n1) into out1[0, n1], v2 over [0, n2) into out2[0, n2].  Blocks
-// [0, nb1) work on the first, [nb1, nb1 + nb2) on the second.
-template <class V1, class V2>
-__global__ __launch_bounds__(kBlock) void k_vsum2(V1 v1, int n1, int nb1, V2 v2, int n2, uint32_t* __restrict__ part) {
-    const int b = blockIdx.x;
-    if (b < nb1) tile_sum(v1, n1, b, part + b);
-    else tile_sum(v2, n2, b - nb1, part + b);
-}
-template <class V1, class V2>
-// scanned = 0: part holds the raw block sums, and each block sums those
+// Exclusive prefixes of two per-slot values, v1 over [0, n1) into out1[0, n1]
+// and v2 over [0, n2) into out2[0, n2], whose sums per tile of kWpTile slots
+// are in part (nb1 tiles of the first, then the second's).  Blocks [0, nb1)
+// work on the first, the others on the second.
+// scanned = 0: part holds the raw tile sums, and each block sums those
 // before it within its own prefix (the block holding slot n thereby ends on
 // the total, as the scan would give it).
-__global__ __launch_bounds__(kBlock) void k_vprefix2(V1 v1, int n1, int nb1, uint32_t* __restrict__ out1, V2 v2,
-                                                     int n2, uint32_t* __restrict__ out2,
-                                                     const uint32_t* __restrict__ part, int scanned) {
+template <class V1, class V2>
+__global__ __launch_bounds__(kBlock) void k_vprefix2(V1 v1, int n1, int nb1, uint64_t* __restrict__ out1, V2 v2,
+                                                     int n2, uint64_t* __restrict__ out2,
+                                                     const uint64_t* __restrict__ part, int scanned) {
     const int b = blockIdx.x;
-    uint32_t pb = 0;
+    uint64_t pb = 0;
     if (scanned) {
         pb = part[b];
     } else {
-        uint32_t all;
+        uint64_t all;
         if (b < nb1) block_sums(part, 0u, (uint32_t)b, (uint32_t)nb1, pb, all);
         else block_sums(part, (uint32_t)nb1, (uint32_t)b, gridDim.x, pb, all);
     }
     if (b < nb1) tile_prefix(v1, n1, b, pb, out1, NoEmit{});
     else tile_prefix(v2, n2, b - nb1, pb, out2, NoEmit{});
-}
-int vprefix2_partials(int n1, int n2) { return wprefix_blocks(n1 + 1) + wprefix_blocks(n2 + 1); }
-template <class V1, class V2>
-void launch_vprefix2(V1 v1, int n1, uint32_t* out1, V2 v2, int n2, uint32_t* out2, uint32_t* part, hipStream_t s) {
-    // blocks cover slots [0, n]; the block holding slot n counts nothing and
-    // receives the total from the prefix of the blocks before it
-    const int nb1 = wprefix_blocks(n1 + 1), nb2 = wprefix_blocks(n2 + 1);
-    k_vsum2<<<nb1 + nb2, kBlock, 0, s>>>(v1, n1, nb1, v2, n2, part);
-    const int scanned = nb1 + nb2 > g_direct_tiles ? 1 : 0;
-    if (scanned) k_rs_scan2<<<1, 1024, 0, s>>>(part, nb1, nb2, nullptr);
-    k_vprefix2<<<nb1 + nb2, kBlock, 0, s>>>(v1, n1, nb1, out1, v2, n2, out2, part, scanned);
 }
 // Per-slot values of the prefixes; load8(i, f) reads slots i .. i + 7 (i a
 // multiple of 8, all below n) with vector loads.
@@ -513,26 +476,39 @@ SF_DEV void load8_u32(const uint32_t* a, int i, uint4& x, uint4& y) {
     x = *reinterpret_cast<const uint4*>(a + i);
     y = *reinterpret_cast<const uint4*>(a + i + 4);
 }
-struct StayVal {
+// A count of particles and, in the upper half, of the water among them
+// (counts stay below 2^27).
+SF_DEV uint64_t counted(bool one, bool water) { return one ? (water ? 0x100000001ull : 1ull) : 0ull; }
+struct StayVal {  // slots whose key did not change
     const uint32_t* key;
     const uint32_t* old;
-    SF_DEV uint32_t operator()(int i) const { return key[i] == old[i] ? 1u : 0u; }
-    SF_DEV void load8(int i, uint32_t* f) const {
+    const uint8_t* wflag;
+    SF_DEV uint64_t operator()(int i) const { return counted(key[i] == old[i], wflag[i] != 0); }
+    SF_DEV void load8(int i, uint64_t* f) const {
         uint4 k0, k1, o0, o1;
         load8_u32(key, i, k0, k1);
         load8_u32(old, i, o0, o1);
-        f[0] = k0.x == o0.x; f[1] = k0.y == o0.y; f[2] = k0.z == o0.z; f[3] = k0.w == o0.w;
-        f[4] = k1.x == o1.x; f[5] = k1.y == o1.y; f[6] = k1.z == o1.z; f[7] = k1.w == o1.w;
+        const uint2 w = *reinterpret_cast<const uint2*>(wflag + i);
+        f[0] = counted(k0.x == o0.x, w.x & 0xffu);
+        f[1] = counted(k0.y == o0.y, w.x & 0xff00u);
+        f[2] = counted(k0.z == o0.z, w.x & 0xff0000u);
+        f[3] = counted(k0.w == o0.w, w.x & 0xff000000u);
+        f[4] = counted(k1.x == o1.x, w.y & 0xffu);
+        f[5] = counted(k1.y == o1.y, w.y & 0xff00u);
+        f[6] = counted(k1.z == o1.z, w.y & 0xff0000u);
+        f[7] = counted(k1.w == o1.w, w.y & 0xff000000u);
     }
 };
 struct ArrayVal {
-    const uint32_t* a;
-    SF_DEV uint32_t operator()(int i) const { return a[i]; }
-    SF_DEV void load8(int i, uint32_t* f) const {
-        uint4 x, y;
-        load8_u32(a, i, x, y);
-        f[0] = x.x; f[1] = x.y; f[2] = x.z; f[3] = x.w;
-        f[4] = y.x; f[5] = y.y; f[6] = y.z; f[7] = y.w;
+    const uint64_t* a;
+    SF_DEV uint64_t operator()(int i) const { return a[i]; }
+    SF_DEV void load8(int i, uint64_t* f) const {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(a + i + 2 * q);
+            f[2 * q] = v.x;
+            f[2 * q + 1] = v.y;
+        }
     }
 };
 struct FlagVal {
@@ -565,7 +541,7 @@ __global__ __launch_bounds__(kBlock) void k_wprefix_plist(const uint8_t* __restr
     } else {
         block_sums(wpart, 0u, blockIdx.x, gridDim.x, part, nwater);
     }
-    tile_prefix(FlagVal{wflag}, n, (int)blockIdx.x, part, wpre, [&](int i, uint32_t pre, uint32_t water) {
+    tile_prefix<uint32_t>(FlagVal{wflag}, n, (int)blockIdx.x, part, wpre, [&](int i, uint32_t pre, uint32_t water) {
         plist[water ? pre : nwater + (uint32_t)i - pre] = (uint32_t)i;
     });
 }
@@ -579,76 +555,108 @@ void launch_gather_wprefix(const GatherArgs& a, int n, uint32_t* wpart, uint32_t
     const int nb = wprefix_blocks(n + 1);
     k_gather<<<nb, kBlock, 0, s>>>(a, n, wpart);
     const int scanned = nb > g_direct_tiles ? 1 : 0;
-    if (scanned) k_rs_scan2<<<1, 1024, 0, s>>>(wpart, nb, 0, wpart + nb);
+    if (scanned) k_rs_scan2<uint32_t><<<1, 1024, 0, s>>>(wpart, nb, 0, wpart + nb);
     k_wprefix_plist<<<nb, kBlock, 0, s>>>(a.wflag, n, wpart, scanned, wpre, plist);
 }
 
 // ---------------------------------------------------------------------------
-// Incremental stable sort.  The particles are in the previous step's sorted
-// order and most keep their cell, so the stable sort by the new keys is
-// rebuilt without radix passes: within each new cell the particles are
-// ordered by current index, so a particle's output slot is
+// Incremental stable sort and reorder.  The particles are in the previous
+// step's sorted order and most keep their cell, so the stable sort by the new
+// keys is rebuilt without radix passes: within each new cell the particles
+// are ordered by current index, so a particle's output slot is
 //   newStart(c) + #(stayers of c before it) + #(newcomers of c before it),
 // where stayers of c are the particles of c's old block whose key is still c
 // (a prefix over "key unchanged" flags counts them) and newcomers are the
-// few particles whose key changed to c (collected per cell, in the order the
+// few particles whose key changed to c (chained per cell, in the order the
 // atomics leave; a newcomer's rank is the count of smaller indices in its
-// cell's list, which that order does not change).
+// cell's chain, which that order does not change).
 // newStart(c) = stayers in cells < c + newcomers in cells < c.
 // The result is the stable sort's, element for element.
+//
+// Every count carries the water's share in its upper half, so the same sums
+// give the number of water particles before a slot, that is the particle's
+// index within its phase, and the placement reorders everything at once:
+// permutation, keys, the persistent state, the phase list, the positions in
+// phase order and the cell table.  With the tile sums of both prefixes taken
+// by whoever wrote the keys, two launches follow the advect; they were seven
+// (two prefix passes, newcomer lists, permutation, gather, water prefix,
+// cell table), each at least 2-4 us however small the scene, and they moved
+// the permutation, the flags and the positions once more each.
 __global__ __launch_bounds__(kBlock) void k_inc_flag(const uint32_t* __restrict__ key, const uint32_t* __restrict__ old,
-                                                     int n, uint32_t* __restrict__ in_count,
-                                                     uint32_t* __restrict__ slot) {
+                                                     const uint8_t* __restrict__ wflag, int n, Newcomers nc) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t c = key[i];
-    if (c != old[i]) slot[i] = atomicAdd(in_count + c, 1u);
+    const bool valid = i < n;
+    count_moves(valid, valid ? key[i] : 0u, valid ? old[i] : 0u, valid && wflag[i] != 0, i, nc);
 }
-__global__ __launch_bounds__(kBlock) void k_inc_fill(const uint32_t* __restrict__ key, const uint32_t* __restrict__ old,
-                                                     int n, const uint32_t* __restrict__ in_start,
-                                                     const uint32_t* __restrict__ slot, uint32_t* __restrict__ in_list) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t c = key[i];
-    if (c != old[i]) in_list[in_start[c] + slot[i]] = (uint32_t)i;
-}
-__global__ __launch_bounds__(kBlock) void k_inc_place(const uint32_t* __restrict__ key, const uint32_t* __restrict__ old,
-                                                      int n, const uint32_t* __restrict__ old_start,
-                                                      const uint32_t* __restrict__ stay_pre,
-                                                      const uint32_t* __restrict__ in_start,
-                                                      const uint32_t* __restrict__ in_list, uint32_t* __restrict__ perm,
-                                                      uint32_t* __restrict__ sorted_keys) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t c = key[i];
-    const uint32_t oa = old_start[c], ob = old_start[c + 1];
-    const uint32_t sa = stay_pre[oa];
-    const uint32_t s = in_start[c], e = in_start[c + 1];
-    uint32_t rank_in = 0;
-    for (uint32_t q = s; q < e; ++q) rank_in += in_list[q] < (uint32_t)i ? 1u : 0u;
-    uint32_t rank_stay;
-    if (c == old[i]) {
-        rank_stay = stay_pre[i] - sa;
-    } else {
-        const uint32_t u = (uint32_t)i;
-        rank_stay = u < oa ? 0u : (u >= ob ? stay_pre[ob] - sa : stay_pre[u] - sa);
+__global__ __launch_bounds__(kBlock) void k_inc_place(PlaceArgs a, int n, uint32_t C, int place_blocks) {
+    if ((int)blockIdx.x >= place_blocks) {
+        // the new cell table, and the next sort's counters
+        const uint32_t c = (blockIdx.x - (uint32_t)place_blocks) * kBlock + threadIdx.x;
+        if (c < a.parts) a.part[c] = 0ull;
+        if (c > C) return;
+        const uint64_t before = a.stay_pre[a.ct_old[c].x] + a.in_start[c];
+        const uint2 e = make_uint2((uint32_t)before, (uint32_t)(before >> 32));
+        a.cell[c] = e.x;
+        a.ct[c] = e;
+        a.in_count[c] = 0ull;
+        a.head_next[c] = 0u;
+        if (c == C) *a.nwater = e.y;
+        return;
     }
-    const uint32_t pos = sa + s + rank_stay + rank_in;
-    perm[pos] = (uint32_t)i;
-    sorted_keys[pos] = c;
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t c = a.key[i], o = a.old_key[i];
+    const float4 pm = a.g.pm_in[i], vr = a.g.vr_in[i], cs = a.g.cs_in[i];
+    const uint32_t oa = a.ct_old[c].x, ob = a.ct_old[c + 1].x;
+    const uint64_t s = a.in_start[c], e = a.in_start[c + 1];
+    const uint64_t nwater = a.stay_pre[n] + a.in_start[C];  // all water, in the upper half
+    const uint64_t sa = a.stay_pre[oa];
+    const uint32_t u = (uint32_t)i;
+    uint64_t rank = 0;  // of the cell: stayers before, then newcomers before
+    if (c == o || (u >= oa && u < ob)) rank = a.stay_pre[u] - sa;
+    else if (u >= ob) rank = a.stay_pre[ob] - sa;
+    // the cell's chain is as long as its newcomer count; the count ends the walk
+    uint32_t left = (uint32_t)e - (uint32_t)s;
+    for (uint32_t q = left ? a.head[c] : 0u; q != 0u; q = a.next[(q & kChainIndex) - 1u]) {
+        if ((q & kChainIndex) - 1u < u) rank += counted(true, (q & ~kChainIndex) != 0u);
+        if (--left == 0u) break;
+    }
+    const uint64_t at = sa + s + rank;
+    const uint32_t pos = (uint32_t)at, wbefore = (uint32_t)(at >> 32);
+    if (pos >= (uint32_t)n) return;  // never for consistent counts; keeps a bug in bounds
+    const bool water = pm.w > 0.f;
+    const uint32_t t = water ? wbefore : (uint32_t)(nwater >> 32) + pos - wbefore;
+    a.perm[pos] = u;
+    a.sorted_keys[pos] = c;
+    a.g.pm_out[pos] = pm;
+    a.g.vr_out[pos] = vr;
+    a.g.cs_out[pos] = cs;
+    if (a.g.multi) {
+        a.g.cda_out[pos] = a.g.cda_in[i];
+        a.g.amc_out[pos] = a.g.amc_in[i];
+    }
+    a.g.wflag[pos] = water ? 1 : 0;
+    if (t < (uint32_t)n) {
+        a.plist[t] = pos;
+        a.pph[t] = pm;
+    }
 }
 
-void launch_incremental_sort(const uint32_t* key, const uint32_t* old_key, const uint32_t* old_start, int n,
-                             uint32_t C, const IncSortBuffers& b, uint32_t* perm, uint32_t* sorted_keys,
-                             bool flags_done, hipStream_t s) {
+uint32_t inc_parts(int n, uint32_t C) { return (uint32_t)(wprefix_blocks(n + 1) + wprefix_blocks((int)C + 1)); }
+void launch_incremental_sort(const PlaceArgs& a, const Newcomers& nc, int n, uint32_t C, bool flags_done,
+                             hipStream_t s) {
     if (n <= 0) return;
     const int gn = (n + kBlock - 1) / kBlock;
-    // in_count is zero here: the cell-start kernel after every sort clears it
-    if (!flags_done) k_inc_flag<<<gn, kBlock, 0, s>>>(key, old_key, n, b.in_count, b.slot);
-    launch_vprefix2(StayVal{key, old_key}, n, b.stay_pre, ArrayVal{b.in_count}, (int)C, b.in_start, b.part, s);
-    k_inc_fill<<<gn, kBlock, 0, s>>>(key, old_key, n, b.in_start, b.slot, b.in_list);
-    k_inc_place<<<gn, kBlock, 0, s>>>(key, old_key, n, old_start, b.stay_pre, b.in_start, b.in_list, perm,
-                                       sorted_keys);
+    // in_count, the chains and part are zero here: every build clears them
+    if (!flags_done) k_inc_flag<<<gn, kBlock, 0, s>>>(a.key, a.old_key, a.wflag_in, n, nc);
+    const int nb1 = wprefix_blocks(n + 1), nb2 = wprefix_blocks((int)C + 1);
+    const int scanned = nb1 + nb2 > g_direct_tiles ? 1 : 0;
+    if (scanned) k_rs_scan2<uint64_t><<<1, 1024, 0, s>>>(a.part, nb1, nb2, nullptr);
+    k_vprefix2<<<nb1 + nb2, kBlock, 0, s>>>(StayVal{a.key, a.old_key, a.wflag_in}, n, nb1, a.stay_pre,
+                                            ArrayVal{a.in_count}, (int)C, a.in_start, a.part, scanned);
+    uint32_t cells = C + 1;
+    if (a.parts > cells) cells = a.parts;
+    k_inc_place<<<gn + (int)((cells + kBlock - 1) / kBlock), kBlock, 0, s>>>(a, n, C, gn);
 }
 
 // in-range neighbour counts: r^2 = dx*dx + dy*dy + dz*dz in FP32, left to

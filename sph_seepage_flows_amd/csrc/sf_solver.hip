@@ -1253,60 +1253,65 @@ void launch_cfl(const SFConst& k, const float4* acc, int n, float* partials, Cfl
 SF_DEV float sgnf(float v) { return (float)((0.f < v) - (v < 0.f)); }
 __global__ __launch_bounds__(kBlock) void k_advect(SFConst k, AdvectArgs a, int n) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const float dt = a.dt_dev ? a.dt_dev->ri / (float)a.dt_dev->nsub : a.dt;
-    const float4 p = a.pm_in[i];
-    const float4 v = a.vr_in[i];
-    float4 ac = a.acc[i];
-    if (p.w < 0.f) {
-        const float qx = ac.x * (v.x + 0.5f * dt * ac.x);
-        const float qy = ac.y * (v.y + 0.5f * dt * ac.y);
-        const float qz = ac.z * (v.z + 0.5f * dt * ac.z);
-        ac.x *= 1.f - k.damping * sgnf(qx);
-        ac.y *= 1.f - k.damping * sgnf(qy);
-        ac.z *= 1.f - k.damping * sgnf(qz);
-        a.acc[i] = ac;  // the reference stores the damped acceleration
-    }
-    v3 nv = mk3(v.x + dt * ac.x, v.y + dt * ac.y, v.z + dt * ac.z);
-    v3 np = mk3(p.x + dt * nv.x, p.y + dt * nv.y, p.z + dt * nv.z);
-    if (p.w > 0.f) {
-        const v3 pre = np;
-        const float r2 = 2.f * k.rw;
-        if (np.x > k.hix - r2) { np.x = k.hix - r2; nv.x = fminf(nv.x, 0.f); }
-        if (np.x < k.lox + r2) { np.x = k.lox + r2; nv.x = fmaxf(nv.x, 0.f); }
-        if (np.y > k.hiy - r2) { np.y = k.hiy - r2; nv.y = fminf(nv.y, 0.f); }
-        if (np.y < k.loy + r2) { np.y = k.loy + r2; nv.y = fmaxf(nv.y, 0.f); }
-        if (np.z > k.hiz - r2) { np.z = k.hiz - r2; nv.z = fminf(nv.z, 0.f); }
-        if (np.z < k.loz + r2) { np.z = k.loz + r2; nv.z = fmaxf(nv.z, 0.f); }
-        if (k.blabel1) {
-            int cx, cy, cz;
-            cell_of(k, pre.x, pre.y, pre.z, cx, cy, cz);
-            for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
-                const uint32_t be = a.bcell[c1];
-                for (uint32_t j = a.bcell[c0]; j < be; ++j) {
-                    const float4 b = a.bpv[j];
-                    if (b.w >= 0.f) continue;
-                    const v3 dp = pre - xyz(b);
-                    const float dl = sqrtf(dot(dp, dp));
-                    const float ov = dl - r2;
-                    if (ov < 0.f) {
-                        nv = nv * 0.f;
-                        np += dp * (1.f / dl) * (-ov);
+    uint32_t key = 0, old = 0;
+    bool is_water = false;
+    if (i < n) {
+        const float dt = a.dt_dev ? a.dt_dev->ri / (float)a.dt_dev->nsub : a.dt;
+        const float4 p = a.pm_in[i];
+        const float4 v = a.vr_in[i];
+        float4 ac = a.acc[i];
+        if (p.w < 0.f) {
+            const float qx = ac.x * (v.x + 0.5f * dt * ac.x);
+            const float qy = ac.y * (v.y + 0.5f * dt * ac.y);
+            const float qz = ac.z * (v.z + 0.5f * dt * ac.z);
+            ac.x *= 1.f - k.damping * sgnf(qx);
+            ac.y *= 1.f - k.damping * sgnf(qy);
+            ac.z *= 1.f - k.damping * sgnf(qz);
+            a.acc[i] = ac;  // the reference stores the damped acceleration
+        }
+        v3 nv = mk3(v.x + dt * ac.x, v.y + dt * ac.y, v.z + dt * ac.z);
+        v3 np = mk3(p.x + dt * nv.x, p.y + dt * nv.y, p.z + dt * nv.z);
+        if (p.w > 0.f) {
+            const v3 pre = np;
+            const float r2 = 2.f * k.rw;
+            if (np.x > k.hix - r2) { np.x = k.hix - r2; nv.x = fminf(nv.x, 0.f); }
+            if (np.x < k.lox + r2) { np.x = k.lox + r2; nv.x = fmaxf(nv.x, 0.f); }
+            if (np.y > k.hiy - r2) { np.y = k.hiy - r2; nv.y = fminf(nv.y, 0.f); }
+            if (np.y < k.loy + r2) { np.y = k.loy + r2; nv.y = fmaxf(nv.y, 0.f); }
+            if (np.z > k.hiz - r2) { np.z = k.hiz - r2; nv.z = fminf(nv.z, 0.f); }
+            if (np.z < k.loz + r2) { np.z = k.loz + r2; nv.z = fmaxf(nv.z, 0.f); }
+            if (k.blabel1) {
+                int cx, cy, cz;
+                cell_of(k, pre.x, pre.y, pre.z, cx, cy, cz);
+                for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
+                    const uint32_t be = a.bcell[c1];
+                    for (uint32_t j = a.bcell[c0]; j < be; ++j) {
+                        const float4 b = a.bpv[j];
+                        if (b.w >= 0.f) continue;
+                        const v3 dp = pre - xyz(b);
+                        const float dl = sqrtf(dot(dp, dp));
+                        const float ov = dl - r2;
+                        if (ov < 0.f) {
+                            nv = nv * 0.f;
+                            np += dp * (1.f / dl) * (-ov);
+                        }
                     }
-                }
-            });
+                });
+            }
+        }
+        a.pm_out[i] = f4(np, p.w);
+        a.vr_out[i] = f4(nv, v.w);
+        if (a.keys_out) {  // the next build's hash (k_hash)
+            int cx, cy, cz;
+            cell_of(k, np.x, np.y, np.z, cx, cy, cz);
+            key = cell_key(k, cx, cy, cz);
+            if (a.scene) key += (uint32_t)a.scene[i] * k.C;
+            a.keys_out[i] = key;
+            old = a.old_keys[i];
+            is_water = p.w > 0.f;
         }
     }
-    a.pm_out[i] = f4(np, p.w);
-    a.vr_out[i] = f4(nv, v.w);
-    if (a.keys_out) {  // the next build's hash and change flag (k_hash, k_inc_flag)
-        int cx, cy, cz;
-        cell_of(k, np.x, np.y, np.z, cx, cy, cz);
-        uint32_t key = cell_key(k, cx, cy, cz);
-        if (a.scene) key += (uint32_t)a.scene[i] * k.C;
-        a.keys_out[i] = key;
-        if (key != a.old_keys[i]) a.slot[i] = atomicAdd(a.in_count + key, 1u);
-    }
+    if (a.keys_out) count_moves(i < n, key, old, is_water, i, a.nc);  // and its change flags (k_inc_flag)
 }
 void launch_advect(const SFConst& k, const AdvectArgs& a, int n, hipStream_t s) {
     if (n <= 0) return;

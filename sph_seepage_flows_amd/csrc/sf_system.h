@@ -57,9 +57,11 @@ struct sf_system {
     DevBuf<float4> vq, wq, xq, wbq;   // listed particles' fields by phase index (Fields::wq)
     DevBuf<float4> rec0, rec1;        // water momentum neighbour records (Fields::rec0)
     DevBuf<uint8_t> wflag;
-    DevBuf<uint2> ct;
+    DevBuf<uint2> ct[2];  // cell table: the incremental sort reads the previous one
+    int cur_ct = 0;       // ct and head (the next advect's chains hang from head[cur_ct])
     // incremental sort (sf_set_sort_strategy): sorted-key ping-pong, permutation, work arrays
-    DevBuf<uint32_t> skeys[2], sperm, slot, in_list, stay_pre, in_count, in_start, part2;
+    DevBuf<uint32_t> skeys[2], sperm, head[2], next;
+    DevBuf<uint64_t> stay_pre, in_count, in_start, part2;
     bool sort_inc = true;
     size_t sort_cap = 0;
     const uint32_t* sorted_keys = nullptr;
@@ -127,7 +129,7 @@ struct sf_system {
         f.vr = vr[cur].p;
         f.cs = cs[cur_cs].p;
         f.cda = cda[cur_aux].p;
-        f.ct = ct.p;
+        f.ct = ct[cur_ct].p;
         f.bpv = bpv.p;
         f.bcell = bcell.p;
         f.bnear = bnear.p;
@@ -160,7 +162,11 @@ struct sf_system {
         return f;
     }
     uint32_t local_cells() const { return K.C; }
-    int parity() const { return cur | (cur_cs << 1) | (cur_aux << 2); }
+    int parity() const { return cur | (cur_cs << 1) | (cur_aux << 2) | (cur_ct << 3); }
+    // where the particles that change cell are counted for the next build
+    Newcomers newcomers() const {
+        return Newcomers{in_count.p, head[cur_ct].p, next.p, part2.p, (uint32_t)wprefix_blocks((int)n + 1)};
+    }
     // Two steps leave every buffer and flag where they found them, so that a
     // captured pair of steps can be replayed: with the incremental sort this
     // holds once the previous sorted keys sit in its two buffers (after a
