@@ -51,14 +51,13 @@ def pass_bytes(n_w: int, n_s: int, nb: int, cells: int, multi: bool, listed=(0, 
     lw, ls = listed
     return {
         # stepping loop: the advect computes the next keys and counts the
-        # moves (below).  The prefixes read both keys and the water flag and
-        # write the packed stay prefix, per cell the newcomer counts; the
-        # placement reads the keys and the prefix, reads and writes the
-        # persistent state and writes permutation, keys, flag, phase list and
-        # the positions in phase order; per cell the old table, the newcomer
-        # prefix and the chain head are read, the new tables and the cleared
+        # moves (below).  The placement reads both keys and the stay prefix,
+        # reads and writes the persistent state and writes permutation, keys,
+        # flag, phase list and the positions in phase order; per cell the
+        # newcomer counts are read and their prefix written, the old table,
+        # that prefix and the chain head read, the new tables and the cleared
         # counters written.
-        "sort": n * (4 + 4 + 1 + 8 + 4 + 4 + 8 + 2 * (48 + aux) + 4 + 4 + 1 + 4 + 16) + (cells + 1) * (8 + 8 + 8 + 8 + 4 + 24),
+        "sort": n * (4 + 4 + 4 + 2 * (48 + aux) + 4 + 4 + 1 + 4 + 16) + (cells + 1) * (8 + 8 + 8 + 8 + 4 + 24),
         "gather": 0,  # within the placement, as the cell table
         "cell_start": 0,
         # plist, own position (water: pm, sand: pph), water candidates' pph, rho/p (water);
@@ -89,8 +88,9 @@ def pass_bytes(n_w: int, n_s: int, nb: int, cells: int, multi: bool, listed=(0, 
         "water_momentum": n * 32 + n_w * (4 + 8 + 16) + 8 * (cells + 1)
                           + 4 * (cells + 1) + cells + nb * 16,
         # position, velocity, acc read; position, velocity written; sand colour;
-        # the next key written and the current sorted key read (change flag)
-        "advect": n * (16 * 3 + 16 * 2) + n_s * 16 + n * (4 + 4),
+        # the next key written, the current sorted key read (change flag), the
+        # stay prefix within the block written
+        "advect": n * (16 * 3 + 16 * 2) + n_s * 16 + n * (4 + 4 + 4),
     }
 
 

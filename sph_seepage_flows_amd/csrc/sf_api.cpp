@@ -142,7 +142,8 @@ int ensure_sort_capacity(sf_system* h, size_t m) {
     // clears them for the next)
     SF_HIP(hipMemsetAsync(h->icount.p, 0, h->icount.n * sizeof(uint32_t), h->stream));
     if ((rc = h->skeys[0].alloc(c)) || (rc = h->skeys[1].alloc(c)) || (rc = h->sperm.alloc(c)) ||
-        (rc = h->next.alloc(c)) || (rc = h->stay_pre.alloc(c + 1)))
+        (rc = h->next.alloc(c)) || (rc = h->local.alloc(c + 1)) || (rc = h->totals.alloc((c + kBlock - 1) / kBlock)) ||
+        (rc = h->stay_base.alloc((c + kBlock - 1) / kBlock + 1)))
         return rc;
     h->sort_cap = c;
     return ensure_cell_capacity(h);
@@ -160,7 +161,7 @@ int ensure_cell_capacity(sf_system* h) {
         // zero before the first incremental sort; afterwards every build clears them
         if ((rc = zero(h, h->in_count)) || (rc = zero(h, h->head[0])) || (rc = zero(h, h->head[1]))) return rc;
     }
-    const size_t np = (size_t)inc_parts((int)h->sort_cap, h->C);
+    const size_t np = (size_t)inc_parts(h->C);
     if (h->part2.n < np) {
         if ((rc = h->part2.alloc(np)) || (rc = zero(h, h->part2))) return rc;
     }
@@ -202,16 +203,16 @@ int build_neighbors(sf_system* h, hipEvent_t* ev) {
         a.g.perm = nullptr;
         a.key = h->keys.p;
         a.old_key = h->sorted_keys;
-        a.wflag_in = h->wflag.p;
         a.ct_old = h->ct[h->cur_ct].p;
-        a.stay_pre = h->stay_pre.p;
+        a.local = h->local.p;
+        a.stay_base = h->stay_base.p;
         a.in_start = h->in_start.p;
         a.in_count = h->in_count.p;
         a.head = h->head[h->cur_ct].p;
         a.next = h->next.p;
         a.head_next = h->head[h->cur_ct ^ 1].p;
         a.part = h->part2.p;
-        a.parts = inc_parts(n, h->C);
+        a.parts = inc_parts(h->C);
         a.perm = h->sperm.p;
         a.sorted_keys = out;
         a.plist = h->plist.p;
@@ -235,7 +236,7 @@ int build_neighbors(sf_system* h, hipEvent_t* ev) {
         SF_MARK(ev, SF_PASS_CELL_START);
         launch_cell_start(h->sorted_keys, n, h->C, h->wpre.p, h->cell.p, h->ct[h->cur_ct].p,
                           PhasePos{h->plist.p, g.pm_out, h->pph.p},
-                          IncClear{h->in_count.p, h->head[h->cur_ct].p, h->part2.p, inc_parts(n, h->C)}, s);
+                          IncClear{h->in_count.p, h->head[h->cur_ct].p, h->part2.p, inc_parts(h->C)}, s);
     }
     h->cur ^= 1;
     h->cur_cs ^= 1;

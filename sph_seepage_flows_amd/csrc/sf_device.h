@@ -221,22 +221,25 @@ SF_DEV v3 world_walls(const SFConst& k, v3 p, v3 v) {
 //   in_count[c]  particles whose key changed to c
 //   head, next   those particles chained: head[c] and next[i] hold 1 + a slot
 //                (0: end), with the slot's water flag in the top bit
-//   part         per tile of kMoveTile slots (tiles of slots, then of cells
-//                from part + cell_part on): the slots whose key did not change,
-//                and the newcomers of the tile's cells
+//   part         the newcomers of each tile of kMoveTile cells
+//   totals[b]    the slots of block b (kBlock slots) whose key did not change
+//   local[i]     those before slot i in its block (water << 16), i in [0, n]
+//                (not written for an n at a block's start: 0 by definition)
 struct Newcomers {
     uint64_t* in_count;
     uint32_t* head;
     uint32_t* next;
     uint64_t* part;
-    uint32_t cell_part;
+    uint64_t* totals;
+    uint32_t* local;
 };
 constexpr int kMoveTile = 2048;
 constexpr uint32_t kChainIndex = 0x7fffffffu;
-// Must be called by all threads of a kBlock block (kMoveTile is a multiple of
-// it); slot i = the thread's, not `valid` past the last.
-SF_DEV void count_moves(bool valid, uint32_t key, uint32_t old, bool water, int i, const Newcomers& nc) {
-    __shared__ uint32_t stays[kBlock / 64], wets[kBlock / 64];
+// Must be called by all threads of a kBlock block, slot i the thread's of n.
+SF_DEV void count_moves(uint32_t key, uint32_t old, bool water, int i, int n, const Newcomers& nc) {
+    __shared__ uint32_t stays[kBlock / 64];
+    const int w = (int)(threadIdx.x >> 6);
+    const bool valid = i < n;
     const bool move = valid && key != old;
     if (move) {
         atomicAdd((unsigned long long*)nc.in_count + key, water ? 0x100000001ull : 1ull);
@@ -244,30 +247,27 @@ SF_DEV void count_moves(bool valid, uint32_t key, uint32_t old, bool water, int 
     }
     // movers of a wave mostly go to cells of one tile: one atomic per tile
     uint64_t todo = __ballot(move);
-    const uint64_t wet = __ballot(water);
+    const uint64_t wet = __ballot(valid && water);
     while (todo) {
         const int lead = __builtin_ctzll(todo);
         const uint32_t tile = (uint32_t)__builtin_amdgcn_readlane((int)(key / (uint32_t)kMoveTile), lead);
         const uint64_t mine = __ballot(move && key / (uint32_t)kMoveTile == tile);
         if ((int)(threadIdx.x & 63u) == lead)
-            atomicAdd((unsigned long long*)nc.part + nc.cell_part + tile,
+            atomicAdd((unsigned long long*)nc.part + tile,
                       ((unsigned long long)__popcll(mine & wet) << 32) + (unsigned long long)__popcll(mine));
         todo &= ~mine;
     }
-    const uint64_t stay = __ballot(valid && !move);
-    if ((threadIdx.x & 63u) == 0) {
-        stays[threadIdx.x >> 6] = (uint32_t)__popcll(stay);
-        wets[threadIdx.x >> 6] = (uint32_t)__popcll(stay & wet);
-    }
+    const uint64_t stay = __ballot(valid && !move), below = (1ull << (threadIdx.x & 63u)) - 1ull;
+    auto count = [&](uint64_t m) { return (uint32_t)__popcll(m) | ((uint32_t)__popcll(m & wet) << 16); };
+    if ((threadIdx.x & 63u) == 0) stays[w] = count(stay);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t a = 0, b = 0;
-        for (int q = 0; q < kBlock / 64; ++q) {
-            a += stays[q];
-            b += wets[q];
-        }
-        if (a) atomicAdd((unsigned long long*)nc.part + i / kMoveTile, ((unsigned long long)b << 32) + a);
+    uint32_t before = count(stay & below), all = 0;
+    for (int q = 0; q < kBlock / 64; ++q) {
+        before += q < w ? stays[q] : 0u;
+        all += stays[q];
     }
+    if (i <= n) nc.local[i] = before;
+    if (threadIdx.x == 0) nc.totals[blockIdx.x] = ((uint64_t)(all >> 16) << 32) | (all & 0xffffu);
 }
 
 // Block mapping of a pass over two phases of a slot list: na blocks of phase

@@ -142,18 +142,18 @@ void launch_hash_boundary(const SFConst& k, const float4* bp, uint32_t* keys, in
 // sort's order).  ct_old is the previous cell table; nwater receives the
 // water count, cell / ct the new cellStart and cell table (C + 1 entries).
 struct PlaceArgs {
-    GatherArgs g;  // perm unused
+    GatherArgs g;  // perm unused; wflag read by the counting, written by the placement
     const uint32_t* key;
     const uint32_t* old_key;
-    const uint8_t* wflag_in;  // water flags of the current slots
     const uint2* ct_old;
-    uint64_t* stay_pre;  // n + 1
-    uint64_t* in_start;  // C + 1
+    const uint32_t* local;  // count_moves; the blocks' prefix goes to stay_base
+    uint64_t* stay_base;    // ceil(n / kBlock) + 1
+    uint64_t* in_start;     // C + 1
     uint64_t* in_count;  // C + 1, zero on entry of the counting, cleared here
     const uint32_t* head;
     const uint32_t* next;
     uint32_t* head_next;  // the next sort's heads, cleared here
-    uint64_t* part;       // inc_parts(n, C) tile sums, cleared here
+    uint64_t* part;       // inc_parts(C) tile sums, cleared here
     uint32_t parts;
     uint32_t* perm;
     uint32_t* sorted_keys;
@@ -166,7 +166,7 @@ struct PlaceArgs {
 // flags_done: the moves were already counted, by the advect that wrote key
 void launch_incremental_sort(const PlaceArgs& a, const Newcomers& nc, int n, uint32_t C, bool flags_done,
                              hipStream_t s);
-uint32_t inc_parts(int n, uint32_t C);
+uint32_t inc_parts(uint32_t C);
 // partial-sum counts of the prefix kernels
 int wprefix_blocks(int n);
 

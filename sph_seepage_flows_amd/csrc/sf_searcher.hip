@@ -387,7 +387,18 @@ template <class U>
 SF_DEV void block_sums(const U* __restrict__ cnt, uint32_t lo, uint32_t b, uint32_t hi, U& before, U& all) {
     __shared__ U red[2][kBlock / 64];
     U a = 0, p = 0;
-    for (uint32_t q = lo + threadIdx.x; q < hi; q += kBlock) {
+    uint32_t q = lo + threadIdx.x;
+    for (; q + 7u * kBlock < hi; q += 8u * kBlock) {  // eight loads in flight
+        U c[8];
+#pragma unroll
+        for (uint32_t m = 0; m < 8u; ++m) c[m] = cnt[q + m * kBlock];
+#pragma unroll
+        for (uint32_t m = 0; m < 8u; ++m) {
+            a += c[m];
+            p += q + m * kBlock < b ? c[m] : (U)0;
+        }
+    }
+    for (; q < hi; q += kBlock) {
         const U c = cnt[q];
         a += c;
         p += q < b ? c : (U)0;
@@ -447,58 +458,11 @@ struct NoEmit {
     SF_DEV void operator()(int, U, U) const {}
 };
 
-// Exclusive prefixes of two per-slot values, v1 over [0, n1) into out1[0, n1]
-// and v2 over [0, n2) into out2[0, n2], whose sums per tile of kWpTile slots
-// are in part (nb1 tiles of the first, then the second's).  Blocks [0, nb1)
-// work on the first, the others on the second.
-// scanned = 0: part holds the raw tile sums, and each block sums those
-// before it within its own prefix (the block holding slot n thereby ends on
-// the total, as the scan would give it).
-template <class V1, class V2>
-__global__ __launch_bounds__(kBlock) void k_vprefix2(V1 v1, int n1, int nb1, uint64_t* __restrict__ out1, V2 v2,
-                                                     int n2, uint64_t* __restrict__ out2,
-                                                     const uint64_t* __restrict__ part, int scanned) {
-    const int b = blockIdx.x;
-    uint64_t pb = 0;
-    if (scanned) {
-        pb = part[b];
-    } else {
-        uint64_t all;
-        if (b < nb1) block_sums(part, 0u, (uint32_t)b, (uint32_t)nb1, pb, all);
-        else block_sums(part, (uint32_t)nb1, (uint32_t)b, gridDim.x, pb, all);
-    }
-    if (b < nb1) tile_prefix(v1, n1, b, pb, out1, NoEmit{});
-    else tile_prefix(v2, n2, b - nb1, pb, out2, NoEmit{});
-}
 // Per-slot values of the prefixes; load8(i, f) reads slots i .. i + 7 (i a
 // multiple of 8, all below n) with vector loads.
-SF_DEV void load8_u32(const uint32_t* a, int i, uint4& x, uint4& y) {
-    x = *reinterpret_cast<const uint4*>(a + i);
-    y = *reinterpret_cast<const uint4*>(a + i + 4);
-}
 // A count of particles and, in the upper half, of the water among them
 // (counts stay below 2^27).
 SF_DEV uint64_t counted(bool one, bool water) { return one ? (water ? 0x100000001ull : 1ull) : 0ull; }
-struct StayVal {  // slots whose key did not change
-    const uint32_t* key;
-    const uint32_t* old;
-    const uint8_t* wflag;
-    SF_DEV uint64_t operator()(int i) const { return counted(key[i] == old[i], wflag[i] != 0); }
-    SF_DEV void load8(int i, uint64_t* f) const {
-        uint4 k0, k1, o0, o1;
-        load8_u32(key, i, k0, k1);
-        load8_u32(old, i, o0, o1);
-        const uint2 w = *reinterpret_cast<const uint2*>(wflag + i);
-        f[0] = counted(k0.x == o0.x, w.x & 0xffu);
-        f[1] = counted(k0.y == o0.y, w.x & 0xff00u);
-        f[2] = counted(k0.z == o0.z, w.x & 0xff0000u);
-        f[3] = counted(k0.w == o0.w, w.x & 0xff000000u);
-        f[4] = counted(k1.x == o1.x, w.y & 0xffu);
-        f[5] = counted(k1.y == o1.y, w.y & 0xff00u);
-        f[6] = counted(k1.z == o1.z, w.y & 0xff0000u);
-        f[7] = counted(k1.w == o1.w, w.y & 0xff000000u);
-    }
-};
 struct ArrayVal {
     const uint64_t* a;
     SF_DEV uint64_t operator()(int i) const { return a[i]; }
@@ -524,6 +488,31 @@ struct FlagVal {
     }
 };
 
+// Exclusive prefixes of the incremental sort: the blocks' totals over
+// [0, n1) into out1[0, n1] (blocks [0, nb1); there is one total per kBlock
+// slots, so each block sums all of those before its own itself), and the
+// newcomer counts over [0, n2) into out2[0, n2], whose sums per tile of
+// kWpTile cells are in part.
+// scanned = 0: part holds the raw tile sums, and each block sums those
+// before it within its own prefix (the block holding slot n thereby ends on
+// the total, as the scan would give it).
+__global__ __launch_bounds__(kBlock) void k_inc_prefix(const uint64_t* __restrict__ totals, int n1, int nb1,
+                                                       uint64_t* __restrict__ out1,
+                                                       const uint64_t* __restrict__ in_count, int n2,
+                                                       uint64_t* __restrict__ out2, const uint64_t* __restrict__ part,
+                                                       int scanned) {
+    const int b = (int)blockIdx.x - nb1;  // tile of the counts
+    uint64_t before = 0, all;
+    if (b < 0) {
+        const uint32_t first = blockIdx.x * (uint32_t)kWpTile;
+        block_sums(totals, 0u, first, first, before, all);
+        tile_prefix(ArrayVal{totals}, n1, (int)blockIdx.x, before, out1, NoEmit{});
+        return;
+    }
+    if (scanned) before = part[b];
+    else block_sums(part, 0u, (uint32_t)b, gridDim.x - (uint32_t)nb1, before, all);
+    tile_prefix(ArrayVal{in_count}, n2, b, before, out2, NoEmit{});
+}
 // Water prefix of the gathered slots (k_gather left the tile counts in
 // wpart) and the slots grouped by phase (water first, each group in slot
 // order) so that a pass over one phase can give every XCD an equal
@@ -586,7 +575,13 @@ __global__ __launch_bounds__(kBlock) void k_inc_flag(const uint32_t* __restrict_
                                                      const uint8_t* __restrict__ wflag, int n, Newcomers nc) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     const bool valid = i < n;
-    count_moves(valid, valid ? key[i] : 0u, valid ? old[i] : 0u, valid && wflag[i] != 0, i, nc);
+    count_moves(valid ? key[i] : 0u, valid ? old[i] : 0u, valid && wflag[i] != 0, i, n, nc);
+}
+// The slots before j whose key did not change (count_moves: the block's own
+// before it, and the blocks' totals before its block).
+SF_DEV uint64_t stay_before(const PlaceArgs& a, uint32_t j) {
+    const uint32_t l = j % (uint32_t)kBlock ? a.local[j] : 0u;
+    return a.stay_base[j / (uint32_t)kBlock] + (((uint64_t)(l >> 16) << 32) | (l & 0xffffu));
 }
 __global__ __launch_bounds__(kBlock) void k_inc_place(PlaceArgs a, int n, uint32_t C, int place_blocks) {
     if ((int)blockIdx.x >= place_blocks) {
@@ -594,7 +589,7 @@ __global__ __launch_bounds__(kBlock) void k_inc_place(PlaceArgs a, int n, uint32
         const uint32_t c = (blockIdx.x - (uint32_t)place_blocks) * kBlock + threadIdx.x;
         if (c < a.parts) a.part[c] = 0ull;
         if (c > C) return;
-        const uint64_t before = a.stay_pre[a.ct_old[c].x] + a.in_start[c];
+        const uint64_t before = stay_before(a, a.ct_old[c].x) + a.in_start[c];
         const uint2 e = make_uint2((uint32_t)before, (uint32_t)(before >> 32));
         a.cell[c] = e.x;
         a.ct[c] = e;
@@ -609,12 +604,12 @@ __global__ __launch_bounds__(kBlock) void k_inc_place(PlaceArgs a, int n, uint32
     const float4 pm = a.g.pm_in[i], vr = a.g.vr_in[i], cs = a.g.cs_in[i];
     const uint32_t oa = a.ct_old[c].x, ob = a.ct_old[c + 1].x;
     const uint64_t s = a.in_start[c], e = a.in_start[c + 1];
-    const uint64_t nwater = a.stay_pre[n] + a.in_start[C];  // all water, in the upper half
-    const uint64_t sa = a.stay_pre[oa];
+    const uint64_t nwater = stay_before(a, (uint32_t)n) + a.in_start[C];  // all water, in the upper half
+    const uint64_t sa = stay_before(a, oa);
     const uint32_t u = (uint32_t)i;
     uint64_t rank = 0;  // of the cell: stayers before, then newcomers before
-    if (c == o || (u >= oa && u < ob)) rank = a.stay_pre[u] - sa;
-    else if (u >= ob) rank = a.stay_pre[ob] - sa;
+    if (c == o || (u >= oa && u < ob)) rank = stay_before(a, u) - sa;
+    else if (u >= ob) rank = stay_before(a, ob) - sa;
     // the cell's chain is as long as its newcomer count; the count ends the walk
     uint32_t left = (uint32_t)e - (uint32_t)s;
     for (uint32_t q = left ? a.head[c] : 0u; q != 0u; q = a.next[(q & kChainIndex) - 1u]) {
@@ -642,21 +637,19 @@ __global__ __launch_bounds__(kBlock) void k_inc_place(PlaceArgs a, int n, uint32
     }
 }
 
-uint32_t inc_parts(int n, uint32_t C) { return (uint32_t)(wprefix_blocks(n + 1) + wprefix_blocks((int)C + 1)); }
+uint32_t inc_parts(uint32_t C) { return (uint32_t)wprefix_blocks((int)C + 1); }
 void launch_incremental_sort(const PlaceArgs& a, const Newcomers& nc, int n, uint32_t C, bool flags_done,
                              hipStream_t s) {
     if (n <= 0) return;
     const int gn = (n + kBlock - 1) / kBlock;
     // in_count, the chains and part are zero here: every build clears them
-    if (!flags_done) k_inc_flag<<<gn, kBlock, 0, s>>>(a.key, a.old_key, a.wflag_in, n, nc);
-    const int nb1 = wprefix_blocks(n + 1), nb2 = wprefix_blocks((int)C + 1);
-    const int scanned = nb1 + nb2 > g_direct_tiles ? 1 : 0;
-    if (scanned) k_rs_scan2<uint64_t><<<1, 1024, 0, s>>>(a.part, nb1, nb2, nullptr);
-    k_vprefix2<<<nb1 + nb2, kBlock, 0, s>>>(StayVal{a.key, a.old_key, a.wflag_in}, n, nb1, a.stay_pre,
-                                            ArrayVal{a.in_count}, (int)C, a.in_start, a.part, scanned);
-    uint32_t cells = C + 1;
-    if (a.parts > cells) cells = a.parts;
-    k_inc_place<<<gn + (int)((cells + kBlock - 1) / kBlock), kBlock, 0, s>>>(a, n, C, gn);
+    if (!flags_done) k_inc_flag<<<gn, kBlock, 0, s>>>(a.key, a.old_key, a.g.wflag, n, nc);
+    const int nb1 = wprefix_blocks(gn + 1), nb2 = (int)a.parts;
+    const int scanned = nb2 > g_direct_tiles ? 1 : 0;
+    if (scanned) k_rs_scan2<uint64_t><<<1, 1024, 0, s>>>(a.part, nb2, 0, nullptr);
+    k_inc_prefix<<<nb1 + nb2, kBlock, 0, s>>>(nc.totals, gn, nb1, a.stay_base, a.in_count, (int)C, a.in_start, a.part,
+                                              scanned);
+    k_inc_place<<<gn + (int)((C + 1 + kBlock - 1) / kBlock), kBlock, 0, s>>>(a, n, C, gn);
 }
 
 // in-range neighbour counts: r^2 = dx*dx + dy*dy + dz*dz in FP32, left to

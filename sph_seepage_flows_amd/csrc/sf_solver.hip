@@ -1311,7 +1311,7 @@ __global__ __launch_bounds__(kBlock) void k_advect(SFConst k, AdvectArgs a, int 
             is_water = p.w > 0.f;
         }
     }
-    if (a.keys_out) count_moves(i < n, key, old, is_water, i, a.nc);  // and its change flags (k_inc_flag)
+    if (a.keys_out) count_moves(key, old, is_water, i, n, a.nc);  // and its change flags (k_inc_flag)
 }
 void launch_advect(const SFConst& k, const AdvectArgs& a, int n, hipStream_t s) {
     if (n <= 0) return;

@@ -60,8 +60,8 @@ struct sf_system {
     DevBuf<uint2> ct[2];  // cell table: the incremental sort reads the previous one
     int cur_ct = 0;       // ct and head (the next advect's chains hang from head[cur_ct])
     // incremental sort (sf_set_sort_strategy): sorted-key ping-pong, permutation, work arrays
-    DevBuf<uint32_t> skeys[2], sperm, head[2], next;
-    DevBuf<uint64_t> stay_pre, in_count, in_start, part2;
+    DevBuf<uint32_t> skeys[2], sperm, head[2], next, local;
+    DevBuf<uint64_t> totals, stay_base, in_count, in_start, part2;
     bool sort_inc = true;
     size_t sort_cap = 0;
     const uint32_t* sorted_keys = nullptr;
@@ -165,7 +165,7 @@ struct sf_system {
     int parity() const { return cur | (cur_cs << 1) | (cur_aux << 2) | (cur_ct << 3); }
     // where the particles that change cell are counted for the next build
     Newcomers newcomers() const {
-        return Newcomers{in_count.p, head[cur_ct].p, next.p, part2.p, (uint32_t)wprefix_blocks((int)n + 1)};
+        return Newcomers{in_count.p, head[cur_ct].p, next.p, part2.p, totals.p, local.p};
     }
     // Two steps leave every buffer and flag where they found them, so that a
     // captured pair of steps can be replayed: with the incremental sort this
