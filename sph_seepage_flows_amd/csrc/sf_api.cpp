@@ -414,6 +414,7 @@ int fill_empty(sf_system* h) {
     if (!h->empty_pending) return SF_OK;
     Fields f = h->fields();
     f.nwater = h->wpre.p + h->n_built;
+    f.nw = -1;  // particles may have been emitted since
     launch_fill_empty(h->K, f, (int)h->n_built, h->stream);
     SF_HIP(hipGetLastError());
     h->empty_pending = false;
@@ -669,9 +670,11 @@ int sf_upload_particles(sf_handle h, size_t n, const float* pos3, const float* v
     std::vector<float2> amc(n);
     int wstate = 0;
     float wmass = 0.f;
+    size_t n_water = 0;
     for (size_t i = 0; i < n; ++i) {
         if (label[i] > 1) return set_error(SF_E_INVALID, "labels must be 0 (water) or 1 (sand)");
         if (!(mass[i] > 0.f) || !std::isfinite(mass[i])) return set_error(SF_E_INVALID, "masses must be finite and > 0");
+        n_water += label[i] == 0;
         if (label[i] == 0 && wstate == 0) {
             wstate = 1;
             wmass = mass[i];
@@ -702,6 +705,7 @@ int sf_upload_particles(sf_handle h, size_t n, const float* pos3, const float* v
     h->build_pending = false;
     h->water_mass_state = wstate;
     h->water_mass = wmass;
+    h->n_water = n_water;
     h->drop_graph();
     diff_release(h->diff);  // a recorded window no longer matches the particles
     h->diff = nullptr;

@@ -68,6 +68,7 @@ int append_water(sf_system* h, const std::vector<F3>& p) {
     SF_HIP(hipMemcpyAsync(h->amc[h->cur_aux].p + n, amc.data(), k * sizeof(float2), hipMemcpyHostToDevice, s));
     SF_HIP(hipStreamSynchronize(s));
     h->n = n + k;
+    h->n_water += k;
     if (k && h->water_mass_state == 0) {
         h->water_mass_state = 1;
         h->water_mass = h->P.sph_mass;

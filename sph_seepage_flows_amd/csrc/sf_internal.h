@@ -201,6 +201,10 @@ struct Fields {
     // slots, each in slot order; *nwater = nw (device)
     const uint32_t* plist;
     const uint32_t* nwater;
+    // nw where the host knows it (no caller holds the position, mass or label
+    // buffer: labels then change by uploads and emissions only, and
+    // pph[t] == pm[plist[t]] holds up to the advect), -1 otherwise
+    int nw;
     // pph[t] = pm[plist[t]]: positions and masses in phase order, so the
     // water candidates of a column range [s, e) are pph[wpre[s], wpre[e]) and
     // the sand ones pph[nw + s - wpre[s], nw + e - wpre[e])

@@ -36,6 +36,17 @@ SF_DEV float eos(const SFConst& k, float rho) {
     return p;
 }
 
+// The water count: a wave that knows it from its arguments, and its own
+// position (and in P4 velocity and saturation) from the phase order, starts
+// its walk two dependent loads earlier and reads contiguously: P4 257 -> 230
+// us and P1 189 -> 183 at 4M.  P5 keeps the slot's record, which it needs
+// anyway (with the position from the phase order 124 -> 127 us at 1M).
+SF_DEV uint32_t water_count(const Fields& f) { return f.nw >= 0 ? (uint32_t)f.nw : *f.nwater; }
+// Position and mass of the particle of phase index t in slot i.
+SF_DEV float4 own_pos(const Fields& f, uint32_t t, int i) {
+    return f.nw >= 0 ? ldo(f.pph, t) : ldo(f.pm, (uint32_t)i);
+}
+
 // First cell key of slot i's scene (batched handles), 0 otherwise.
 template <bool B>
 SF_DEV uint32_t scene_base(const SFConst& k, const Fields& f, int i) {
@@ -446,7 +457,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
     __shared__ float4 stage_lds[(NB / 64) * kStage];
     float4* stage = stage_lds + (threadIdx.x >> 6) * kStage;
     constexpr uint32_t PB = NB / kDenL;  // water particles per block
-    const uint32_t nw = *f.nwater, ns = (uint32_t)n - nw;
+    const uint32_t nw = water_count(f), ns = (uint32_t)n - nw;
     const PhaseBlock pb = phase_block((nw + PB - 1) / PB, (ns + NB - 1) / NB);
     if (pb.phase < 0) return;
     if (pb.phase == 1) {  // sand: rho_sand, p = 0; listed if a column range holds water
@@ -483,7 +494,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
     const bool lead = (threadIdx.x % kDenL) == 0;
     const bool water = t < nw;
     const int i = water ? (int)ldo(f.plist, t) : 0;
-    const float4 pi = water ? ldo(f.pm, (uint32_t)i) : make_float4(0.f, 0.f, 0.f, -1.f);
+    const float4 pi = water ? own_pos(f, t, i) : make_float4(0.f, 0.f, 0.f, -1.f);
     const uint32_t cb = water ? scene_base<B>(k, f, i) : 0u;
     int cx, cy, cz;
     cell_of(k, pi.x, pi.y, pi.z, cx, cy, cz);
@@ -582,7 +593,7 @@ __global__ void k_zero_counts(uint32_t* __restrict__ c) {
 }
 template <bool B>
 __global__ __launch_bounds__(kBlock) void k_interface(SFConst k, Fields f, int n) {
-    const uint32_t nw = *f.nwater, ns = (uint32_t)n - nw;
+    const uint32_t nw = water_count(f), ns = (uint32_t)n - nw;
     const PhaseBlock pb = phase_block((nw + kBlock - 1) / kBlock, (ns + kBlock - 1) / kBlock);
     if (pb.phase < 0) return;
     const bool sand_i = pb.phase == 1;
@@ -614,7 +625,7 @@ __global__ __launch_bounds__(kBlock) void k_interface(SFConst k, Fields f, int n
 __global__ __launch_bounds__(kBlock) void k_fill_empty(SFConst k, Fields f, int n) {
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
     if (t >= (uint32_t)n) return;
-    const uint32_t nw = *f.nwater;
+    const uint32_t nw = water_count(f);
     const bool sand = t >= nw;
     const int i = (int)ldo(f.plist, t);
     if (sand) f.rp[i] = make_float2(k.rho_s, 0.f);
@@ -673,14 +684,14 @@ template <bool B, int NB, int CAP, int LP>
 __global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
     SF_NLIST(L);
     SF_STAGE(stage, kStageList);
-    const uint32_t nw = *f.nwater;
+    const uint32_t nw = water_count(f);
     PhaseSlot<NB, LP> ps;
     const bool active = phase_slot(f, nw, ps);
     if (!__ballot(active)) return;  // the other lanes of a wave help to stage its candidates
     const int i = ps.i;
     const uint32_t sub = ps.sub;
     const bool sand_i = ps.sand;
-    const float4 pi = ldo(f.pm, (uint32_t)i);
+    const float4 pi = own_pos(f, ps.t, i);
     const uint32_t cb = scene_base<B>(k, f, i);
     int cx, cy, cz;
     cell_of(k, pi.x, pi.y, pi.z, cx, cy, cz);
@@ -749,13 +760,13 @@ template <bool B, int NB, int CAP, int LP>
 __global__ __launch_bounds__(NB) void k_voidage_adhesion(SFConst k, Fields f, int n) {
     SF_NLIST(L);
     SF_STAGE(stage, kStageList);
-    const uint32_t nw = *f.nwater;
+    const uint32_t nw = water_count(f);
     PhaseSlot<NB, LP> ps;
     const bool active = phase_slot(f, nw, ps);
     if (!__ballot(active)) return;
     const int i = ps.i;
     const uint32_t sub = ps.sub;
-    const float4 pi = ldo(f.pm, (uint32_t)i);
+    const float4 pi = own_pos(f, ps.t, i);
     const uint32_t cb = scene_base<B>(k, f, i);
     int cx, cy, cz;
     cell_of(k, pi.x, pi.y, pi.z, cx, cy, cz);
@@ -864,15 +875,15 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
     SF_NLIST(L);
     SF_STAGE(stage, kStageList);
     constexpr uint32_t PB = NB / kSmL;  // sand particles per block
-    const uint32_t nw = *f.nwater, ns = (uint32_t)n - nw;
+    const uint32_t nw = water_count(f), ns = (uint32_t)n - nw;
     const PhaseBlock pb = phase_block(0u, (ns + PB - 1) / PB);
     const uint32_t t = pb.blk * PB + threadIdx.x / kSmL;
     const uint32_t sub = threadIdx.x % kSmL;  // this lane's share of the particle's candidates
     if (pb.phase < 0) return;  // the whole block
     // lanes past the last grain help to stage their wave's water candidates
     const int i = t < ns ? (int)ldo(f.plist, nw + t) : 0;
-    const uint32_t self = nw + t;  // this particle's phase index
-    const float4 pi = ldo(f.pm, (uint32_t)i);
+    const uint32_t self = t < ns ? nw + t : 0u;  // this particle's phase index
+    const float4 pi = own_pos(f, self, i);
     const bool active = t < ns && pi.w < 0.f;
     if (!__ballot(active)) return;
     const uint32_t cb = scene_base<B>(k, f, i);
@@ -885,10 +896,11 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
     }
     const float mi = -pi.w;
     const v3 xi = xyz(pi);
-    const v3 vi = xyz(ldo(f.vr, (uint32_t)i));
+    const float4 vsi = ldo(f.vq, self);  // velocity, saturation
+    const v3 vi = xyz(vsi);
     const float rho_i = k.rho_s;  // the density pass's value for every grain
     const float2 esi = ldo(f.es, (uint32_t)i);
-    const float sat_i = esi.y;
+    const float sat_i = vsi.w;
     const float twoR = 2.f * k.R;
     const float cap_r = twoR + k.cap_srup;
     const float cap_r2 = cap_r * cap_r;
@@ -1066,7 +1078,7 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     // into counters that start at zero
     if (blockIdx.x == 0 && threadIdx.x < 2) f.icount[threadIdx.x * kCountStride] = 0u;
     constexpr uint32_t PB = NB / kWmL;  // water particles per block
-    const uint32_t nw = *f.nwater;
+    const uint32_t nw = water_count(f);
     const PhaseBlock pb = phase_block((nw + PB - 1) / PB, 0u);
     if (pb.phase < 0) return;  // the whole block
     const uint32_t t = pb.blk * PB + threadIdx.x / kWmL;

@@ -74,6 +74,7 @@ struct sf_system {
     // 2 not all equal (set by the upload and the emitter)
     int water_mass_state = 0;
     float water_mass = 0.f;
+    size_t n_water = 0;  // water particles, as uploaded and emitted
     // the neighbour records are used while the water masses are equal and
     // known on the host (a caller holding the position / mass buffer may
     // change them)
@@ -145,6 +146,7 @@ struct sf_system {
         f.sct = nscenes ? sct.p : nullptr;
         f.plist = plist.p;
         f.nwater = wpre.p + n;
+        f.nw = pm_shared ? -1 : (int)n_water;
         f.pph = pph.p;
         f.ilist = ilist.p;
         f.icount = icount.p;
