@@ -279,8 +279,8 @@ struct PhaseBlock {
     int phase;
     uint32_t blk;  // block within the phase
 };
-SF_DEV PhaseBlock phase_block(uint32_t na, uint32_t nb) {
-    const uint32_t b = blockIdx.x, x = b & 7u, l = b >> 3;
+SF_DEV PhaseBlock phase_block(uint32_t na, uint32_t nb, uint32_t b = blockIdx.x) {
+    const uint32_t x = b & 7u, l = b >> 3;
     const uint32_t qa = na >> 3, ra = na & 7u, qb = nb >> 3, rb = nb & 7u;
     const uint32_t ca = qa + (x < ra ? 1u : 0u), cbn = qb + (x < rb ? 1u : 0u);
     if (l < ca) return {0, x * qa + (x < ra ? x : ra) + l};

@@ -651,14 +651,11 @@ struct PhaseSlot {
 // The listed particle of this thread (false: none; slot and phase index 0
 // then, the phase still the block's).
 template <int NB, int LP>
-SF_DEV bool phase_slot(const Fields& f, uint32_t nw, PhaseSlot<NB, LP>& ps) {
+SF_DEV bool phase_slot(const Fields& f, uint32_t nw, uint32_t cw, uint32_t cs, PhaseBlock pb, PhaseSlot<NB, LP>& ps) {
     constexpr uint32_t PB = NB / LP;  // particles per block
-    const uint32_t cw = f.icount[0], cs = f.icount[kCountStride];
-    const PhaseBlock pb = phase_block((cw + PB - 1) / PB, (cs + PB - 1) / PB);
     ps.i = 0;
     ps.t = 0;
     ps.sand = pb.phase == 1;
-    if (pb.phase < 0) return false;
     const uint32_t q = pb.blk * PB + threadIdx.x / LP;
     ps.sub = threadIdx.x % LP;
     if (q >= (ps.sand ? cs : cw)) return false;
@@ -666,8 +663,31 @@ SF_DEV bool phase_slot(const Fields& f, uint32_t nw, PhaseSlot<NB, LP>& ps) {
     ps.i = (int)ldo(f.plist, ps.t);
     return true;
 }
-// enough blocks for every particle listed
-inline int phase_slot_grid(int n, int lanes, int nb) { return phase_grid(n * lanes, nb); }
+// body(phase_block) for the blocks of listed particles this block takes.  How
+// much is listed is known on the device only, and a block for every particle
+// that could be listed launches mostly waves that find nothing to do where
+// the interface is thin (250k of them at 4M: 2 x 31 us).  The grid stops at
+// kListBlocks, a multiple of 8 so that a block stays on its XCD's share, and
+// each block takes every kListBlocks-th block of the mapping.
+constexpr int kListBlocks = 16384;
+inline int list_grid(int n, int lanes, int nb) {
+    const int all = phase_grid(n * lanes, nb);
+    return all < kListBlocks ? all : kListBlocks;
+}
+template <int NB, int LP, class Body>
+SF_DEV void for_listed(const Fields& f, Body&& body) {
+    constexpr uint32_t PB = NB / LP;  // particles per block
+    const uint32_t cw = f.icount[0], cs = f.icount[kCountStride];
+    const uint32_t na = (cw + PB - 1) / PB, nb = (cs + PB - 1) / PB;
+    uint32_t b = blockIdx.x;
+    PhaseBlock pb = phase_block(na, nb, b);
+    if (pb.phase < 0) return;  // before the loop: nothing it hoists is waited for
+    do {
+        body(cw, cs, pb);
+        b += gridDim.x;
+        pb = phase_block(na, nb, b);
+    } while (pb.phase >= 0);  // past the share's end, so are all later ones
+}
 
 // ---------------------------------------------------------------------------
 // P2 (ComputeSFAvgFlow_CUDA): water i -> voidage 1 - sum_sand V W and the
@@ -681,12 +701,10 @@ inline int phase_slot_grid(int n, int lanes, int nb) { return phase_grid(n * lan
 // fetches each kept neighbour's fields (by phase index u: every neighbour
 // within h is listed, see Fields::vq) ahead of its use.
 template <bool B, int NB, int CAP, int LP>
-__global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
-    SF_NLIST(L);
-    SF_STAGE(stage, kStageList);
-    const uint32_t nw = water_count(f);
+SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float4* __restrict__ stage, uint32_t nw,
+                     uint32_t cw, uint32_t cs, PhaseBlock pb) {
     PhaseSlot<NB, LP> ps;
-    const bool active = phase_slot(f, nw, ps);
+    const bool active = phase_slot(f, nw, cw, cs, pb, ps);
     if (!__ballot(active)) return;  // the other lanes of a wave help to stage its candidates
     const int i = ps.i;
     const uint32_t sub = ps.sub;
@@ -743,12 +761,21 @@ __global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
         reinterpret_cast<float*>(f.wq)[4 * ps.t + 2] = eps_i;
     }
 }
+template <bool B, int NB, int CAP, int LP>
+__global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
+    SF_NLIST(L);
+    SF_STAGE(stage, kStageList);
+    const uint32_t nw = water_count(f);
+    for_listed<NB, LP>(f, [&](uint32_t cw, uint32_t cs, PhaseBlock pb) {
+        avg_flow<B, NB, CAP, LP>(k, f, L, stage, nw, cw, cs, pb);
+    });
+}
 void launch_avg_flow(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
     if (n <= 0) return;
     dispatch(f, c, [&](auto B, auto NB, auto CAP) {
         with_lanes(c.lanes, [&](auto LP) {
             k_avg_flow<decltype(B)::value, decltype(NB)::value, decltype(CAP)::value, decltype(LP)::value>
-                <<<phase_slot_grid(n, LP, NB), (int)NB, 0, s>>>(k, f, n);
+                <<<list_grid(n, LP, NB), (int)NB, 0, s>>>(k, f, n);
         });
     });
 }
@@ -757,12 +784,10 @@ void launch_avg_flow(const SFConst& k, const Fields& f, int n, PassCfg c, hipStr
 // P3: sand i -> voidage from water neighbours; water i -> adhesion force.
 // Same walk as P2.
 template <bool B, int NB, int CAP, int LP>
-__global__ __launch_bounds__(NB) void k_voidage_adhesion(SFConst k, Fields f, int n) {
-    SF_NLIST(L);
-    SF_STAGE(stage, kStageList);
-    const uint32_t nw = water_count(f);
+SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float4* __restrict__ stage,
+                             uint32_t nw, uint32_t cw, uint32_t cs, PhaseBlock pb) {
     PhaseSlot<NB, LP> ps;
-    const bool active = phase_slot(f, nw, ps);
+    const bool active = phase_slot(f, nw, cw, cs, pb, ps);
     if (!__ballot(active)) return;
     const int i = ps.i;
     const uint32_t sub = ps.sub;
@@ -850,12 +875,21 @@ __global__ __launch_bounds__(NB) void k_voidage_adhesion(SFConst k, Fields f, in
     f.wbq[ps.t] = make_float4(pi.x, pi.y, pi.z, a);
     if (f.den4) reinterpret_cast<float*>(f.den4)[4 * i + 1] = vs;
 }
+template <bool B, int NB, int CAP, int LP>
+__global__ __launch_bounds__(NB) void k_voidage_adhesion(SFConst k, Fields f, int n) {
+    SF_NLIST(L);
+    SF_STAGE(stage, kStageList);
+    const uint32_t nw = water_count(f);
+    for_listed<NB, LP>(f, [&](uint32_t cw, uint32_t cs, PhaseBlock pb) {
+        voidage_adhesion<B, NB, CAP, LP>(k, f, L, stage, nw, cw, cs, pb);
+    });
+}
 void launch_voidage_adhesion(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
     if (n <= 0) return;
     dispatch(f, c, [&](auto B, auto NB, auto CAP) {
         with_lanes(c.lanes, [&](auto LP) {
             k_voidage_adhesion<decltype(B)::value, decltype(NB)::value, decltype(CAP)::value, decltype(LP)::value>
-                <<<phase_slot_grid(n, LP, NB), (int)NB, 0, s>>>(k, f, n);
+                <<<list_grid(n, LP, NB), (int)NB, 0, s>>>(k, f, n);
         });
     });
 }
