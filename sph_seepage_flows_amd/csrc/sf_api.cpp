@@ -279,6 +279,7 @@ int advect(sf_system* h, float dt, const CflOut* dt_dev, hipEvent_t* ev) {
     a.vr_out = h->vr[h->cur ^ 1].p;
     a.bpv = h->bpv.p;
     a.bcell = h->bcell.p;
+    a.bnear = h->bnear.p;
     a.dt = dt;
     a.dt_dev = dt_dev;
     // the next build's hash and change flags, when it will be incremental
@@ -740,12 +741,22 @@ int sf_upload_boundary(sf_handle h, size_t nb, const float* pos3, const uint64_t
     launch_cell_start(sk, (int)nb, h->local_cells(), nullptr, h->bcell.p, nullptr, PhasePos{}, IncClear{}, h->stream);
     launch_boundary_gather(bperm, tmp.p, h->bpv.p, (int)nb, h->stream);
     launch_boundary_volume(h->K, h->bpv.p, h->bcell.p, (int)nb, h->stream);
-    launch_boundary_near(h->K, h->bcell.p, h->bnear.p, h->stream);
-    SF_HIP(hipGetLastError());
-    SF_HIP(hipStreamSynchronize(h->stream));
-    h->nb = nb;
     h->blabel1 = l1;
     h->K = make_const(h->P, h->B, h->O, h->blabel1);
+    {  // the cells near it and their columns' ranges
+        DevBuf<unsigned long long> sums;
+        unsigned long long total = 0;
+        if ((rc = sums.alloc(2)) || (rc = zero(h, sums))) return rc;
+        launch_boundary_near(h->K, h->bpv.p, h->bcell.p, h->bnear.p, sums.p, h->stream);
+        SF_HIP(hipMemcpyAsync(&total, sums.p, sizeof(total), hipMemcpyDeviceToHost, h->stream));
+        SF_HIP(hipStreamSynchronize(h->stream));
+        if (total > 0xffffffffull) return set_error(SF_E_CAPACITY, "too many cells near the boundary");
+        if ((rc = h->brange.alloc((size_t)total)) || (rc = h->brow.alloc(h->local_cells()))) return rc;
+        launch_boundary_rows(h->K, h->bcell.p, h->bnear.p, h->brow.p, h->brange.p, sums.p + 1, h->stream);
+        SF_HIP(hipGetLastError());
+        SF_HIP(hipStreamSynchronize(h->stream));
+    }
+    h->nb = nb;
     h->built = false;  // the particle searcher buffers were reused
     h->build_pending = false;
     h->drop_graph();

@@ -130,9 +130,13 @@ void launch_gather_wprefix(const GatherArgs& a, int n, uint32_t* wpart, uint32_t
                            hipStream_t s);
 void launch_boundary_gather(const uint32_t* perm, const float4* bp_in, float4* bp_out, int nb, hipStream_t s);
 void launch_boundary_volume(const SFConst& k, float4* bpv, const uint32_t* bcs, int nb, hipStream_t s);
-// near[c] for every local cell c: whether any of its 9 neighbour column
-// ranges of the boundary cellStart bcs is non-empty.
-void launch_boundary_near(const SFConst& k, const uint32_t* bcs, uint8_t* near, hipStream_t s);
+// near[c] for every local cell c (Fields::bnear) and the sum of its column
+// counts in *total; then the rows of those columns' ranges (Fields::brow,
+// brange, *total entries).  total and next zero on entry.
+void launch_boundary_near(const SFConst& k, const float4* bpv, const uint32_t* bcs, uint8_t* near,
+                          unsigned long long* total, hipStream_t s);
+void launch_boundary_rows(const SFConst& k, const uint32_t* bcs, const uint8_t* near, uint32_t* row, uint2* ranges,
+                          unsigned long long* next, hipStream_t s);
 void launch_nbr_count(const SFConst& k, const float4* pm, const uint16_t* scene, const uint32_t* cs, uint32_t* cnt,
                       uint32_t* cand, int n, hipStream_t s);
 void launch_hash_boundary(const SFConst& k, const float4* bp, uint32_t* keys, int nb, hipStream_t s);
@@ -180,9 +184,13 @@ struct Fields {
     const uint2* ct;  // (cellStart[c], water prefix at cellStart[c]), c in [0, C]
     const float4* bpv;
     const uint32_t* bcell;
-    // bnear[c] = 1 when a boundary particle lies in cell c's 27-cell
-    // neighbourhood (local cell keys; set at boundary upload)
+    // bnear[c] (local cell keys, set at boundary upload): 0, or 1 when a
+    // boundary particle lies in cell c's 27-cell neighbourhood, + 2 when one
+    // of label 1 does, + 16 x the number of its columns that hold any; those
+    // columns' ranges of bpv are brange[brow[c] ..), in for_columns order
     const uint8_t* bnear;
+    const uint32_t* brow;
+    const uint2* brange;
     float2* rp;
     float2* es;
     float2* wt;  // water: (rho / max(eps, voidage), p / max(eps, (rho / max(eps, voidage))^2))
@@ -318,6 +326,7 @@ struct AdvectArgs {
     float4* vr_out;
     const float4* bpv;
     const uint32_t* bcell;
+    const uint8_t* bnear;
     float dt;
     const CflOut* dt_dev;  // when non-null, dt = ri / nsub from the device
     // The next neighbour build's hash and change flags, written here from the

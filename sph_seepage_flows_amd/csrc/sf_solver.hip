@@ -418,36 +418,38 @@ SF_DEV void list_interface(const Fields& f, bool listed, bool sand, uint32_t t, 
 // rho_sand and p = 0.  Only water candidates are walked (sand adds nothing);
 // branch-free: max(h^2 - r^2, 0) vanishes outside the support.  The kDenL
 // lanes of a particle split both the candidates and the boundary particles.
-// The boundary particles of the 27 cells around (cx, cy, cz) for lane sub
-// of L lanes per particle: fn(b) for j = s + sub + L m of each column's
-// range [s, e), columns in for_columns order and j increasing (the order of
-// a plain walk).  The nine ranges, then each range's first candidate of the
-// lane, are loaded together: a lane near a wall has about one candidate per
-// column, so a column-by-column walk waited on three dependent loads per
-// column.
+// The boundary particles of the 27 cells around a cell for lane sub of L
+// lanes per particle: fn(b) for j = s + sub + L m of each column's range
+// [s, e), columns in for_columns order and j increasing (the order of a plain
+// walk of the 9 columns; near = bnear[cell] counts those that hold any).
+// Three columns' ranges, then the lane's first three candidates of each, are
+// loaded together: a face cell's 3 columns take two round trips (P5 124 -> 117
+// us at 1M against all nine columns' ranges and first candidates; P1 60 -> 57,
+// one column's range ahead).
 template <int L, class Fn>
-SF_DEV void boundary_walk(const SFConst& k, const Fields& f, int cx, int cy, int cz, uint32_t sub, Fn&& fn) {
-    const int zlo = cz > 0 ? cz - 1 : 0;
-    const int zhi = cz + 1 < k.gz ? cz + 1 : k.gz - 1;
-    uint32_t s[9], e[9];
+SF_DEV void boundary_walk(const Fields& f, uint32_t near, uint32_t cell, uint32_t sub, Fn&& fn) {
+    const uint32_t n = near >> 4, row = ldo(f.brow, cell);
+    for (uint32_t q = 0; q < n; q += 3u) {
+        uint2 r[3];
+        float4 b[3][3];
 #pragma unroll
-    for (int q = 0; q < 9; ++q) {
-        const int x = cx + q / 3 - 1, y = cy + q % 3 - 1;
-        s[q] = 0u;
-        e[q] = 0u;
-        if (x >= 0 && x < k.gx && y >= 0 && y < k.gy) {
-            const uint32_t base = (uint32_t)((x * k.gy + y) * k.gz);
-            s[q] = ldo(f.bcell, base + (uint32_t)zlo) + sub;
-            e[q] = ldo(f.bcell, base + (uint32_t)zhi + 1u);
+        for (uint32_t m = 0; m < 3u; ++m) {
+            r[m] = q + m < n ? ldo(f.brange, row + q + m) : make_uint2(0u, 0u);
+            r[m].x += sub;
         }
-    }
-    float4 b0[9];
 #pragma unroll
-    for (int q = 0; q < 9; ++q) b0[q] = s[q] < e[q] ? ldo(f.bpv, s[q]) : make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int m = 0; m < 3; ++m)
 #pragma unroll
-    for (int q = 0; q < 9; ++q) {
-        if (s[q] < e[q]) fn(b0[q]);
-        for (uint32_t j = s[q] + (uint32_t)L; j < e[q]; j += (uint32_t)L) fn(ldo(f.bpv, j));
+            for (uint32_t t = 0; t < 3u; ++t)
+                b[m][t] = r[m].x + t * (uint32_t)L < r[m].y ? ldo(f.bpv, r[m].x + t * (uint32_t)L)
+                                                            : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+#pragma unroll
+            for (uint32_t t = 0; t < 3u; ++t)
+                if (r[m].x + t * (uint32_t)L < r[m].y) fn(b[m][t]);
+            for (uint32_t j = r[m].x + 3u * (uint32_t)L; j < r[m].y; j += (uint32_t)L) fn(ldo(f.bpv, j));
+        }
     }
 }
 
@@ -536,19 +538,25 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
             for (; j < b.y; j += kDenL) add(j, ldo(f.pph, j));
         });
     }
-    if (water && ldo(f.bnear, cell_key(k, cx, cy, cz))) {  // boundary particles within the 27 cells
+    const uint32_t cell = cell_key(k, cx, cy, cz);
+    const uint32_t near = water ? ldo(f.bnear, cell) : 0u;
+    if (near) {  // boundary particles within the 27 cells
         const uint32_t sub = threadIdx.x % kDenL;
         auto badd = [&](const float4& b) {
             const float dx = pi.x - b.x, dy = pi.y - b.y, dz = pi.z - b.z;
             const float d = fmaxf(k.h2 - (dx * dx + dy * dy + dz * dz), 0.f);
             sb += fabsf(b.w) * sq3(d);
         };
-        // column by column (this pass keeps its registers low), four
-        // candidates' loads in flight at a time, summed in increasing j
-        for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
-            const uint32_t be = ldo(f.bcell, c1);
-            uint32_t j = ldo(f.bcell, c0) + sub;
-            for (; j + 3u * kDenL < be; j += 4u * kDenL) {
+        // the columns that hold any, one after another (this pass keeps its
+        // registers low), the next one's range and four candidates' loads in
+        // flight at a time, summed in increasing j
+        const uint32_t n = near >> 4, row = ldo(f.brow, cell);
+        uint2 next = ldo(f.brange, row);
+        for (uint32_t q = 0; q < n; ++q) {
+            const uint2 r = next;
+            next = ldo(f.brange, row + (q + 1u < n ? q + 1u : q));
+            uint32_t j = r.x + sub;
+            for (; j + 3u * kDenL < r.y; j += 4u * kDenL) {
                 const float4 b0 = ldo(f.bpv, j), b1 = ldo(f.bpv, j + kDenL), b2 = ldo(f.bpv, j + 2u * kDenL),
                              b3 = ldo(f.bpv, j + 3u * kDenL);
                 badd(b0);
@@ -556,8 +564,8 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
                 badd(b2);
                 badd(b3);
             }
-            for (; j < be; j += kDenL) badd(ldo(f.bpv, j));
-        });
+            for (; j < r.y; j += kDenL) badd(ldo(f.bpv, j));
+        }
     }
 #pragma unroll
     for (int o = 1; o < kDenL; o <<= 1) {
@@ -1017,15 +1025,12 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
         fetch_water, water);
     nl_flush2(L, fetch_water, water);
     if (!active) return;
-    if (k.blabel1 && ldo(f.bnear, cell_key(k, cx, cy, cz))) {  // ComputeSFUniRadiusDemBoundaryForces: label 1 only
-        for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
-            const uint32_t be = ldo(f.bcell, c1);
-            for (uint32_t j = ldo(f.bcell, c0) + sub; j < be; j += kSmL) {
-                const float4 b = ldo(f.bpv, j);
-                if (b.w >= 0.f) continue;
-                fsum += dem_force(xi - xyz(b), -vi, twoR, k.kn, k.ks, k.tan2);
-            }
-        });
+    if (k.blabel1) {  // ComputeSFUniRadiusDemBoundaryForces: label 1 only
+        const uint32_t cell = cell_key(k, cx, cy, cz), near = ldo(f.bnear, cell);
+        if (near & 2u)
+            boundary_walk<kSmL>(f, near, cell, sub, [&](const float4& b) {
+                if (b.w < 0.f) fsum += dem_force(xi - xyz(b), -vi, twoR, k.kn, k.ks, k.tan2);
+            });
     }
 #pragma unroll
     for (int o = 1; o < kSmL; o <<= 1) {
@@ -1173,8 +1178,9 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
         in_range, fetch, pair);
     nl_flush2(L, fetch, pair);
     if (!active) return;
-    if (ldo(f.bnear, cell_key(k, cx, cy, cz))) {  // boundary particles within the 27 cells
-        boundary_walk<kWmL>(k, f, cx, cy, cz, sub, [&](const float4& b) {
+    const uint32_t cell = cell_key(k, cx, cy, cz);
+    if (const uint32_t near = ldo(f.bnear, cell)) {  // boundary particles within the 27 cells
+        boundary_walk<kWmL>(f, near, cell, sub, [&](const float4& b) {
             const v3 d = mk3(pi.x - b.x, pi.y - b.y, pi.z - b.z);
             const float r2 = dot(d, d);
             if (r2 >= k.h2) return;
@@ -1329,17 +1335,26 @@ __global__ __launch_bounds__(kBlock) void k_advect(SFConst k, AdvectArgs a, int 
             if (k.blabel1) {
                 int cx, cy, cz;
                 cell_of(k, pre.x, pre.y, pre.z, cx, cy, cz);
-                for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
+                // only where a label-1 particle is near: four candidates' loads
+                // in flight, in increasing j
+                const bool collider = a.bnear[cell_key(k, cx, cy, cz)] & 2u;
+                if (collider) for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
                     const uint32_t be = a.bcell[c1];
-                    for (uint32_t j = a.bcell[c0]; j < be; ++j) {
-                        const float4 b = a.bpv[j];
-                        if (b.w >= 0.f) continue;
-                        const v3 dp = pre - xyz(b);
-                        const float dl = sqrtf(dot(dp, dp));
-                        const float ov = dl - r2;
-                        if (ov < 0.f) {
-                            nv = nv * 0.f;
-                            np += dp * (1.f / dl) * (-ov);
+                    for (uint32_t j0 = a.bcell[c0]; j0 < be; j0 += 4u) {
+                        float4 q[4];
+#pragma unroll
+                        for (uint32_t m = 0; m < 4u; ++m) q[m] = a.bpv[j0 + m < be ? j0 + m : j0];
+#pragma unroll
+                        for (uint32_t m = 0; m < 4u; ++m) {
+                            const float4 b = q[m];
+                            if (j0 + m >= be || b.w >= 0.f) continue;
+                            const v3 dp = pre - xyz(b);
+                            const float dl = sqrtf(dot(dp, dp));
+                            const float ov = dl - r2;
+                            if (ov < 0.f) {
+                                nv = nv * 0.f;
+                                np += dp * (1.f / dl) * (-ov);
+                            }
                         }
                     }
                 });

@@ -54,6 +54,8 @@ struct sf_system {
     bool empty_pending = false;
     size_t n_built = 0;
     DevBuf<uint8_t> bnear;            // cells with boundary particles near (Fields::bnear)
+    DevBuf<uint32_t> brow;            // their columns' ranges (Fields::brange)
+    DevBuf<uint2> brange;
     DevBuf<float4> vq, wq, xq, wbq;   // listed particles' fields by phase index (Fields::wq)
     DevBuf<float4> rec0, rec1;        // water momentum neighbour records (Fields::rec0)
     DevBuf<uint8_t> wflag;
@@ -134,6 +136,8 @@ struct sf_system {
         f.bpv = bpv.p;
         f.bcell = bcell.p;
         f.bnear = bnear.p;
+        f.brow = brow.p;
+        f.brange = brange.p;
         f.rp = rp.p;
         f.es = es.p;
         f.wt = wt.p;
