@@ -136,7 +136,8 @@ int ensure_sort_capacity(sf_system* h, size_t m) {
     if ((rc = h->wpre.alloc(c + 1)) || (rc = h->wpart.alloc((size_t)wprefix_blocks((int)c + 1) + 1)) ||
         (rc = h->plist.alloc(c)) || (rc = h->wflag.alloc(c)) || (rc = h->pph.alloc(c)) || (rc = h->ilist.alloc(c)) ||
         (rc = h->icount.alloc(2 * kCountStride)) || (rc = h->iface.alloc(c)) || (rc = h->wl.alloc(c)) || (rc = h->vq.alloc(c)) || (rc = h->wq.alloc(c)) ||
-        (rc = h->xq.alloc(c)) || (rc = h->wbq.alloc(c)) || (rc = h->rec0.alloc(c)) || (rc = h->rec1.alloc(c)))
+        (rc = h->xq.alloc(c)) || (rc = h->wbq.alloc(c)) || (rc = h->rec0.alloc(c)) || (rc = h->rec1.alloc(c)) ||
+        (rc = h->nl.alloc(saved_entries(c))) || (rc = h->nlc.alloc(4 * c + 2 * 64)) || (rc = h->nlq.alloc(c)))
         return rc;
     // the interface counters start at zero (each step's water momentum pass
     // clears them for the next)
@@ -178,6 +179,7 @@ int build_neighbors(sf_system* h, hipEvent_t* ev) {
     const bool inc = h->sort_inc && h->built && h->sorted_keys && n > 0;
     const bool fused = inc && h->keys_fresh;  // the last advect hashed and counted the moves
     h->keys_fresh = false;
+    h->pph_current = true;
     SF_MARK(ev, SF_PASS_HASH);
     if (!fused) launch_hash(h->K, h->pm[h->cur].p, h->nscenes ? h->scene.p : nullptr, h->keys.p, h->wflag.p, n, s);
     GatherArgs g;
@@ -905,6 +907,7 @@ int sf_update_solver(sf_handle h, float render_interval, float* ms_out) {
     if (!h->build_pending)
         return set_error(SF_E_STATE, "sf_update_solver needs a neighbour build (sf_build_neighbors) since the last step");
     if ((rc = views_in(h))) return rc;
+    h->pph_current = false;  // a caller may have written positions since that build
     SF_HIP(hipEventRecord(h->ev0, h->stream));
     if ((rc = update_solver(h, render_interval))) return rc;
     if ((rc = views_out(h))) return rc;

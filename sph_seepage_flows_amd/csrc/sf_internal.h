@@ -175,6 +175,12 @@ uint32_t inc_parts(uint32_t C);
 int wprefix_blocks(int n);
 
 // ---- solver launchers (sf_solver.hip) ----
+// Saved neighbours per listed particle, over its lanes.  h is twice the
+// spacing of grains or water at rest: 33 within it, 8.4 a lane of four; 20 rows
+// a lane leave five deviations of that.  A particle with more is walked again.
+constexpr int kSaved = 80;
+constexpr uint32_t kSavedOver = 255u;
+inline size_t saved_entries(size_t n) { return (n + 2 * 64) * (size_t)kSaved; }
 constexpr int kCountStride = 64;  // words between the two interface counters (a cache line each)
 struct Fields {
     const float4* pm;
@@ -253,16 +259,32 @@ struct Fields {
     // m p / max(eps, rho_sand rho~) (voidage/adhesion pass; sand momentum's
     // buoyancy pairs)
     float4* wbq;
-    // Neighbour records of the water momentum pass, by slot, written when
-    // rec is set (every water particle has the same mass mw): water
+    // The other phase's neighbours of every listed particle (phase indices, in
+    // the order its lanes met them), saved by the avg-flow pass for the passes
+    // after it: lane s of the nl_lanes of the particle at place q of its
+    // phase's list wrote lane G = q nl_lanes + s (sand: from the next wave
+    // after the water's on), entry r of lane G at
+    // nl[((G / 64) (kSaved / nl_lanes) + r) 64 + G % 64], nlc[G] entries
+    // (kSavedOver: more than its rows hold), and q at nlq[t].
+    uint32_t* nl;
+    uint8_t* nlc;
+    uint32_t* nlq;
+    int nl_lanes;
+    // fresh: pph[t] == pm[plist[t]] (the build is this call's, or no caller
+    // holds the position, mass or label buffer).  Then the neighbour records of
+    // the water momentum pass are written, by phase index: water
     // rec0 = (position, rho~), rec1 = (velocity, p / rho~^2); sand
-    // rec0 = (position, -mass), rec1 = avgDrag.  A neighbour then costs two
-    // 16-byte loads instead of the three of pm, wt and vr (or pm and xf).
-    // With rec set, wt is written only for the differentiable window (den4).
+    // rec1 = avgDrag (its position and -mass are pph's).  A neighbour then
+    // costs two 16-byte loads instead of the three of pm, wt and vr (or pm
+    // and xf), the water's mass among them when it is known to be one, mw
+    // (rec), a 4-byte load of its own otherwise.
+    // Otherwise rec0 holds every particle's position as it is now, the rest is
+    // read from the slots.  With fresh set, wt is written only for the differentiable window (den4).
     float4* rec0;
     float4* rec1;
     float mw;
     int rec;
+    int fresh;
 };
 // Launch shape of a neighbour pass: workgroup size and the per-lane LDS
 // candidate-list capacity (the latter only for the passes that use one).

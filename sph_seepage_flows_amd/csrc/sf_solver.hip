@@ -360,22 +360,23 @@ SF_DEV void write_empty_outputs(const Fields& f, int i, bool sand) {
     }
 }
 // Water particle i's (rho~, p / rho~^2) from (rho, p) and its voidage eps:
-// wt, or the neighbour records with pi = (position, mass) (Fields::rec0).
-SF_DEV void write_water_terms(const Fields& f, int i, const float4& pi, float2 rpi, float eps) {
+// wt, or the neighbour records (Fields::rec0) with pi = (position, mass), t
+// its phase index.
+SF_DEV void write_water_terms(const Fields& f, int i, uint32_t t, const float4& pi, float2 rpi, float eps) {
     const float rt = rpi.x / fmaxf(kEps, eps);
     const float pt = rpi.y / fmaxf(kEps, rt * rt);
-    if (!f.rec || f.den4) f.wt[i] = make_float2(rt, pt);
-    if (f.rec) {
+    if (!f.fresh || f.den4) f.wt[i] = make_float2(rt, pt);
+    f.rec0[t] = make_float4(pi.x, pi.y, pi.z, rt);
+    if (f.fresh) {
         const float4 v = ldo(f.vr, (uint32_t)i);
-        f.rec0[i] = make_float4(pi.x, pi.y, pi.z, rt);
-        f.rec1[i] = make_float4(v.x, v.y, v.z, pt);
+        f.rec1[t] = make_float4(v.x, v.y, v.z, pt);
     }
 }
-SF_DEV void write_no_interface(const Fields& f, int i, bool sand, float2 rpi, const float4& pi) {
+SF_DEV void write_no_interface(const Fields& f, int i, uint32_t t, bool sand, float2 rpi, const float4& pi) {
     if (sand) {
         f.es[i] = make_float2(0.f, 0.f);
     } else {
-        write_water_terms(f, i, pi, rpi, 1.f);
+        write_water_terms(f, i, t, pi, rpi, 1.f);
     }
     if (f.full_empty || f.den4) write_empty_outputs(f, i, sand);
     if (f.den4) {
@@ -474,7 +475,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
             // taped, else on request (launch_fill_empty)
             if (f.full_empty || f.den4) f.rp[i] = make_float2(k.rho_s, 0.f);
             const float4 p = ldo(f.pph, nw + t);
-            if (f.rec) f.rec0[i] = p;
+            if (!f.fresh) f.rec0[nw + t] = ldo(f.pm, (uint32_t)i);
             const uint32_t cb = scene_base<B>(k, f, i);
             int cx, cy, cz;
             cell_of(k, p.x, p.y, p.z, cx, cy, cz);
@@ -489,7 +490,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
             const float4 v = ldo(f.vr, (uint32_t)i);
             f.vq[nw + t] = make_float4(v.x, v.y, v.z, 0.f);
         }
-        if (valid && !listed) write_no_interface(f, i, true, make_float2(k.rho_s, 0.f), make_float4(0.f, 0.f, 0.f, 0.f));
+        if (valid && !listed) write_no_interface(f, i, nw + t, true, make_float2(k.rho_s, 0.f), make_float4(0.f, 0.f, 0.f, 0.f));
         return;
     }
     const uint32_t t = pb.blk * PB + threadIdx.x / kDenL;
@@ -580,7 +581,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
     const float2 rpi = make_float2(rho, eos(k, rho));
     f.rp[i] = rpi;
     if (!listed) {
-        write_no_interface(f, i, false, rpi, pi);
+        write_no_interface(f, i, t, false, rpi, pi);
     } else {
         f.vq[t] = ldo(f.vr, (uint32_t)i);
         f.wq[t] = make_float4(rpi.x, rpi.y, 0.f, 0.f);  // voidage: avg flow
@@ -614,7 +615,7 @@ __global__ __launch_bounds__(kBlock) void k_interface(SFConst k, Fields f, int n
     if (valid) {
         i = (int)ldo(f.plist, t);
         pi = ldo(f.pph, t);
-        if (f.rec && sand_i) f.rec0[i] = pi;
+        if (!f.fresh && sand_i) f.rec0[t] = ldo(f.pm, (uint32_t)i);
         const uint32_t cb = scene_base<B>(k, f, i);
         int cx, cy, cz;
         cell_of(k, pi.x, pi.y, pi.z, cx, cy, cz);
@@ -628,7 +629,7 @@ __global__ __launch_bounds__(kBlock) void k_interface(SFConst k, Fields f, int n
     list_interface<kBlock>(f, listed, sand_i, t, nw, (uint32_t)n);
     if (valid && !sand_i) f.wl[u] = listed ? 1 : 0;
     if (valid && sand_i) f.iface[u] = listed ? 1 : 0;
-    if (valid && !listed) write_no_interface(f, i, sand_i, ldo(f.rp, (uint32_t)i), pi);
+    if (valid && !listed) write_no_interface(f, i, t, sand_i, ldo(f.rp, (uint32_t)i), pi);
 }
 __global__ __launch_bounds__(kBlock) void k_fill_empty(SFConst k, Fields f, int n) {
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
@@ -653,6 +654,7 @@ template <int NB, int LP>
 struct PhaseSlot {
     int i;         // the particle's slot
     uint32_t t;    // its phase index (plist[t] = i)
+    uint32_t q;    // its place in its phase's list
     uint32_t sub;  // its lane among LP
     bool sand;
 };
@@ -663,10 +665,12 @@ SF_DEV bool phase_slot(const Fields& f, uint32_t nw, uint32_t cw, uint32_t cs, P
     constexpr uint32_t PB = NB / LP;  // particles per block
     ps.i = 0;
     ps.t = 0;
+    ps.q = 0;
     ps.sand = pb.phase == 1;
     const uint32_t q = pb.blk * PB + threadIdx.x / LP;
     ps.sub = threadIdx.x % LP;
     if (q >= (ps.sand ? cs : cw)) return false;
+    ps.q = q;
     ps.t = ldo(f.ilist, (ps.sand ? nw : 0u) + q);
     ps.i = (int)ldo(f.plist, ps.t);
     return true;
@@ -695,6 +699,54 @@ SF_DEV void for_listed(const Fields& f, Body&& body) {
         b += gridDim.x;
         pb = phase_block(na, nb, b);
     } while (pb.phase >= 0);  // past the share's end, so are all later ones
+}
+
+// ---------------------------------------------------------------------------
+// Saved neighbours (Fields::nl).  P2, P3 and P4's water walk need the same
+// pairs, a particle and the other phase's within h, of which a walk of the 27
+// cells keeps one candidate in six: the walk's filter was most of each pass.
+// P2 saves what it keeps (a coalesced 4-byte store per pair) and the others
+// read that.  500k + 500k interpenetrating: P3 203 -> 141 us, P4 150 -> 132, P5
+// (with its walk over the water alone) 221 -> 161, for 200 -> 235 in P2: step
+// 916 -> 851.  An entry costs its store and loads (4 bytes a row, rows of a
+// wave as long as its fullest lane); what is left is the pairs' gathers.
+// First saved lane of the particle at place q of its phase's list.
+SF_DEV uint32_t saved_lane(uint32_t lanes, bool sand, uint32_t nw, uint32_t q) {
+    return (sand ? (nw * lanes + 63u) & ~63u : 0u) + q * lanes;
+}
+// Entry 0 of saved lane G, of `rows` entries 64 apart.
+SF_DEV uint32_t* saved_row(const Fields& f, uint32_t G, uint32_t rows) {
+    return f.nl + ((size_t)(G >> 6) * rows * 64u + (G & 63u));
+}
+// apply over the saved neighbours of the particle whose lanes start at G0,
+// lane sub of S taking its share: whole lanes of the writer's where there are
+// as many or more, every (S / lanes)-th entry of one where there are fewer.
+// The indices go through the lane's LDS list, eight loads in flight.
+template <uint32_t S, int NB, int CAP, class Fetch, class Apply>
+SF_DEV void saved_pairs(const Fields& f, uint32_t lanes, uint32_t G0, uint32_t sub, NList<NB, CAP>& L, Fetch&& fetch,
+                        Apply&& apply) {
+    static_assert(CAP >= 8, "a round takes eight entries");
+    const uint32_t step = S > lanes ? S / lanes : 1u, rows = (uint32_t)kSaved / lanes;
+    for (uint32_t l = sub & (lanes - 1u); l < lanes; l += S) {
+        const uint32_t G = G0 + l, cnt = ldo(f.nlc, G);
+        const uint32_t* __restrict__ e = saved_row(f, G, rows);
+        for (uint32_t r = S > lanes ? sub / lanes : 0u; r < cnt;) {
+            L.cnt = 0;
+            do {
+                uint32_t v[8];
+#pragma unroll
+                for (uint32_t c = 0; c < 8u; ++c) v[c] = e[(r + c * step < cnt ? r + c * step : r) * 64u];
+#pragma unroll
+                for (uint32_t c = 0; c < 8u; ++c) {
+                    L.slot[(L.cnt + (int)c) * NB] = v[c];
+                }
+                const uint32_t left = (cnt - r + step - 1u) / step;
+                L.cnt += left < 8u ? (int)left : 8;
+                r += 8u * step;
+            } while (r < cnt && L.cnt + 8 <= CAP);
+            nl_flush2(L, fetch, apply);
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -736,7 +788,13 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
     // sand i: water neighbours (rho_j needed); water i: sand neighbours
     // neighbours within h are listed: their fields by phase index
     auto fetch = [&](uint32_t u) { return Nbr{ldo(f.pph, u), ldo(f.vq, u), sand_i ? ldo(f.wq, u).x : 0.f}; };
-    auto pair = [&](uint32_t, const Nbr& q) {
+    const uint32_t G = saved_lane(LP, sand_i, nw, ps.q) + sub;
+    constexpr uint32_t rows = (uint32_t)kSaved / LP;
+    uint32_t* __restrict__ saved = saved_row(f, G, rows);
+    uint32_t kept = 0;
+    auto pair = [&](uint32_t u, const Nbr& q) {
+        if (kept < rows) saved[kept * 64u] = u;
+        ++kept;
         const float4 pj = q.pj;
         const float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         const float r2 = dx * dx + dy * dy + dz * dz;
@@ -751,10 +809,18 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
         [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, sand_i, nw); }, in_range, fetch, pair);
     nl_flush2(L, fetch, pair);
     if (!active) return;
+    uint32_t most = kept;
+#pragma unroll
+    for (int o = 1; o < LP; o <<= 1) {
+        const uint32_t other = __shfl_xor(most, o);
+        most = most > other ? most : other;
+    }
+    f.nlc[G] = (uint8_t)(most > rows ? kSavedOver : kept);
     sandv = lane_sum<LP>(sandv);
     vsum = lane_sum<LP>(vsum);
     av = mk3(lane_sum<LP>(av.x), lane_sum<LP>(av.y), lane_sum<LP>(av.z));
     if (sub != 0) return;
+    f.nlq[ps.t] = ps.q;
     const v3 fl = vsum != 0.f ? av * (1.f / vsum) : mk3(0.f, 0.f, 0.f);
     f.flow[i] = f4(fl, 0.f);
     if (f.den4) reinterpret_cast<float*>(f.den4)[4 * i] = vsum;
@@ -765,7 +831,7 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
         reinterpret_cast<float*>(f.vq)[4 * ps.t + 3] = vsum;
     }
     if (!sand_i) {
-        write_water_terms(f, i, pi, ldo(f.rp, (uint32_t)i), eps_i);
+        write_water_terms(f, i, ps.t, pi, ldo(f.rp, (uint32_t)i), eps_i);
         reinterpret_cast<float*>(f.wq)[4 * ps.t + 2] = eps_i;
     }
 }
@@ -790,7 +856,8 @@ void launch_avg_flow(const SFConst& k, const Fields& f, int n, PassCfg c, hipStr
 
 // ---------------------------------------------------------------------------
 // P3: sand i -> voidage from water neighbours; water i -> adhesion force.
-// Same walk as P2.
+// Over the neighbours P2 saved, each lane its own; the walk of P2 where they
+// were too many.
 template <bool B, int NB, int CAP, int LP>
 SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float4* __restrict__ stage,
                              uint32_t nw, uint32_t cw, uint32_t cs, PhaseBlock pb) {
@@ -812,6 +879,9 @@ SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& 
         float4 pj;
         float2 x;  // sand i: (rho_j, voidage_j) of a water j; water i: saturation of a sand j in y
     };
+    const uint32_t G = saved_lane(LP, ps.sand, nw, ps.q);
+    const bool over = active && ldo(f.nlc, G + sub) == kSavedOver;  // of all the particle's lanes
+    const bool read = active && !over;
     // neighbours within h are listed: water (rho, voidage) or sand saturation
     // (in y) by phase index
     auto fetch = [&](uint32_t u) {
@@ -828,8 +898,9 @@ SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& 
             num += q.x.y * vw;
             den += vw;
         };
+        if (read) saved_pairs<LP>(f, LP, G, sub, L, fetch, pair);
         column_filter<LP, kStageList>(
-            k, f.pph, stage, active, cb, cx, cy, cz, L,
+            k, f.pph, stage, over, cb, cx, cy, cz, L,
             [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); }, in_range, fetch, pair);
         nl_flush2(L, fetch, pair);
         if (!active) return;
@@ -854,12 +925,13 @@ SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& 
         const float l = fsqrt(r2);
         const float A = adhesion_A(k, l);
         if (A != 0.f) {
-            const float G = bezier(k.gadh, q.x.y);
-            F += dp * (G * mi * mj * A * frcp(fmaxf(kEps, l)));
+            const float curve = bezier(k.gadh, q.x.y);
+            F += dp * (curve * mi * mj * A * frcp(fmaxf(kEps, l)));
         }
     };
+    if (read) saved_pairs<LP>(f, LP, G, sub, L, fetch, pair);
     column_filter<LP, kStageList>(
-        k, f.pph, stage, active, cb, cx, cy, cz, L,
+        k, f.pph, stage, over, cb, cx, cy, cz, L,
         [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, false, nw); }, in_range, fetch, pair);
     nl_flush2(L, fetch, pair);
     if (!active) return;
@@ -1014,8 +1086,14 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
     // a grain with no water in its 9 column ranges (the density pass flagged
     // the others) has nothing to walk
     const bool wet = active && ldo(f.iface, t);
+    bool over = false;
+    if (wet) {  // P2 saved its neighbours
+        const uint32_t G = saved_lane((uint32_t)f.nl_lanes, true, nw, ldo(f.nlq, self));
+        over = ldo(f.nlc, G) == kSavedOver;
+        if (!over) saved_pairs<kSmL>(f, (uint32_t)f.nl_lanes, G, sub, L, fetch_water, water);
+    }
     column_filter<kSmL, kStageList>(
-        k, f.pph, stage, wet, cb, cx, cy, cz, L,
+        k, f.pph, stage, over, cb, cx, cy, cz, L,
         [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); },
         [&](uint32_t, const float4& pj) {
             const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
@@ -1054,7 +1132,7 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
     }
     const float4 drag = vw != 0.f ? f4(df * (1.f / vw), 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
     f.xf[i] = drag;
-    if (f.rec) f.rec1[i] = drag;
+    if (f.fresh) f.rec1[self] = drag;
     if (f.den4) reinterpret_cast<float*>(f.den4)[4 * i + 2] = vw;
     const v3 a = mk3(k.gvx, k.gvy, k.gvz) + (fsum + df) * (2.f / mi);
     f.acc[i] = f4(a, 0.f);
@@ -1087,27 +1165,48 @@ void launch_sand_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, h
 // its own list (column_filter, which stages the candidates in LDS where the
 // wave's ranges overlap), and the partial sums are combined with shuffles.
 constexpr int kWmL = 4;
-// A neighbour's data in the water momentum pass: r0 = (position, w) with
-// w > 0 for water, w = -mass for sand.  WmRecords reads the two records
-// (Fields::rec0; every water particle has mass f.mw); WmSlots reads the
-// slot arrays pm (w = mass), wt and vr, and a grain's xf on its own.
+// A neighbour's data in the water momentum pass, by phase index u:
+// r0 = (position, w) with w > 0 for water, w = -mass for a grain (load_sand).
+// WmRecords reads the two records (Fields::rec0; every water particle has mass
+// f.mw), WmMasses the mass besides; both walk the water alone and take the
+// grains that P2 saved, so an interpenetrating cell's grains are not filtered
+// again (P5 221 -> 161 us at 500k + 500k interpenetrating, 4M dam 323 -> 300).
+// WmSlots is for positions a caller may have written since the build (two
+// calls, a handed-out buffer): everything from the slots as they are now, both
+// phases walked.  All three give a particle the same terms in the same order.
 struct WmRecords {
+    static constexpr bool fresh = true;
     float4 r0, r1;
-    SF_DEV static WmRecords load(const Fields& f, uint32_t j) { return {ldo(f.rec0, j), ldo(f.rec1, j)}; }
+    SF_DEV static WmRecords load(const Fields& f, uint32_t u) { return {ldo(f.rec0, u), ldo(f.rec1, u)}; }
+    SF_DEV static WmRecords load_sand(const Fields& f, uint32_t u) { return {ldo(f.pph, u), ldo(f.rec1, u)}; }
     SF_DEV float water_mass(const Fields& f) const { return f.mw; }
     SF_DEV float2 wt() const { return make_float2(r0.w, r1.w); }
     SF_DEV v3 vel() const { return xyz(r1); }
-    SF_DEV v3 drag(const Fields&, uint32_t) const { return xyz(r1); }
+    SF_DEV v3 drag() const { return xyz(r1); }
+};
+struct WmMasses : WmRecords {
+    float m;
+    SF_DEV static WmMasses load(const Fields& f, uint32_t u) {
+        return {WmRecords::load(f, u), ldo(reinterpret_cast<const float*>(f.pph), 4u * u + 3u)};
+    }
+    SF_DEV static WmMasses load_sand(const Fields& f, uint32_t u) { return {WmRecords::load_sand(f, u), 0.f}; }
+    SF_DEV float water_mass(const Fields&) const { return m; }
 };
 struct WmSlots {
+    static constexpr bool fresh = false;
     float4 r0;
     float2 w;
-    float4 v;
-    SF_DEV static WmSlots load(const Fields& f, uint32_t j) { return {ldo(f.pm, j), ldo(f.wt, j), ldo(f.vr, j)}; }
+    float4 v;  // a grain's: the drag
+    SF_DEV static WmSlots load(const Fields& f, uint32_t u) {
+        const uint32_t j = ldo(f.plist, u);
+        const float4 r0 = ldo(f.pm, j);
+        return {r0, ldo(f.wt, j), ldo(r0.w > 0.f ? f.vr : f.xf, j)};
+    }
+    SF_DEV static WmSlots load_sand(const Fields& f, uint32_t u) { return load(f, u); }
     SF_DEV float water_mass(const Fields&) const { return r0.w; }
     SF_DEV float2 wt() const { return w; }
     SF_DEV v3 vel() const { return xyz(v); }
-    SF_DEV v3 drag(const Fields& f, uint32_t j) const { return xyz(ldo(f.xf, j)); }
+    SF_DEV v3 drag() const { return xyz(v); }
 };
 template <bool B, class Nbr, int NB, int CAP>
 __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int n) {
@@ -1124,7 +1223,7 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     const uint32_t sub = threadIdx.x % kWmL;  // this lane's share of the particle's candidates
     // lanes past the last particle take part in the staged walk without a range
     const int i = t < nw ? (int)ldo(f.plist, t) : 0;
-    const Nbr self = Nbr::load(f, (uint32_t)i);
+    const Nbr self = Nbr::load(f, t < nw ? t : 0u);
     const float4 pi = self.r0;  // position; w > 0 for water
     const bool active = t < nw && pi.w >= 0.f;
     const uint32_t cb = scene_base<B>(k, f, i);
@@ -1139,31 +1238,41 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     int cx, cy, cz;
     cell_of(k, pi.x, pi.y, pi.z, cx, cy, cz);
     v3 a = mk3(0.f, 0.f, 0.f);
-    auto fetch = [&](uint32_t j) { return Nbr::load(f, j); };
-    auto pair = [&](uint32_t j, const Nbr& q) {
-        const float4 pj = q.r0;
-        const v3 d = mk3(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z);
-        const float r2 = dot(d, d);
-        const float rs = frsq(r2);
+    auto fetch = [&](uint32_t u) { return Nbr::load(f, u); };
+    auto fetch_sand = [&](uint32_t u) { return Nbr::load_sand(f, u); };
+    // the products in one order of roundings wherever the body is inlined
+    auto dot_yxz = [](v3 u, v3 w) { return fmaf(u.z, w.z, fmaf(u.x, w.x, u.y * w.y)); };
+    auto spiky = [&](float r2, float rs) {  // spiky gradient / r
         const float r = r2 * rs;
         const float hr = k.h - r;
-        const float gs = r >= kEps ? k.g_coef * hr * hr * rs : 0.f;  // spiky gradient / r
-        if (pj.w > 0.f) {  // water j: ComputeSFWaterPressureTerm + ArtificialViscosity
-            const float2 wtj = q.wt();
-            const float mj = q.water_mass(f);
-            float s = -mj * (wti.y + wtj.y);
-            const v3 dv = vi - q.vel();
-            const float dd = dot(dv, d);
-            const float pij = -k.nu * frcp(rt_i + wtj.x) * (dd * frcp(r2 + kEps));
-            s += dd < 0.f ? -mj * pij : 0.f;
-            a += d * (s * gs);
-        } else {  // sand j: ComputeSFWaterSeepageTerm
-            const float mj = -pj.w;
-            const float rho_j = k.rho_s;  // the density pass gives every grain rho_sand
-            const float w = k.w_coef * sq3(k.h2 - r2);
-            a += d * (-mj * p_i * frcp(fmaxf(kEps, rt_i * rho_j)) * gs);
-            a += q.drag(f, j) * (-w * inv_rt_i);
-        }
+        return r >= kEps ? k.g_coef * hr * hr * rs : 0.f;
+    };
+    // water j: ComputeSFWaterPressureTerm + ArtificialViscosity
+    auto water = [&](uint32_t, const Nbr& q) {
+        const float4 pj = q.r0;
+        const v3 d = mk3(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z);
+        const float r2 = dot_yxz(d, d);
+        const float gs = spiky(r2, frsq(r2));
+        const float2 wtj = q.wt();
+        const float mj = q.water_mass(f);
+        float s = -mj * (wti.y + wtj.y);
+        const v3 dv = vi - q.vel();
+        const float dd = dot_yxz(dv, d);
+        const float pij = -k.nu * frcp(rt_i + wtj.x) * (dd * frcp(r2 + kEps));
+        s += dd < 0.f ? -mj * pij : 0.f;
+        a += d * (s * gs);
+    };
+    // sand j: ComputeSFWaterSeepageTerm
+    auto sand = [&](uint32_t, const Nbr& q) {
+        const float4 pj = q.r0;
+        const v3 d = mk3(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z);
+        const float r2 = dot_yxz(d, d);
+        const float gs = spiky(r2, frsq(r2));
+        const float mj = -pj.w;
+        const float rho_j = k.rho_s;  // the density pass gives every grain rho_sand
+        const float w = k.w_coef * sq3(k.h2 - r2);
+        a += d * (-mj * p_i * frcp(fmaxf(kEps, rt_i * rho_j)) * gs);
+        a += q.drag() * (-w * inv_rt_i);
     };
     // the particle's own slot passes too: d = 0 makes its term exactly zero
     // (the spiky factor is 0 below r = eps), and acc adds g afterwards
@@ -1172,11 +1281,35 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
         const float r2 = dx * dx + dy * dy + dz * dz;
         return r2 < k.h2;
     };
-    column_filter<kWmL, kStageWm>(
-        k, f.pm, stage, active, cb, cx, cy, cz, L,
-        [&](uint32_t b, uint32_t c0, uint32_t c1) { return make_uint2(ldo(f.ct + b, c0).x, ldo(f.ct + b, c1).x); },
-        in_range, fetch, pair);
-    nl_flush2(L, fetch, pair);
+    if constexpr (Nbr::fresh) {
+        column_filter<kWmL, kStageWm>(
+            k, f.rec0, stage, active, cb, cx, cy, cz, L,
+            [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); }, in_range,
+            fetch, water);
+        nl_flush2(L, fetch, water);
+        bool over = false;
+        if (active && ldo(f.wl, t)) {  // listed
+            const uint32_t G = saved_lane((uint32_t)f.nl_lanes, false, nw, ldo(f.nlq, t));
+            over = ldo(f.nlc, G) == kSavedOver;
+            if (!over) saved_pairs<kWmL>(f, (uint32_t)f.nl_lanes, G, sub, L, fetch_sand, sand);
+        }
+        column_filter<kWmL, kStageWm>(
+            k, f.pph, stage, over, cb, cx, cy, cz, L,
+            [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, false, nw); }, in_range,
+            fetch_sand, sand);
+        nl_flush2(L, fetch_sand, sand);
+    } else {
+        auto pair = [&](uint32_t u, const Nbr& q) {
+            if (q.r0.w > 0.f) water(u, q);
+            else sand(u, q);
+        };
+        for (int phase = 0; phase < 2; ++phase)
+            column_filter<kWmL, kStageWm>(
+                k, f.rec0, stage, active, cb, cx, cy, cz, L,
+                [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, phase == 0, nw); },
+                in_range, fetch, pair);
+        nl_flush2(L, fetch, pair);
+    }
     if (!active) return;
     const uint32_t cell = cell_key(k, cx, cy, cz);
     if (const uint32_t near = ldo(f.bnear, cell)) {  // boundary particles within the 27 cells
@@ -1219,6 +1352,7 @@ void launch_water_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, 
         constexpr bool b = decltype(B)::value;
         constexpr int nb = decltype(NB)::value, cap = decltype(CAP)::value;
         if (f.rec) k_water_momentum<b, WmRecords, nb, cap><<<phase_grid(n * kWmL, NB), nb, 0, s>>>(k, f, n);
+        else if (f.fresh) k_water_momentum<b, WmMasses, nb, cap><<<phase_grid(n * kWmL, NB), nb, 0, s>>>(k, f, n);
         else k_water_momentum<b, WmSlots, nb, cap><<<phase_grid(n * kWmL, NB), nb, 0, s>>>(k, f, n);
     });
 }

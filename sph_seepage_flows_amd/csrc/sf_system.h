@@ -57,6 +57,8 @@ struct sf_system {
     DevBuf<uint32_t> brow;            // their columns' ranges (Fields::brange)
     DevBuf<uint2> brange;
     DevBuf<float4> vq, wq, xq, wbq;   // listed particles' fields by phase index (Fields::wq)
+    DevBuf<uint32_t> nl, nlq;         // saved neighbours (Fields::nl)
+    DevBuf<uint8_t> nlc;
     DevBuf<float4> rec0, rec1;        // water momentum neighbour records (Fields::rec0)
     DevBuf<uint8_t> wflag;
     DevBuf<uint2> ct[2];  // cell table: the incremental sort reads the previous one
@@ -72,13 +74,15 @@ struct sf_system {
     // anything else that changes positions
     bool keys_fresh = false;
     bool pm_shared = false;  // the position buffer was handed out (sf_device_buffer)
+    // the last build is the running call's own: no caller wrote since
+    bool pph_current = false;
     // water masses of the particles: 0 no water, 1 all equal to water_mass,
     // 2 not all equal (set by the upload and the emitter)
     int water_mass_state = 0;
     float water_mass = 0.f;
     size_t n_water = 0;  // water particles, as uploaded and emitted
-    // the neighbour records are used while the water masses are equal and
-    // known on the host (a caller holding the position / mass buffer may
+    // the neighbour records carry no mass while the water masses are equal
+    // and known on the host (a caller holding the position / mass buffer may
     // change them)
     bool records_on() const { return water_mass_state < 2 && !pm_shared; }
     const uint32_t* perm = nullptr;
@@ -161,10 +165,15 @@ struct sf_system {
         f.wq = wq.p;
         f.xq = xq.p;
         f.wbq = wbq.p;
+        f.nl = nl.p;
+        f.nlc = nlc.p;
+        f.nlq = nlq.p;
+        f.nl_lanes = cfg[SF_PASS_AVG_FLOW - SF_PASS_DENSITY].lanes;
         f.rec0 = rec0.p;
         f.rec1 = rec1.p;
         f.mw = water_mass;
         f.rec = records_on() ? 1 : 0;
+        f.fresh = !pm_shared || pph_current ? 1 : 0;
         return f;
     }
     uint32_t local_cells() const { return K.C; }
