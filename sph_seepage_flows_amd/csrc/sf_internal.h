@@ -245,10 +245,13 @@ struct Fields {
     // column ranges) by phase index t, written only for those:
     //   vq[t] = the velocity (density pass); for every grain, not only the
     //   listed ones, with its saturation in vq[t].w (0 from the density
-    //   pass, the avg-flow pass's value for the listed);
-    //   water: wq[t] = (rho, p) (density pass), voidage in wq[t].z (avg
-    //   flow), xq[t] = avgAdhesion (voidage/adhesion pass);
-    //   sand: saturation in wq[t].w (avg flow).
+    //   pass, the avg-flow pass's value for the listed); water's volume
+    //   m / rho in vq[t].w;
+    //   wq[t] = (position, water: volume times voidage, sand: m times the
+    //   adhesion curve at its saturation) (avg flow): all that the
+    //   voidage/adhesion pass needs of a neighbour;
+    //   water: xq[t] = avgAdhesion (voidage/adhesion pass), sum of the grains'
+    //   V W in wbq[t].w from the avg-flow to the voidage/adhesion pass.
     // Every other-phase neighbour within h of a particle is listed, so the
     // interface and sand momentum passes read these without the slot
     // indirection plist[t].

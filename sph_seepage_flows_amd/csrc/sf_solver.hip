@@ -583,8 +583,8 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
     if (!listed) {
         write_no_interface(f, i, t, false, rpi, pi);
     } else {
-        f.vq[t] = ldo(f.vr, (uint32_t)i);
-        f.wq[t] = make_float4(rpi.x, rpi.y, 0.f, 0.f);  // voidage: avg flow
+        const float4 v = ldo(f.vr, (uint32_t)i);
+        f.vq[t] = make_float4(v.x, v.y, v.z, pi.w * frcp(rho));
     }
 }
 void launch_density(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
@@ -701,12 +701,20 @@ SF_DEV void for_listed(const Fields& f, Body&& body) {
     } while (pb.phase >= 0);  // past the share's end, so are all later ones
 }
 
+// Squared length and kernel weight of a pair within h, their roundings the
+// same wherever they are inlined: near the edge h^2 - r^2 keeps few digits, and
+// P3's quotients (its own sums over P2's) are only as good as the two agree.
+SF_DEV float pair_r2(v3 d) { return fmaf(d.z, d.z, fmaf(d.x, d.x, d.y * d.y)); }
+SF_DEV float edge_weight(const SFConst& k, const float4& pi, const float4& pj) {
+    return k.w_coef * sq3(k.h2 - pair_r2(mk3(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z)));
+}
+
 // ---------------------------------------------------------------------------
 // Saved neighbours (Fields::nl).  P2, P3 and P4's water walk need the same
 // pairs, a particle and the other phase's within h, of which a walk of the 27
 // cells keeps one candidate in six: the walk's filter was most of each pass.
 // P2 saves what it keeps (a coalesced 4-byte store per pair) and the others
-// read that.  500k + 500k interpenetrating: P3 203 -> 141 us, P4 150 -> 132, P5
+// read that.  500k + 500k interpenetrating: P3 203 -> 143 us, P4 150 -> 132, P5
 // (with its walk over the water alone) 221 -> 161, for 200 -> 235 in P2: step
 // 916 -> 851.  An entry costs its store and loads (4 bytes a row, rows of a
 // wave as long as its fullest lane); what is left is the pairs' gathers.
@@ -773,7 +781,7 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
     const uint32_t cb = scene_base<B>(k, f, i);
     int cx, cy, cz;
     cell_of(k, pi.x, pi.y, pi.z, cx, cy, cz);
-    float sandv = 0.f, vsum = 0.f;
+    float vsum = 0.f;
     v3 av = mk3(0.f, 0.f, 0.f);
     const float inv_rho_s = k.rho_s != 0.f ? 1.f / k.rho_s : 0.f;
     auto in_range = [&](uint32_t, const float4& pj) {
@@ -783,11 +791,10 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
     };
     struct Nbr {
         float4 pj, vj;
-        float rho;
     };
-    // sand i: water neighbours (rho_j needed); water i: sand neighbours
-    // neighbours within h are listed: their fields by phase index
-    auto fetch = [&](uint32_t u) { return Nbr{ldo(f.pph, u), ldo(f.vq, u), sand_i ? ldo(f.wq, u).x : 0.f}; };
+    // neighbours within h are listed: their fields by phase index (a water
+    // neighbour's volume beside its velocity: two 16-byte loads a pair)
+    auto fetch = [&](uint32_t u) { return Nbr{ldo(f.pph, u), ldo(f.vq, u)}; };
     const uint32_t G = saved_lane(LP, sand_i, nw, ps.q) + sub;
     constexpr uint32_t rows = (uint32_t)kSaved / LP;
     uint32_t* __restrict__ saved = saved_row(f, G, rows);
@@ -796,11 +803,8 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
         if (kept < rows) saved[kept * 64u] = u;
         ++kept;
         const float4 pj = q.pj;
-        const float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-        const float r2 = dx * dx + dy * dy + dz * dz;
-        const float w = k.w_coef * sq3(k.h2 - r2);
-        const float vw = (sand_i ? pj.w * frcp(q.rho) : -pj.w * inv_rho_s) * w;
-        if (!sand_i) sandv += vw;
+        const float w = edge_weight(k, pi, pj);
+        const float vw = (sand_i ? q.vj.w : -pj.w * inv_rho_s) * w;
         av += xyz(q.vj) * vw;
         vsum += vw;
     };
@@ -816,7 +820,6 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
         most = most > other ? most : other;
     }
     f.nlc[G] = (uint8_t)(most > rows ? kSavedOver : kept);
-    sandv = lane_sum<LP>(sandv);
     vsum = lane_sum<LP>(vsum);
     av = mk3(lane_sum<LP>(av.x), lane_sum<LP>(av.y), lane_sum<LP>(av.z));
     if (sub != 0) return;
@@ -824,16 +827,19 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
     const v3 fl = vsum != 0.f ? av * (1.f / vsum) : mk3(0.f, 0.f, 0.f);
     f.flow[i] = f4(fl, 0.f);
     if (f.den4) reinterpret_cast<float*>(f.den4)[4 * i] = vsum;
-    const float eps_i = 1.f - sandv;
+    const float eps_i = sand_i ? 1.f : 1.f - vsum;
     f.es[i] = make_float2(eps_i, sand_i ? vsum : 0.f);
-    if (sand_i) {  // saturation, for P3 and (with the velocity) P4
-        reinterpret_cast<float*>(f.wq)[4 * ps.t + 3] = vsum;
-        reinterpret_cast<float*>(f.vq)[4 * ps.t + 3] = vsum;
+    float x;  // what P3's neighbours need besides the position
+    if (sand_i) {
+        x = -pi.w * bezier(k.gadh, vsum);
+        reinterpret_cast<float*>(f.vq)[4 * ps.t + 3] = vsum;  // saturation, for P4
+    } else {
+        const float2 rpi = ldo(f.rp, (uint32_t)i);
+        write_water_terms(f, i, ps.t, pi, rpi, eps_i);
+        x = pi.w * frcp(rpi.x) * eps_i;
+        reinterpret_cast<float*>(f.wbq)[4 * ps.t + 3] = vsum;
     }
-    if (!sand_i) {
-        write_water_terms(f, i, ps.t, pi, ldo(f.rp, (uint32_t)i), eps_i);
-        reinterpret_cast<float*>(f.wq)[4 * ps.t + 2] = eps_i;
-    }
+    f.wq[ps.t] = make_float4(pi.x, pi.y, pi.z, x);
 }
 template <bool B, int NB, int CAP, int LP>
 __global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
@@ -858,6 +864,11 @@ void launch_avg_flow(const SFConst& k, const Fields& f, int n, PassCfg c, hipStr
 // P3: sand i -> voidage from water neighbours; water i -> adhesion force.
 // Over the neighbours P2 saved, each lane its own; the walk of P2 where they
 // were too many.
+// A pair is bound by its gathers, so P2 leaves one 16-byte record per neighbour
+// (Fields::wq), with the adhesion curve taken once a grain and not once a pair,
+// and the sums of weights that P2 has already made (P3 143 -> 122 us, and P2,
+// which reads the volume instead of dividing, 235 -> 207 at 500k + 500k
+// interpenetrating).
 template <bool B, int NB, int CAP, int LP>
 SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float4* __restrict__ stage,
                              uint32_t nw, uint32_t cw, uint32_t cs, PhaseBlock pb) {
@@ -875,28 +886,15 @@ SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& 
         const float r2 = dx * dx + dy * dy + dz * dz;
         return r2 < k.h2;
     };
-    struct Nbr {
-        float4 pj;
-        float2 x;  // sand i: (rho_j, voidage_j) of a water j; water i: saturation of a sand j in y
-    };
     const uint32_t G = saved_lane(LP, ps.sand, nw, ps.q);
     const bool over = active && ldo(f.nlc, G + sub) == kSavedOver;  // of all the particle's lanes
     const bool read = active && !over;
-    // neighbours within h are listed: water (rho, voidage) or sand saturation
-    // (in y) by phase index
-    auto fetch = [&](uint32_t u) {
-        const float4 w = ldo(f.wq, u);
-        return Nbr{ldo(f.pph, u), ps.sand ? make_float2(w.x, w.z) : make_float2(0.f, w.w)};
-    };
+    // neighbours within h are listed: P2 left all that a pair needs of them
+    auto fetch = [&](uint32_t u) { return ldo(f.wq, u); };
     if (ps.sand) {
-        float num = 0.f, den = 0.f;
-        auto pair = [&](uint32_t, const Nbr& q) {
-            const float4 pj = q.pj;
-            const float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-            const float r2 = dx * dx + dy * dy + dz * dz;
-            const float vw = (pj.w * frcp(q.x.x)) * (k.w_coef * sq3(k.h2 - r2));
-            num += q.x.y * vw;
-            den += vw;
+        float num = 0.f;
+        auto pair = [&](uint32_t, const float4& pj) {
+            num += pj.w * edge_weight(k, pi, pj);
         };
         if (read) saved_pairs<LP>(f, LP, G, sub, L, fetch, pair);
         column_filter<LP, kStageList>(
@@ -905,29 +903,20 @@ SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& 
         nl_flush2(L, fetch, pair);
         if (!active) return;
         num = lane_sum<LP>(num);
-        den = lane_sum<LP>(den);
         if (sub != 0) return;
+        const float den = ldo(f.vq, ps.t).w;  // the sum of the weights: the saturation
         f.es[i].x = den != 0.f ? num / den : 0.f;
         f.adh[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (f.den4) reinterpret_cast<float*>(f.den4)[4 * i + 1] = den;
         return;
     }
     const float mi = pi.w;
-    const float inv_rho_s = k.rho_s != 0.f ? 1.f / k.rho_s : 0.f;
-    float vs = 0.f;
     v3 F = mk3(0.f, 0.f, 0.f);
-    auto pair = [&](uint32_t, const Nbr& q) {
-        const float4 pj = q.pj;
+    auto pair = [&](uint32_t, const float4& pj) {
         const v3 dp = mk3(pi.x - pj.x, pi.y - pj.y, pi.z - pj.z);
-        const float r2 = dot(dp, dp);
-        const float mj = -pj.w;
-        vs += (mj * inv_rho_s) * (k.w_coef * sq3(k.h2 - r2));
-        const float l = fsqrt(r2);
+        const float l = fsqrt(pair_r2(dp));
         const float A = adhesion_A(k, l);
-        if (A != 0.f) {
-            const float curve = bezier(k.gadh, q.x.y);
-            F += dp * (curve * mi * mj * A * frcp(fmaxf(kEps, l)));
-        }
+        if (A != 0.f) F += dp * (pj.w * mi * A * frcp(fmaxf(kEps, l)));
     };
     if (read) saved_pairs<LP>(f, LP, G, sub, L, fetch, pair);
     column_filter<LP, kStageList>(
@@ -935,21 +924,22 @@ SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& 
         [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, false, nw); }, in_range, fetch, pair);
     nl_flush2(L, fetch, pair);
     if (!active) return;
-    vs = lane_sum<LP>(vs);
     F = mk3(lane_sum<LP>(F.x), lane_sum<LP>(F.y), lane_sum<LP>(F.z));
     if (sub != 0) return;
     f.adh[i] = f4(F, 0.f);
+    const float vs = reinterpret_cast<const float*>(f.wbq)[4 * ps.t + 3];  // P2's sum of the grains' V W
     const float4 avg = vs != 0.f ? f4(F * (1.f / vs), 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
     f.xf[i] = avg;
     // what a grain's buoyancy sums need of this particle (sand momentum
     // pass): m / rho~ and m p / max(eps, rho_sand rho~), both zero unless the
     // voidage lies in (0, 1]
-    const float4 w = ldo(f.wq, ps.t);  // (rho, p, voidage)
+    const float2 rpi = ldo(f.rp, (uint32_t)i);
+    const float eps = f.es[i].x;
     float a = 0.f, g = 0.f;
-    if (w.z > 0.f && w.z <= 1.f) {
-        const float dj = w.x * frcp(fmaxf(kEps, w.z));
+    if (eps > 0.f && eps <= 1.f) {
+        const float dj = rpi.x * frcp(fmaxf(kEps, eps));
         a = mi * frcp(dj);
-        g = mi * w.y * frcp(fmaxf(kEps, k.rho_s * dj));
+        g = mi * rpi.y * frcp(fmaxf(kEps, k.rho_s * dj));
     }
     f.xq[ps.t] = make_float4(avg.x, avg.y, avg.z, g);
     f.wbq[ps.t] = make_float4(pi.x, pi.y, pi.z, a);
