@@ -49,6 +49,7 @@ def pass_bytes(n_w: int, n_s: int, nb: int, cells: int, multi: bool, listed=(0, 
     n = n_w + n_s
     aux = 24 if multi else 0
     lw, ls = listed
+    saved = 4 * 33 + 8  # a listed particle's saved neighbours at rest spacing, counts and place
     return {
         # stepping loop: the advect computes the next keys and counts the
         # moves (below).  The placement reads both keys and the stay prefix,
@@ -61,31 +62,32 @@ def pass_bytes(n_w: int, n_s: int, nb: int, cells: int, multi: bool, listed=(0, 
         "gather": 0,  # within the placement, as the cell table
         "cell_start": 0,
         # plist, own position (water: pm, sand: pph), water candidates' pph, rho/p (water);
-        # sand: position record, velocity read and written in phase order;
-        # unlisted water: velocity read, both records written; unlisted
-        # sand: es + flag; listed water: velocity read and written, (rho, p);
-        # listed: list entry
-        "density": n_w * (4 + 16 + 16 + 8 + 1) + n_s * (4 + 16 + 1 + 16 + 32) + (n_w - lw) * (16 + 32)
-                   + (n_s - ls) * 8 + lw * (32 + 16) + (lw + ls) * 4 + 8 * (cells + 1) + 4 * (cells + 1) + cells
+        # sand: velocity read and written in phase order; unlisted water:
+        # velocity read, both records written; unlisted sand: es + flag;
+        # listed water: velocity read and written; listed: list entry
+        "density": n_w * (4 + 16 + 16 + 8 + 1) + n_s * (4 + 16 + 1 + 32) + (n_w - lw) * (16 + 32)
+                   + (n_s - ls) * 8 + lw * 32 + (lw + ls) * 4 + 8 * (cells + 1) + 4 * (cells + 1) + cells
                    + nb * 16,
         # listed only: list + slot, own position, phase-index position / velocity
-        # (/ rho for water), flow, es, water velocity, records and voidage, sand
-        # saturation (twice: for P3, and beside the phase-order velocity for P4)
-        "avg_flow": lw * (4 + 4 + 16 + 16 + 16 + 16 + 8 + 16 + 8 + 16 + 32 + 4) + ls * (4 + 4 + 16 + 16 + 16 + 16 + 8 + 4 + 4)
-                    + 8 * (cells + 1),
-        # listed only: list + slot, own position, phase-index position / (rho, voidage, sat);
-        # sand voidage + adhesion 0, water adhesion + avgAdhesion (slot and phase index)
-        # and the buoyancy record (own (rho, p, voidage) read, position + factor written)
-        "voidage_adhesion": lw * (4 + 4 + 16 + 16 + 16 + 48 + 16 + 16) + ls * (4 + 4 + 16 + 16 + 16 + 4 + 16)
-                            + 8 * (cells + 1),
+        # (and volume), flow, es, the next pass's record, the saved neighbours,
+        # water: rho/p, velocity, records, weight sum; sand: saturation
+        "avg_flow": lw * (4 + 4 + 16 + 16 + 16 + 16 + 8 + 16 + saved + 8 + 16 + 32 + 4)
+                    + ls * (4 + 4 + 16 + 16 + 16 + 16 + 8 + 16 + saved + 4) + 8 * (cells + 1),
+        # listed only: list + slot, own position, the neighbours' records, the
+        # saved neighbours; sand voidage + adhesion 0, water rho/p, es, weight
+        # sum, adhesion + avgAdhesion (slot and phase index), buoyancy record
+        "voidage_adhesion": lw * (4 + 4 + 16 + 16 + saved + 8 + 8 + 4 + 48 + 16)
+                            + ls * (4 + 4 + 16 + 16 + saved + 4 + 4 + 16),
         # per grain: plist, position, velocity, es, colour read and written,
         # interface flag, avgDrag (and its record) and acc written; the sand
-        # candidates' phase-order positions and velocities touched once; the cell table
-        "sand_momentum": n_s * (4 + 16 + 16 + 8 + 16 + 16 + 1 + 16 + 16 + 16) + n_s * 32 + 8 * (cells + 1),
-        # both records of every particle once (own and candidates); per water
-        # particle plist, rho/p and acc written; the cell and boundary
-        # tables, boundary particles
-        "water_momentum": n * 32 + n_w * (4 + 8 + 16) + 8 * (cells + 1)
+        # candidates' phase-order positions and velocities touched once; the listed
+        # ones' saved water and its two records; the cell table
+        "sand_momentum": n_s * (4 + 16 + 16 + 8 + 16 + 16 + 1 + 16 + 16 + 16) + n_s * 32 + ls * saved + lw * 32 + 8 * (cells + 1),
+        # both records of every water particle once (own and candidates), of the
+        # listed grains their position and drag, the listed water's saved
+        # grains; per water particle plist, rho/p and acc written; the cell and
+        # boundary tables, boundary particles
+        "water_momentum": n_w * 32 + ls * 32 + lw * saved + n_w * (4 + 8 + 16) + 8 * (cells + 1)
                           + 4 * (cells + 1) + cells + nb * 16,
         # position, velocity, acc read; position, velocity written; sand colour;
         # the next key written, the current sorted key read (change flag), the
