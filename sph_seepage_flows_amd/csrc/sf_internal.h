@@ -250,8 +250,10 @@ struct Fields {
     //   wq[t] = (position, water: volume times voidage, sand: m times the
     //   adhesion curve at its saturation) (avg flow): all that the
     //   voidage/adhesion pass needs of a neighbour;
-    //   water: xq[t] = avgAdhesion (voidage/adhesion pass), sum of the grains'
-    //   V W in wbq[t].w from the avg-flow to the voidage/adhesion pass.
+    //   water: vws[t] = sum of the grains' V W (avg flow), xq[t] = avgAdhesion
+    //   (voidage/adhesion pass).
+    // No pass overwrites what it reads here, so each may run again on the same
+    // inputs (sf_autotune does).
     // Every other-phase neighbour within h of a particle is listed, so the
     // interface and sand momentum passes read these without the slot
     // indirection plist[t].
@@ -262,6 +264,7 @@ struct Fields {
     // m p / max(eps, rho_sand rho~) (voidage/adhesion pass; sand momentum's
     // buoyancy pairs)
     float4* wbq;
+    float* vws;
     // The other phase's neighbours of every listed particle (phase indices, in
     // the order its lanes met them), saved by the avg-flow pass for the passes
     // after it: lane s of the nl_lanes of the particle at place q of its

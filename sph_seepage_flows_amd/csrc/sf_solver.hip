@@ -837,7 +837,7 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
         const float2 rpi = ldo(f.rp, (uint32_t)i);
         write_water_terms(f, i, ps.t, pi, rpi, eps_i);
         x = pi.w * frcp(rpi.x) * eps_i;
-        reinterpret_cast<float*>(f.wbq)[4 * ps.t + 3] = vsum;
+        f.vws[ps.t] = vsum;
     }
     f.wq[ps.t] = make_float4(pi.x, pi.y, pi.z, x);
 }
@@ -927,7 +927,7 @@ SF_DEV void voidage_adhesion(const SFConst& k, const Fields& f, NList<NB, CAP>& 
     F = mk3(lane_sum<LP>(F.x), lane_sum<LP>(F.y), lane_sum<LP>(F.z));
     if (sub != 0) return;
     f.adh[i] = f4(F, 0.f);
-    const float vs = reinterpret_cast<const float*>(f.wbq)[4 * ps.t + 3];  // P2's sum of the grains' V W
+    const float vs = ldo((const float*)f.vws, ps.t);  // P2's sum of the grains' V W
     const float4 avg = vs != 0.f ? f4(F * (1.f / vs), 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
     f.xf[i] = avg;
     // what a grain's buoyancy sums need of this particle (sand momentum

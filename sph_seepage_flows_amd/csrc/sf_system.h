@@ -57,6 +57,7 @@ struct sf_system {
     DevBuf<uint32_t> brow;            // their columns' ranges (Fields::brange)
     DevBuf<uint2> brange;
     DevBuf<float4> vq, wq, xq, wbq;   // listed particles' fields by phase index (Fields::wq)
+    DevBuf<float> vws;
     DevBuf<uint32_t> nl, nlq;         // saved neighbours (Fields::nl)
     DevBuf<uint8_t> nlc;
     DevBuf<float4> rec0, rec1;        // water momentum neighbour records (Fields::rec0)
@@ -165,6 +166,7 @@ struct sf_system {
         f.wq = wq.p;
         f.xq = xq.p;
         f.wbq = wbq.p;
+        f.vws = vws.p;
         f.nl = nl.p;
         f.nlc = nlc.p;
         f.nlq = nlq.p;
