@@ -249,7 +249,9 @@ struct Fields {
     //   m / rho in vq[t].w;
     //   wq[t] = (position, water: volume times voidage, sand: m times the
     //   adhesion curve at its saturation) (avg flow): all that the
-    //   voidage/adhesion pass needs of a neighbour;
+    //   voidage/adhesion pass needs of a neighbour.  Position and mass here and
+    //   in vq[t].w are pph[t]'s, those the avg-flow pass tested and saved the
+    //   neighbours by, also where the slot holds others by now (not fresh);
     //   water: vws[t] = sum of the grains' V W (avg flow), xq[t] = avgAdhesion
     //   (voidage/adhesion pass).
     // No pass overwrites what it reads here, so each may run again on the same

@@ -47,6 +47,10 @@ SF_DEV float4 own_pos(const Fields& f, uint32_t t, int i) {
     return f.nw >= 0 ? ldo(f.pph, t) : ldo(f.pm, (uint32_t)i);
 }
 
+// The same as its neighbours see it: pph[t], which is also pi while nothing was
+// written since the build.
+SF_DEV float4 built_pos(const Fields& f, uint32_t t, const float4& pi) { return f.fresh ? pi : ldo(f.pph, t); }
+
 // First cell key of slot i's scene (batched handles), 0 otherwise.
 template <bool B>
 SF_DEV uint32_t scene_base(const SFConst& k, const Fields& f, int i) {
@@ -584,7 +588,7 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
         write_no_interface(f, i, t, false, rpi, pi);
     } else {
         const float4 v = ldo(f.vr, (uint32_t)i);
-        f.vq[t] = make_float4(v.x, v.y, v.z, pi.w * frcp(rho));
+        f.vq[t] = make_float4(v.x, v.y, v.z, built_pos(f, t, pi).w * frcp(rho));
     }
 }
 void launch_density(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
@@ -829,17 +833,18 @@ SF_DEV void avg_flow(const SFConst& k, const Fields& f, NList<NB, CAP>& L, float
     if (f.den4) reinterpret_cast<float*>(f.den4)[4 * i] = vsum;
     const float eps_i = sand_i ? 1.f : 1.f - vsum;
     f.es[i] = make_float2(eps_i, sand_i ? vsum : 0.f);
+    const float4 pj = built_pos(f, ps.t, pi);
     float x;  // what P3's neighbours need besides the position
     if (sand_i) {
-        x = -pi.w * bezier(k.gadh, vsum);
+        x = -pj.w * bezier(k.gadh, vsum);
         reinterpret_cast<float*>(f.vq)[4 * ps.t + 3] = vsum;  // saturation, for P4
     } else {
         const float2 rpi = ldo(f.rp, (uint32_t)i);
         write_water_terms(f, i, ps.t, pi, rpi, eps_i);
-        x = pi.w * frcp(rpi.x) * eps_i;
+        x = pj.w * frcp(rpi.x) * eps_i;
         f.vws[ps.t] = vsum;
     }
-    f.wq[ps.t] = make_float4(pi.x, pi.y, pi.z, x);
+    f.wq[ps.t] = make_float4(pj.x, pj.y, pj.z, x);
 }
 template <bool B, int NB, int CAP, int LP>
 __global__ __launch_bounds__(NB) void k_avg_flow(SFConst k, Fields f, int n) {
