@@ -136,7 +136,7 @@ int ensure_sort_capacity(sf_system* h, size_t m) {
     if ((rc = h->wpre.alloc(c + 1)) || (rc = h->wpart.alloc((size_t)wprefix_blocks((int)c + 1) + 1)) ||
         (rc = h->plist.alloc(c)) || (rc = h->wflag.alloc(c)) || (rc = h->pph.alloc(c)) || (rc = h->ilist.alloc(c)) ||
         (rc = h->icount.alloc(2 * kCountStride)) || (rc = h->iface.alloc(c)) || (rc = h->wl.alloc(c)) || (rc = h->vq.alloc(c)) || (rc = h->wq.alloc(c)) ||
-        (rc = h->xq.alloc(c)) || (rc = h->wbq.alloc(c)) || (rc = h->vws.alloc(c)) || (rc = h->rec0.alloc(c)) || (rc = h->rec1.alloc(c)) ||
+        (rc = h->xq.alloc(c)) || (rc = h->wbq.alloc(c)) || (rc = h->vws.alloc(c)) || (rc = h->rec0.alloc(c)) || (rc = h->rec1.alloc(c)) || (rc = h->recm.alloc(c)) ||
         (rc = h->nl.alloc(saved_entries(c))) || (rc = h->nlc.alloc(4 * c + 2 * 64)) || (rc = h->nlq.alloc(c)))
         return rc;
     // the interface counters start at zero (each step's water momentum pass
@@ -573,7 +573,7 @@ int sf_create(const sf_params* p, const sf_boundary_params* b, const sf_solver_o
             (rc = h->cda[q].alloc(c)) || (rc = h->amc[q].alloc(c)))
             return bail(rc);
     }
-    if ((rc = h->rp.alloc(c)) || (rc = h->es.alloc(c)) || (rc = h->wt.alloc(c)) || (rc = h->flow.alloc(c)) || (rc = h->adh.alloc(c)) ||
+    if ((rc = h->rp.alloc(c)) || (rc = h->es.alloc(c)) || (rc = h->flow.alloc(c)) || (rc = h->adh.alloc(c)) ||
         (rc = h->xf.alloc(c)) || (rc = h->acc.alloc(c)))
         return bail(rc);
     if ((rc = h->cell.alloc((size_t)h->C + 1)) || (rc = h->bcell.alloc((size_t)h->local_cells() + 1)) ||
@@ -594,7 +594,7 @@ int sf_create(const sf_params* p, const sf_boundary_params* b, const sf_solver_o
     if ((rc = zero(h, h->rp)) || (rc = zero(h, h->es)) || (rc = zero(h, h->flow)) || (rc = zero(h, h->adh)) ||
         (rc = zero(h, h->xf)) || (rc = zero(h, h->acc)) || (rc = zero(h, h->cell)) || (rc = zero(h, h->bcell)) ||
         (rc = zero(h, h->bnear)) ||
-        (rc = zero(h, h->ct[0])) || (rc = zero(h, h->ct[1])) || (rc = zero(h, h->wt)) || (rc = zero(h, h->wpre)) || (rc = zero(h, h->plist)) ||
+        (rc = zero(h, h->ct[0])) || (rc = zero(h, h->ct[1])) || (rc = zero(h, h->wpre)) || (rc = zero(h, h->plist)) ||
         (rc = zero(h, h->keys)) || (rc = zero(h, h->bpv)))
         return bail(rc);
     {

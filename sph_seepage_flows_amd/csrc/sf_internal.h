@@ -199,7 +199,8 @@ struct Fields {
     const uint2* brange;
     float2* rp;
     float2* es;
-    float2* wt;  // water: (rho / max(eps, voidage), p / max(eps, (rho / max(eps, voidage))^2))
+    // water, taped only (den4): (rho / max(eps, voidage), p / max(eps, (rho / max(eps, voidage))^2))
+    float2* wt;
     float4* flow;
     float4* adh;
     float4* xf;
@@ -237,7 +238,7 @@ struct Fields {
     // avgAdhesion are the empty sums' constants; the density pass writes them
     // only when full_empty is set (or den4, the differentiable window),
     // otherwise they are filled in on request (launch_fill_empty).  The
-    // fields a later pass reads (sand voidage / saturation, water wt) are
+    // fields a later pass reads (sand voidage / saturation, water records) are
     // always written.
     uint8_t* wl;
     int full_empty;
@@ -278,18 +279,18 @@ struct Fields {
     uint8_t* nlc;
     uint32_t* nlq;
     int nl_lanes;
-    // fresh: pph[t] == pm[plist[t]] (the build is this call's, or no caller
-    // holds the position, mass or label buffer).  Then the neighbour records of
-    // the water momentum pass are written, by phase index: water
+    // Neighbour records of the water momentum pass, by phase index: water
     // rec0 = (position, rho~), rec1 = (velocity, p / rho~^2); sand
-    // rec1 = avgDrag (its position and -mass are pph's).  A neighbour then
-    // costs two 16-byte loads instead of the three of pm, wt and vr (or pm
-    // and xf), the water's mass among them when it is known to be one, mw
-    // (rec), a 4-byte load of its own otherwise.
-    // Otherwise rec0 holds every particle's position as it is now, the rest is
-    // read from the slots.  With fresh set, wt is written only for the differentiable window (den4).
+    // rec1 = avgDrag.  A neighbour costs two 16-byte loads instead of three by
+    // slot, the water's mass among them when it is known to be one, mw (rec),
+    // a 4-byte load of its own otherwise.
+    // fresh: pph[t] == pm[plist[t]] (the build is this call's, or no caller
+    // holds the position, mass or label buffer).  Then pph has the masses, and
+    // the sand's positions.  Otherwise rec0 holds the sand's position and
+    // -mass as they are now, and recm the water's mass.
     float4* rec0;
     float4* rec1;
+    float* recm;
     float mw;
     int rec;
     int fresh;

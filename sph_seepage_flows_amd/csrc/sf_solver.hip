@@ -353,7 +353,7 @@ void dispatch(const Fields& f, PassCfg c, L&& l) {
 
 // What P2 then P3 leave for particle i with empty sums; rpi = (rho, p).
 // Later passes read the sand's voidage / saturation (drag, capillary bridges)
-// and the water's wt or records; the rest is output only and written here when the
+// and the water's records; the rest is output only and written here when the
 // fields are read directly (full_empty) or taped (den4), else on request.
 SF_DEV void write_empty_outputs(const Fields& f, int i, bool sand) {
     f.flow[i] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -364,17 +364,16 @@ SF_DEV void write_empty_outputs(const Fields& f, int i, bool sand) {
     }
 }
 // Water particle i's (rho~, p / rho~^2) from (rho, p) and its voidage eps:
-// wt, or the neighbour records (Fields::rec0) with pi = (position, mass), t
-// its phase index.
+// the neighbour records (Fields::rec0) with pi = (position, mass), t its phase
+// index, and wt where taped.
 SF_DEV void write_water_terms(const Fields& f, int i, uint32_t t, const float4& pi, float2 rpi, float eps) {
     const float rt = rpi.x / fmaxf(kEps, eps);
     const float pt = rpi.y / fmaxf(kEps, rt * rt);
-    if (!f.fresh || f.den4) f.wt[i] = make_float2(rt, pt);
+    if (f.den4) f.wt[i] = make_float2(rt, pt);
+    if (!f.fresh) f.recm[t] = pi.w;
     f.rec0[t] = make_float4(pi.x, pi.y, pi.z, rt);
-    if (f.fresh) {
-        const float4 v = ldo(f.vr, (uint32_t)i);
-        f.rec1[t] = make_float4(v.x, v.y, v.z, pt);
-    }
+    const float4 v = ldo(f.vr, (uint32_t)i);
+    f.rec1[t] = make_float4(v.x, v.y, v.z, pt);
 }
 SF_DEV void write_no_interface(const Fields& f, int i, uint32_t t, bool sand, float2 rpi, const float4& pi) {
     if (sand) {
@@ -767,8 +766,8 @@ SF_DEV void saved_pairs(const Fields& f, uint32_t lanes, uint32_t G0, uint32_t s
 // (Sand voidage from this pass is overwritten by P3 before anything reads it,
 // so a sand particle only needs its water neighbours, a water particle only
 // its sand neighbours.)
-// Water particles also store wt = (rho / max(eps, voidage), p / max(eps, that^2)),
-// the per-particle factors the water momentum pass needs from every neighbour.
+// Water particles also store (rho / max(eps, voidage), p / max(eps, that^2)), the
+// per-particle factors the water momentum pass needs from every neighbour.
 // Candidates are filtered four at a time into the lane's list; the flush
 // fetches each kept neighbour's fields (by phase index u: every neighbour
 // within h is listed, see Fields::vq) ahead of its use.
@@ -1127,7 +1126,7 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
     }
     const float4 drag = vw != 0.f ? f4(df * (1.f / vw), 0.f) : make_float4(0.f, 0.f, 0.f, 0.f);
     f.xf[i] = drag;
-    if (f.fresh) f.rec1[self] = drag;
+    f.rec1[self] = drag;
     if (f.den4) reinterpret_cast<float*>(f.den4)[4 * i + 2] = vw;
     const v3 a = mk3(k.gvx, k.gvy, k.gvz) + (fsum + df) * (2.f / mi);
     f.acc[i] = f4(a, 0.f);
@@ -1166,9 +1165,14 @@ constexpr int kWmL = 4;
 // f.mw), WmMasses the mass besides; both walk the water alone and take the
 // grains that P2 saved, so an interpenetrating cell's grains are not filtered
 // again (P5 221 -> 161 us at 500k + 500k interpenetrating, 4M dam 323 -> 300).
-// WmSlots is for positions a caller may have written since the build (two
-// calls, a handed-out buffer): everything from the slots as they are now, both
-// phases walked.  All three give a particle the same terms in the same order.
+// WmMoved is for positions a caller may have written since the build (two
+// calls, a handed-out buffer): the records hold everything as it is now, and
+// both phases are walked, what P2 saved having been kept by the build's
+// positions; the grains only where P1 counted any in the 27 cells (1M apart
+// 128 us, 170 with every particle walking both phases and one body for either
+// kind, 133 with one walk over both by slot).  All
+// three give a particle the same terms, water before grains; the same bits
+// where as many lanes saved the grains as share the particle (four).
 struct WmRecords {
     static constexpr bool fresh = true;
     float4 r0, r1;
@@ -1178,6 +1182,7 @@ struct WmRecords {
     SF_DEV float2 wt() const { return make_float2(r0.w, r1.w); }
     SF_DEV v3 vel() const { return xyz(r1); }
     SF_DEV v3 drag() const { return xyz(r1); }
+    SF_DEV bool is_water() const { return r0.w >= 0.f; }
 };
 struct WmMasses : WmRecords {
     float m;
@@ -1187,21 +1192,13 @@ struct WmMasses : WmRecords {
     SF_DEV static WmMasses load_sand(const Fields& f, uint32_t u) { return {WmRecords::load_sand(f, u), 0.f}; }
     SF_DEV float water_mass(const Fields&) const { return m; }
 };
-struct WmSlots {
+struct WmMoved : WmRecords {
     static constexpr bool fresh = false;
-    float4 r0;
-    float2 w;
-    float4 v;  // a grain's: the drag
-    SF_DEV static WmSlots load(const Fields& f, uint32_t u) {
-        const uint32_t j = ldo(f.plist, u);
-        const float4 r0 = ldo(f.pm, j);
-        return {r0, ldo(f.wt, j), ldo(r0.w > 0.f ? f.vr : f.xf, j)};
-    }
-    SF_DEV static WmSlots load_sand(const Fields& f, uint32_t u) { return load(f, u); }
-    SF_DEV float water_mass(const Fields&) const { return r0.w; }
-    SF_DEV float2 wt() const { return w; }
-    SF_DEV v3 vel() const { return xyz(v); }
-    SF_DEV v3 drag() const { return xyz(v); }
+    float m;
+    SF_DEV static WmMoved load(const Fields& f, uint32_t u) { return {WmRecords::load(f, u), ldo((const float*)f.recm, u)}; }
+    SF_DEV static WmMoved load_sand(const Fields& f, uint32_t u) { return {WmRecords::load(f, u), 0.f}; }
+    SF_DEV float water_mass(const Fields&) const { return m; }
+    SF_DEV bool is_water() const { return m >= 0.f; }
 };
 template <bool B, class Nbr, int NB, int CAP>
 __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int n) {
@@ -1219,8 +1216,8 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     // lanes past the last particle take part in the staged walk without a range
     const int i = t < nw ? (int)ldo(f.plist, t) : 0;
     const Nbr self = Nbr::load(f, t < nw ? t : 0u);
-    const float4 pi = self.r0;  // position; w > 0 for water
-    const bool active = t < nw && pi.w >= 0.f;
+    const float4 pi = self.r0;
+    const bool active = t < nw && self.is_water();
     const uint32_t cb = scene_base<B>(k, f, i);
     const float mi = self.water_mass(f);
     const v3 vi = self.vel();
@@ -1276,34 +1273,47 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
         const float r2 = dx * dx + dy * dy + dz * dz;
         return r2 < k.h2;
     };
+    auto water_range = [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); };
+    auto sand_range = [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, false, nw); };
+    const bool listed = active && ldo(f.wl, t);  // grains in its 27 cells
     if constexpr (Nbr::fresh) {
-        column_filter<kWmL, kStageWm>(
-            k, f.rec0, stage, active, cb, cx, cy, cz, L,
-            [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); }, in_range,
-            fetch, water);
+        column_filter<kWmL, kStageWm>(k, f.rec0, stage, active, cb, cx, cy, cz, L, water_range, in_range, fetch, water);
         nl_flush2(L, fetch, water);
         bool over = false;
-        if (active && ldo(f.wl, t)) {  // listed
+        if (listed) {
             const uint32_t G = saved_lane((uint32_t)f.nl_lanes, false, nw, ldo(f.nlq, t));
             over = ldo(f.nlc, G) == kSavedOver;
             if (!over) saved_pairs<kWmL>(f, (uint32_t)f.nl_lanes, G, sub, L, fetch_sand, sand);
         }
-        column_filter<kWmL, kStageWm>(
-            k, f.pph, stage, over, cb, cx, cy, cz, L,
-            [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, false, nw); }, in_range,
-            fetch_sand, sand);
+        column_filter<kWmL, kStageWm>(k, f.pph, stage, over, cb, cx, cy, cz, L, sand_range, in_range, fetch_sand, sand);
         nl_flush2(L, fetch_sand, sand);
     } else {
-        auto pair = [&](uint32_t u, const Nbr& q) {
-            if (q.r0.w > 0.f) water(u, q);
-            else sand(u, q);
+        // the caller may have changed labels too: a neighbour counts as what it is now
+        auto was_water = [&](uint32_t u, Nbr q) {
+            if (q.is_water()) {
+                water(u, q);
+            } else {
+                q.r0.w = q.m;
+                q.r1 = ldo((const float4*)f.xf, ldo(f.plist, u));
+                sand(u, q);
+            }
         };
-        for (int phase = 0; phase < 2; ++phase)
-            column_filter<kWmL, kStageWm>(
-                k, f.rec0, stage, active, cb, cx, cy, cz, L,
-                [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, phase == 0, nw); },
-                in_range, fetch, pair);
-        nl_flush2(L, fetch, pair);
+        auto was_sand = [&](uint32_t u, Nbr q) {
+            if (q.r0.w <= 0.f) {
+                sand(u, q);
+            } else {  // no pass gave it a density
+                q.m = q.r0.w;
+                q.r0.w = 0.f;
+                q.r1 = ldo(f.vr, ldo(f.plist, u));
+                q.r1.w = 0.f;
+                water(u, q);
+            }
+        };
+        column_filter<kWmL, kStageWm>(k, f.rec0, stage, active, cb, cx, cy, cz, L, water_range, in_range, fetch, was_water);
+        nl_flush2(L, fetch, was_water);
+        column_filter<kWmL, kStageWm>(k, f.rec0, stage, listed, cb, cx, cy, cz, L, sand_range, in_range, fetch_sand,
+                                      was_sand);
+        nl_flush2(L, fetch_sand, was_sand);
     }
     if (!active) return;
     const uint32_t cell = cell_key(k, cx, cy, cz);
@@ -1348,7 +1358,7 @@ void launch_water_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, 
         constexpr int nb = decltype(NB)::value, cap = decltype(CAP)::value;
         if (f.rec) k_water_momentum<b, WmRecords, nb, cap><<<phase_grid(n * kWmL, NB), nb, 0, s>>>(k, f, n);
         else if (f.fresh) k_water_momentum<b, WmMasses, nb, cap><<<phase_grid(n * kWmL, NB), nb, 0, s>>>(k, f, n);
-        else k_water_momentum<b, WmSlots, nb, cap><<<phase_grid(n * kWmL, NB), nb, 0, s>>>(k, f, n);
+        else k_water_momentum<b, WmMoved, nb, cap><<<phase_grid(n * kWmL, NB), nb, 0, s>>>(k, f, n);
     });
 }
 

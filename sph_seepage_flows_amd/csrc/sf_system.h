@@ -61,6 +61,7 @@ struct sf_system {
     DevBuf<uint32_t> nl, nlq;         // saved neighbours (Fields::nl)
     DevBuf<uint8_t> nlc;
     DevBuf<float4> rec0, rec1;        // water momentum neighbour records (Fields::rec0)
+    DevBuf<float> recm;
     DevBuf<uint8_t> wflag;
     DevBuf<uint2> ct[2];  // cell table: the incremental sort reads the previous one
     int cur_ct = 0;       // ct and head (the next advect's chains hang from head[cur_ct])
@@ -88,7 +89,7 @@ struct sf_system {
     bool records_on() const { return water_mass_state < 2 && !pm_shared; }
     const uint32_t* perm = nullptr;
     // transient fields
-    DevBuf<float2> rp, es, wt;
+    DevBuf<float2> rp, es;
     DevBuf<float4> flow, adh, xf, acc;
     // boundary
     DevBuf<float4> bpv;
@@ -145,7 +146,7 @@ struct sf_system {
         f.brange = brange.p;
         f.rp = rp.p;
         f.es = es.p;
-        f.wt = wt.p;
+        f.wt = nullptr;
         f.flow = flow.p;
         f.adh = adh.p;
         f.xf = xf.p;
@@ -173,6 +174,7 @@ struct sf_system {
         f.nl_lanes = cfg[SF_PASS_AVG_FLOW - SF_PASS_DENSITY].lanes;
         f.rec0 = rec0.p;
         f.rec1 = rec1.p;
+        f.recm = recm.p;
         f.mw = water_mass;
         f.rec = records_on() ? 1 : 0;
         f.fresh = !pm_shared || pph_current ? 1 : 0;

@@ -157,3 +157,45 @@ def test_interface_sums_on_written_positions(hand_out, masses):
     assert inside.sum() > 100
     avg = F / np.where(vs != 0, vs, 1.0)[:, None]
     assert norm_err(g.get("avg_adhesion_force")[w], avg, inside) < 1e-3
+
+
+@pytest.mark.parametrize("hand_out,masses", CASES)
+def test_water_momentum_on_written_positions(hand_out, masses):
+    sc, g, ref, vel = _write_between(hand_out, masses)
+    rho, pres = g.get("density").astype(np.float64), g.get("pressure").astype(np.float64)
+    w = np.nonzero(ref.water)[0]
+    _, s, *_, w_ok, s_ok = ref.interface(rho)
+    drag = g.get("avg_drag_force").astype(np.float64)
+    bad = s[~s_ok]  # grains without a defined drag, and the water they reach
+    drag[bad] = 0.0
+    w_ok &= ~ref.pairs(w, bad, ref.Q)[2].any(1)
+    assert w_ok.sum() > 1000
+    acc = ref.water_acc(rho, pres, g.get("voidage").astype(np.float64)[w], vel, drag,
+                        np.where(w_ok[:, None], g.get("adhesion_force")[w].astype(np.float64), 0.0))
+    assert norm_err(g.get("acc")[w], acc, w_ok) < 1e-4
+
+
+def test_labels_written_between():
+    """A water particle the caller turned into a grain after the build counts as
+    one in the others' seepage term (with no drag of its own where it had no
+    grain near), and is no longer moved as water."""
+    sc = scenes.mixed(n_sand=1, collider=False)  # the grain touches no water's 27 cells
+    sc.pos[sc.label == 1] = np.float32(0.45)
+    sc.bpos = sc.blabel = None
+    g = SFSystem.from_scene(sc)
+    g.BuildGNSearcher()
+    P, m0, label = g.get("pos"), g.get("mass"), g.get("label")
+    water = label == 0
+    flip = np.nonzero(water)[0][::7]
+    lab = label.copy()
+    lab[flip] = 1
+    h2d(g.view("label"), lab)
+    vel = g.get("vel").astype(np.float64)
+    g.UpdateSolver(1e-5)
+    now = lab == 0
+    ref = _Reference(sc, now, P, m0, P, m0)
+    rho, pres = g.get("density").astype(np.float64), g.get("pressure").astype(np.float64)
+    w = np.nonzero(now)[0]
+    acc = ref.water_acc(rho, pres, np.ones(len(w)), vel, np.zeros_like(vel), np.zeros((len(w), 3)))
+    assert norm_err(g.get("acc")[w], acc) < 1e-4
+    assert np.abs(g.get("acc")[flip]).max() == 0.0
