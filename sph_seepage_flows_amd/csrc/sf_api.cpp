@@ -124,30 +124,46 @@ int zero(sf_system* h, DevBuf<T>& b) {
     return SF_OK;
 }
 
+// Work arrays of a radix sort of up to m keys, particles or boundary
+// particles: all in place or none replaced.
 int ensure_sort_capacity(sf_system* h, size_t m) {
-    if (m <= h->sort_cap && h->kA.p) return SF_OK;
-    size_t c = std::max<size_t>(m, 1);
+    if (m <= h->sort_cap) return SF_OK;
+    DevBuf<uint32_t> keys, kA, kB, vA, vB, hist;
     int rc;
-    if ((rc = h->keys.alloc(c)) || (rc = h->kA.alloc(c)) || (rc = h->kB.alloc(c)) || (rc = h->vA.alloc(c)) ||
-        (rc = h->vB.alloc(c)))
+    if ((rc = keys.alloc(m)) || (rc = kA.alloc(m)) || (rc = kB.alloc(m)) || (rc = vA.alloc(m)) || (rc = vB.alloc(m)) ||
+        (rc = hist.alloc(256 * ((m + kRsTile - 1) / kRsTile))))
         return rc;
-    size_t nblocks = (c + kRsTile - 1) / kRsTile;
-    if ((rc = h->hist.alloc(256 * nblocks))) return rc;
+    h->keys = std::move(keys);
+    h->kA = std::move(kA);
+    h->kB = std::move(kB);
+    h->vA = std::move(vA);
+    h->vB = std::move(vB);
+    h->hist = std::move(hist);
+    h->sort_cap = m;
+    h->built = false;  // the last sort's keys and permutation may have been in these
+    h->build_pending = false;
+    h->drop_graph();
+    return SF_OK;
+}
+
+// Arrays sized by the c particles the handle can hold.
+int alloc_particle_arrays(sf_system* h, size_t c) {
+    int rc;
     if ((rc = h->wpre.alloc(c + 1)) || (rc = h->wpart.alloc((size_t)wprefix_blocks((int)c + 1) + 1)) ||
         (rc = h->plist.alloc(c)) || (rc = h->wflag.alloc(c)) || (rc = h->pph.alloc(c)) || (rc = h->ilist.alloc(c)) ||
-        (rc = h->icount.alloc(2 * kCountStride)) || (rc = h->iface.alloc(c)) || (rc = h->wl.alloc(c)) || (rc = h->vq.alloc(c)) || (rc = h->wq.alloc(c)) ||
-        (rc = h->xq.alloc(c)) || (rc = h->wbq.alloc(c)) || (rc = h->vws.alloc(c)) || (rc = h->rec0.alloc(c)) || (rc = h->rec1.alloc(c)) || (rc = h->recm.alloc(c)) ||
+        (rc = h->icount.alloc(2 * kCountStride)) || (rc = h->iface.alloc(c)) || (rc = h->wl.alloc(c)) ||
+        (rc = h->vq.alloc(c)) || (rc = h->wq.alloc(c)) || (rc = h->xq.alloc(c)) || (rc = h->wbq.alloc(c)) ||
+        (rc = h->vws.alloc(c)) || (rc = h->rec0.alloc(c)) || (rc = h->rec1.alloc(c)) || (rc = h->recm.alloc(c)) ||
         (rc = h->nl.alloc(saved_entries(c))) || (rc = h->nlc.alloc(4 * c + 2 * 64)) || (rc = h->nlq.alloc(c)))
         return rc;
     // the interface counters start at zero (each step's water momentum pass
     // clears them for the next)
-    SF_HIP(hipMemsetAsync(h->icount.p, 0, h->icount.n * sizeof(uint32_t), h->stream));
+    if ((rc = zero(h, h->icount))) return rc;
     if ((rc = h->skeys[0].alloc(c)) || (rc = h->skeys[1].alloc(c)) || (rc = h->sperm.alloc(c)) ||
         (rc = h->next.alloc(c)) || (rc = h->local.alloc(c + 1)) || (rc = h->totals.alloc((c + kBlock - 1) / kBlock)) ||
         (rc = h->stay_base.alloc((c + kBlock - 1) / kBlock + 1)))
         return rc;
-    h->sort_cap = c;
-    return ensure_cell_capacity(h);
+    return SF_OK;
 }
 
 // arrays of the incremental sort sized by the cell count (C + 1) and the
@@ -583,7 +599,8 @@ int sf_create(const sf_params* p, const sf_boundary_params* b, const sf_solver_o
     if ((rc = h->cfl_part.alloc(cfl_partials(0))) || (rc = h->cfl_out.alloc(1)) ||
         (rc = h->frame_dev.alloc(1)))
         return bail(rc);
-    if ((rc = ensure_sort_capacity(h, c))) return bail(rc);
+    if ((rc = ensure_sort_capacity(h, c)) || (rc = alloc_particle_arrays(h, c)) || (rc = ensure_cell_capacity(h)))
+        return bail(rc);
     if ((rc = h->bpv.alloc(1))) return bail(rc);
     // zero everything like CudaArray::Clear (cuda_array.cuh:51-54)
     for (int q = 0; q < 2; ++q) {

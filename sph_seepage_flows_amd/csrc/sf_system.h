@@ -206,6 +206,7 @@ struct sf_system {
 
 namespace sf {
 int ensure_sort_capacity(sf_system* h, size_t m);
+int alloc_particle_arrays(sf_system* h, size_t c);
 int ensure_cell_capacity(sf_system* h);
 int build_neighbors(sf_system* h, hipEvent_t* ev = nullptr);
 int solve(sf_system* h, hipEvent_t* ev = nullptr);
