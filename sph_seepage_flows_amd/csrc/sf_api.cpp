@@ -593,7 +593,7 @@ int sf_create(const sf_params* p, const sf_boundary_params* b, const sf_solver_o
         (rc = h->xf.alloc(c)) || (rc = h->acc.alloc(c)))
         return bail(rc);
     if ((rc = h->cell.alloc((size_t)h->C + 1)) || (rc = h->bcell.alloc((size_t)h->local_cells() + 1)) ||
-        (rc = h->bnear.alloc((size_t)h->local_cells())) || (rc = h->ct[0].alloc((size_t)h->C + 1)) ||
+        (rc = h->bnear.alloc(near_bytes(h->local_cells()))) || (rc = h->ct[0].alloc((size_t)h->C + 1)) ||
         (rc = h->ct[1].alloc((size_t)h->C + 1)))
         return bail(rc);
     if ((rc = h->cfl_part.alloc(cfl_partials(0))) || (rc = h->cfl_out.alloc(1)) ||
@@ -747,38 +747,52 @@ int sf_upload_boundary(sf_handle h, size_t nb, const float* pos3, const uint64_t
         l1 += l == 1;
         bp[i] = make_float4(pos3[3 * i], pos3[3 * i + 1], pos3[3 * i + 2], l == 1 ? -1.f : 1.f);
     }
-    if ((rc = ensure_sort_capacity(h, std::max(h->cap, nb)))) return rc;
-    if ((rc = h->bpv.alloc(std::max<size_t>(nb, 1)))) return rc;
-    DevBuf<float4> tmp;
-    if ((rc = tmp.alloc(std::max<size_t>(nb, 1)))) return rc;
-    if (nb) SF_HIP(hipMemcpyAsync(tmp.p, bp.data(), nb * sizeof(float4), hipMemcpyHostToDevice, h->stream));
+    // Everything is made beside what the handle has and swapped in at the end:
+    // an upload that fails leaves the handle its old boundary.
+    const size_t C = h->local_cells(), m = std::max<size_t>(nb, 1);
+    const SFConst K = make_const(h->P, h->B, h->O, l1);
+    DevBuf<float4> bpv, given_own;
+    DevBuf<uint8_t> bnear;
+    DevBuf<uint32_t> bcell_own;
+    DevBuf<uint2> brange;
+    if ((rc = ensure_sort_capacity(h, nb)) || (rc = bpv.alloc(m)) || (rc = bnear.alloc(near_bytes(C) + 4 * C))) return rc;
+    // the particles as given and their cellStart: in the records, which every
+    // solve writes anew, where they fit
+    if (m > h->rec0.n && (rc = given_own.alloc(m))) return rc;
+    if (C + 1 > 4 * h->rec1.n && (rc = bcell_own.alloc(C + 1))) return rc;
+    float4* given = given_own.p ? given_own.p : h->rec0.p;
+    uint32_t* bcell = bcell_own.p ? bcell_own.p : reinterpret_cast<uint32_t*>(h->rec1.p);
+    uint32_t* brow = reinterpret_cast<uint32_t*>(bnear.p + near_bytes(C));
+    h->built = false;  // the particle searcher buffers are reused
+    h->build_pending = false;
+    h->drop_graph();
+    if (nb) SF_HIP(hipMemcpyAsync(given, bp.data(), nb * sizeof(float4), hipMemcpyHostToDevice, h->stream));
     // CudaGNBoundarySearcher::SortData (cuda_neighbor_searcher.cu:125-139): stable sort by cell
-    launch_hash_boundary(h->K, tmp.p, h->keys.p, (int)nb, h->stream);
+    launch_hash_boundary(K, given, h->keys.p, (int)nb, h->stream);
     SortBuffers sb{h->kA.p, h->vA.p, h->kB.p, h->vB.p, h->hist.p};
     const uint32_t *sk = nullptr, *bperm = nullptr;
     if ((rc = radix_sort(h->keys.p, (int)nb, h->plan, sb, &sk, &bperm, h->stream))) return rc;
-    launch_cell_start(sk, (int)nb, h->local_cells(), nullptr, h->bcell.p, nullptr, PhasePos{}, IncClear{}, h->stream);
-    launch_boundary_gather(bperm, tmp.p, h->bpv.p, (int)nb, h->stream);
-    launch_boundary_volume(h->K, h->bpv.p, h->bcell.p, (int)nb, h->stream);
+    launch_cell_start(sk, (int)nb, (uint32_t)C, nullptr, bcell, nullptr, PhasePos{}, IncClear{}, h->stream);
+    launch_boundary_gather(bperm, given, bpv.p, (int)nb, h->stream);
+    launch_boundary_volume(K, bpv.p, bcell, (int)nb, h->stream);
+    uint32_t total = 0;  // column ranges near the boundary, counted in the sort's histogram
+    SF_HIP(hipMemsetAsync(bnear.p, 0, near_bytes(C), h->stream));
+    SF_HIP(hipMemsetAsync(h->hist.p, 0, sizeof(uint32_t), h->stream));
+    launch_boundary_near(K, bpv.p, (int)nb, bcell, bnear.p, brow, h->hist.p, h->stream);
+    SF_HIP(hipMemcpyAsync(&total, h->hist.p, sizeof(total), hipMemcpyDeviceToHost, h->stream));
+    SF_HIP(hipStreamSynchronize(h->stream));
+    if (total > h->brange.n && (rc = brange.alloc(total))) return rc;
+    // nothing can fail for want of memory from here on
+    if (brange.p) h->brange = std::move(brange);
+    launch_boundary_rows(K, bcell, bnear.p, brow, h->brange.p, h->stream);
+    SF_HIP(hipMemcpyAsync(h->bcell.p, bcell, (C + 1) * sizeof(uint32_t), hipMemcpyDeviceToDevice, h->stream));
+    SF_HIP(hipGetLastError());
+    SF_HIP(hipStreamSynchronize(h->stream));
+    h->bpv = std::move(bpv);
+    h->bnear = std::move(bnear);
     h->blabel1 = l1;
-    h->K = make_const(h->P, h->B, h->O, h->blabel1);
-    {  // the cells near it and their columns' ranges
-        DevBuf<unsigned long long> sums;
-        unsigned long long total = 0;
-        if ((rc = sums.alloc(2)) || (rc = zero(h, sums))) return rc;
-        launch_boundary_near(h->K, h->bpv.p, h->bcell.p, h->bnear.p, sums.p, h->stream);
-        SF_HIP(hipMemcpyAsync(&total, sums.p, sizeof(total), hipMemcpyDeviceToHost, h->stream));
-        SF_HIP(hipStreamSynchronize(h->stream));
-        if (total > 0xffffffffull) return set_error(SF_E_CAPACITY, "too many cells near the boundary");
-        if ((rc = h->brange.alloc((size_t)total)) || (rc = h->brow.alloc(h->local_cells()))) return rc;
-        launch_boundary_rows(h->K, h->bcell.p, h->bnear.p, h->brow.p, h->brange.p, sums.p + 1, h->stream);
-        SF_HIP(hipGetLastError());
-        SF_HIP(hipStreamSynchronize(h->stream));
-    }
+    h->K = K;
     h->nb = nb;
-    h->built = false;  // the particle searcher buffers were reused
-    h->build_pending = false;
-    h->drop_graph();
     if ((rc = upload_scene_table(h))) return rc;
     if ((rc = views_out(h))) return rc;
     SF_HIP(hipStreamSynchronize(h->stream));

@@ -54,6 +54,7 @@ struct DevBuf {
         hipError_t e = hipMalloc((void**)&p, count * sizeof(T));
         if (e != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();  // reported here; the next launch check is not to see it
             return hip_error(e, "hipMalloc");
         }
         n = count;
@@ -130,13 +131,13 @@ void launch_gather_wprefix(const GatherArgs& a, int n, uint32_t* wpart, uint32_t
                            hipStream_t s);
 void launch_boundary_gather(const uint32_t* perm, const float4* bp_in, float4* bp_out, int nb, hipStream_t s);
 void launch_boundary_volume(const SFConst& k, float4* bpv, const uint32_t* bcs, int nb, hipStream_t s);
-// near[c] for every local cell c (Fields::bnear) and the sum of its column
-// counts in *total; then the rows of those columns' ranges (Fields::brow,
-// brange, *total entries).  total and next zero on entry.
-void launch_boundary_near(const SFConst& k, const float4* bpv, const uint32_t* bcs, uint8_t* near,
-                          unsigned long long* total, hipStream_t s);
-void launch_boundary_rows(const SFConst& k, const uint32_t* bcs, const uint8_t* near, uint32_t* row, uint2* ranges,
-                          unsigned long long* next, hipStream_t s);
+// near[c] (zero on entry) and row[c] for every local cell c (Fields::bnear,
+// brow) and the number of column ranges in *total (zero on entry); then those
+// ranges (Fields::brange, *total entries).
+void launch_boundary_near(const SFConst& k, const float4* bpv, int nb, const uint32_t* bcs, uint8_t* near,
+                          uint32_t* row, uint32_t* total, hipStream_t s);
+void launch_boundary_rows(const SFConst& k, const uint32_t* bcs, const uint8_t* near, const uint32_t* row,
+                          uint2* ranges, hipStream_t s);
 void launch_nbr_count(const SFConst& k, const float4* pm, const uint16_t* scene, const uint32_t* cs, uint32_t* cnt,
                       uint32_t* cand, int n, hipStream_t s);
 void launch_hash_boundary(const SFConst& k, const float4* bp, uint32_t* keys, int nb, hipStream_t s);

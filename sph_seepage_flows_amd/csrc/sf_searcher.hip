@@ -355,66 +355,81 @@ void launch_boundary_volume(const SFConst& k, float4* bpv, const uint32_t* bcs, 
 // boundary loops skip the others, and walk only the columns that hold any
 // (a face cell has 3 of 9; the boundary never moves, so the list is made once
 // per upload).  near[c] = 1 if any, + 2 if any of label 1, + 16 x the number
-// of such columns; *total sums those numbers.
-__global__ __launch_bounds__(kBlock) void k_boundary_near(SFConst k, const float4* __restrict__ bpv,
-                                                          const uint32_t* __restrict__ bcs,
-                                                          uint8_t* __restrict__ near,
-                                                          unsigned long long* __restrict__ total) {
+// of such columns.
+// Label 1 first, if there is any: each such particle marks the cells around
+// its own (all that mark a byte write the same).
+__global__ __launch_bounds__(kBlock) void k_boundary_mark(SFConst k, const float4* __restrict__ bpv, int nb,
+                                                          uint8_t* __restrict__ near) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= nb) return;
+    const float4 b = bpv[i];
+    if (b.w >= 0.f) return;
+    int cx, cy, cz;
+    cell_of(k, b.x, b.y, b.z, cx, cy, cz);
+    for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
+        for (uint32_t c = c0; c < c1; ++c) near[c] = 2;
+    });
+}
+// near, and row[c] = where cell c's non-empty column ranges start among those
+// of all cells, whose number is left in *total (the blocks' rows lie in the
+// order the atomics leave).  Each boundary particle is in one column range of
+// at most 27 cells, so at most 27 x 2^27 ranges: the sums fit 32 bits.
+__global__ __launch_bounds__(kBlock) void k_boundary_near(SFConst k, const uint32_t* __restrict__ bcs,
+                                                          uint8_t* __restrict__ near, uint32_t* __restrict__ row,
+                                                          uint32_t* __restrict__ total) {
+    __shared__ uint32_t sums[kBlock / 64], base;
     const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    const int lane = (int)(threadIdx.x & 63u), w = (int)(threadIdx.x >> 6);
     uint32_t cols = 0;
     if (c < k.C) {
         const int cz = (int)(c % (uint32_t)k.gz), cy = (int)((c / (uint32_t)k.gz) % (uint32_t)k.gy);
         const int cx = (int)(c / ((uint32_t)k.gz * (uint32_t)k.gy));
-        bool one = false;
-        for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
-            const uint32_t s = bcs[c0], e = bcs[c1];
-            cols += e > s ? 1u : 0u;
-            if (k.blabel1)
-                for (uint32_t j = s; j < e && !one; ++j) one = bpv[j].w < 0.f;
-        });
-        near[c] = (uint8_t)((cols ? 1u : 0u) | (one ? 2u : 0u) | (cols << 4));
+        for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) { cols += bcs[c1] > bcs[c0] ? 1u : 0u; });
+        near[c] = (uint8_t)((cols ? 1u : 0u) | (near[c] & 2u) | (cols << 4));
     }
-    uint32_t sum = cols;
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_down(sum, o, 64);
-    if ((threadIdx.x & 63u) == 0 && sum) atomicAdd(total, (unsigned long long)sum);
-}
-// row[c] = where cell c's non-empty column ranges [s, e) start in ranges, in
-// for_columns order (the rows lie in the order the atomics leave)
-__global__ __launch_bounds__(kBlock) void k_boundary_rows(SFConst k, const uint32_t* __restrict__ bcs,
-                                                          const uint8_t* __restrict__ near, uint32_t* __restrict__ row,
-                                                          uint2* __restrict__ ranges,
-                                                          unsigned long long* __restrict__ next) {
-    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
-    const int lane = (int)(threadIdx.x & 63u);
-    const uint32_t cols = c < k.C ? (uint32_t)near[c] >> 4 : 0u;
     uint32_t x = cols;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         const uint32_t y = __shfl_up(x, o, 64);
         if (lane >= o) x += y;
     }
-    unsigned long long base = 0;
-    if (lane == 63) base = atomicAdd(next, (unsigned long long)x);
-    uint32_t at = (uint32_t)__shfl(base, 63, 64) + x - cols;
+    if (lane == 63) sums[w] = x;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t all = 0;
+        for (int q = 0; q < kBlock / 64; ++q) all += sums[q];
+        base = all ? atomicAdd(total, all) : 0u;
+    }
+    __syncthreads();
     if (c >= k.C) return;
+    uint32_t at = base + x - cols;
+    for (int q = 0; q < w; ++q) at += sums[q];
     row[c] = at;
-    if (!cols) return;
+}
+// The rows themselves, in for_columns order.
+__global__ __launch_bounds__(kBlock) void k_boundary_rows(SFConst k, const uint32_t* __restrict__ bcs,
+                                                          const uint8_t* __restrict__ near,
+                                                          const uint32_t* __restrict__ row, uint2* __restrict__ ranges) {
+    const uint32_t c = blockIdx.x * kBlock + threadIdx.x;
+    if (c >= k.C || !near[c]) return;
     const int cz = (int)(c % (uint32_t)k.gz), cy = (int)((c / (uint32_t)k.gz) % (uint32_t)k.gy);
     const int cx = (int)(c / ((uint32_t)k.gz * (uint32_t)k.gy));
+    uint2* out = ranges + row[c];
     for_columns(k, cx, cy, cz, [&](uint32_t c0, uint32_t c1) {
         const uint32_t s = bcs[c0], e = bcs[c1];
-        if (e > s) ranges[at++] = make_uint2(s, e);
+        if (e > s) *out++ = make_uint2(s, e);
     });
 }
-void launch_boundary_near(const SFConst& k, const float4* bpv, const uint32_t* bcs, uint8_t* near,
-                          unsigned long long* total, hipStream_t s) {
+void launch_boundary_near(const SFConst& k, const float4* bpv, int nb, const uint32_t* bcs, uint8_t* near,
+                          uint32_t* row, uint32_t* total, hipStream_t s) {
     if (k.C == 0) return;
-    k_boundary_near<<<(k.C + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, bpv, bcs, near, total);
+    if (k.blabel1 && nb > 0) k_boundary_mark<<<(nb + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, bpv, nb, near);
+    k_boundary_near<<<(k.C + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, bcs, near, row, total);
 }
-void launch_boundary_rows(const SFConst& k, const uint32_t* bcs, const uint8_t* near, uint32_t* row, uint2* ranges,
-                          unsigned long long* next, hipStream_t s) {
+void launch_boundary_rows(const SFConst& k, const uint32_t* bcs, const uint8_t* near, const uint32_t* row,
+                          uint2* ranges, hipStream_t s) {
     if (k.C == 0) return;
-    k_boundary_rows<<<(k.C + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, bcs, near, row, ranges, next);
+    k_boundary_rows<<<(k.C + kBlock - 1) / kBlock, kBlock, 0, s>>>(k, bcs, near, row, ranges);
 }
 
 // ---------------------------------------------------------------------------

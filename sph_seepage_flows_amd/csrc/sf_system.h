@@ -23,6 +23,9 @@ struct EmitterState {
     float elapsed = 0.f;
 };
 
+// Bytes of a byte per cell, in whole words.
+inline size_t near_bytes(size_t cells) { return (cells + 3) & ~(size_t)3; }
+
 struct sf_system {
     sf_params P{};
     sf_boundary_params B{};
@@ -53,8 +56,9 @@ struct sf_system {
     bool full_empty = false;
     bool empty_pending = false;
     size_t n_built = 0;
-    DevBuf<uint8_t> bnear;            // cells with boundary particles near (Fields::bnear)
-    DevBuf<uint32_t> brow;            // their columns' ranges (Fields::brange)
+    // cells with boundary particles near (Fields::bnear) and, once there are
+    // any, where their columns' ranges start (Fields::brow), in one allocation
+    DevBuf<uint8_t> bnear;
     DevBuf<uint2> brange;
     DevBuf<float4> vq, wq, xq, wbq;   // listed particles' fields by phase index (Fields::wq)
     DevBuf<float> vws;
@@ -142,7 +146,7 @@ struct sf_system {
         f.bpv = bpv.p;
         f.bcell = bcell.p;
         f.bnear = bnear.p;
-        f.brow = brow.p;
+        f.brow = reinterpret_cast<const uint32_t*>(bnear.p + near_bytes(local_cells()));
         f.brange = brange.p;
         f.rp = rp.p;
         f.es = es.p;

@@ -1,6 +1,9 @@
 """Boundary uploads: what they hold on the device, and what an upload that
 fails leaves behind."""
 import ctypes as C
+import subprocess
+import sys
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -34,3 +37,79 @@ def test_boundary_does_not_size_the_particle_arrays():
     assert took < 64 * n
     g.step(1e-6)
     assert g.sizes()[:2] == (sc.n, n)
+
+
+SHIM = """
+#include <dlfcn.h>
+#include <stddef.h>
+static long left = -1;
+static int refused;
+void refuse_malloc(long k) { left = k; refused = 0; }
+int malloc_refused(void) { return refused; }
+int hipMalloc(void** p, size_t n) {
+    static int (*real)(void**, size_t);
+    if (!real) real = (int (*)(void**, size_t))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD), "hipMalloc");
+    if (left == 0) {
+        left = -1;
+        refused = 1;
+        *p = NULL;
+        return 2; /* hipErrorOutOfMemory */
+    }
+    if (left > 0) --left;
+    return real(p, n);
+}
+"""
+CHILD = """
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before the library: its hipMalloc is this one
+shim.refuse_malloc.argtypes = [ctypes.c_long]
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from sph_seepage_flows_amd import SFError, SFSystem, scenes
+sc = scenes.mixed()
+a, b = SFSystem.from_scene(sc), SFSystem.from_scene(sc)
+names = ("pos", "vel", "acc", "density", "col", "sort_perm", "b_pos", "b_volume", "b_label", "b_cell_start")
+def same(n):
+    a.step(1e-4, n)
+    b.step(1e-4, n)
+    for name in names:
+        np.testing.assert_array_equal(a.get(name), b.get(name), err_msg=name)
+same(3)
+copies = lambda n, d: (np.concatenate([sc.bpos + np.float32(d * q) for q in range(n)]), np.tile(sc.blabel, n))
+# no more than the handle's particles; more than the sort has room for; as many again
+for other, label in (copies(1, 0.003), copies(5, 0.002), copies(5, 0.0015)):
+    failed = 0
+    while True:
+        shim.refuse_malloc(failed)
+        try:
+            a.upload_boundary(other, label)
+        except SFError:
+            assert shim.malloc_refused() == 1
+        else:
+            break
+        failed += 1
+        assert a.sizes() == b.sizes()
+        same(2)
+    assert shim.malloc_refused() == 0
+    shim.refuse_malloc(-1)
+    b.upload_boundary(other, label)
+    same(2)
+    print(len(other), "boundary particles, failed uploads", failed)
+"""
+
+
+def test_failed_upload_leaves_the_old_boundary(tmp_path):
+    """Each allocation of an upload in turn reports that there is no memory (a
+    hipMalloc in front of the runtime's, in a process of its own): the handle
+    steps on with its old boundary, bit for bit like one that was never asked."""
+    src, lib_ = tmp_path / "shim.c", tmp_path / "shim.so"
+    src.write_text(SHIM)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", str(src), "-o", str(lib_), "-ldl"], check=True)
+    root = str(Path(__file__).resolve().parents[1])
+    r = subprocess.run([sys.executable, "-c", CHILD, str(lib_), root], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    print(r.stdout, flush=True)
+    counts = [int(line.split()[-1]) for line in r.stdout.splitlines()]
+    # the state and the cells' bytes; the six arrays of the sort; those two, the
+    # particles as given and, of the larger boundary's, the ranges
+    assert len(counts) == 3 and counts[0] >= 2 and counts[1] >= 6 and counts[2] >= 3
