@@ -432,13 +432,14 @@ SF_DEV void list_interface(const Fields& f, bool listed, bool sand, uint32_t t, 
 // one column's range ahead).
 template <int L, class Fn>
 SF_DEV void boundary_walk(const Fields& f, uint32_t near, uint32_t cell, uint32_t sub, Fn&& fn) {
-    const uint32_t n = near >> 4, row = ldo(f.brow, cell);
+    const uint32_t n = near >> 4;
+    const uint2* __restrict__ ranges = f.brange + ldo(f.brow, cell);  // above 2^29 of them too
     for (uint32_t q = 0; q < n; q += 3u) {
         uint2 r[3];
         float4 b[3][3];
 #pragma unroll
         for (uint32_t m = 0; m < 3u; ++m) {
-            r[m] = q + m < n ? ldo(f.brange, row + q + m) : make_uint2(0u, 0u);
+            r[m] = q + m < n ? ldo(ranges, q + m) : make_uint2(0u, 0u);
             r[m].x += sub;
         }
 #pragma unroll
@@ -554,11 +555,12 @@ __global__ __launch_bounds__(NB) void k_density(SFConst k, Fields f, int n) {
         // the columns that hold any, one after another (this pass keeps its
         // registers low), the next one's range and four candidates' loads in
         // flight at a time, summed in increasing j
-        const uint32_t n = near >> 4, row = ldo(f.brow, cell);
-        uint2 next = ldo(f.brange, row);
+        const uint32_t n = near >> 4;
+        const uint2* __restrict__ ranges = f.brange + ldo(f.brow, cell);
+        uint2 next = ldo(ranges, 0u);
         for (uint32_t q = 0; q < n; ++q) {
             const uint2 r = next;
-            next = ldo(f.brange, row + (q + 1u < n ? q + 1u : q));
+            next = ldo(ranges, q + 1u < n ? q + 1u : q);
             uint32_t j = r.x + sub;
             for (; j + 3u * kDenL < r.y; j += 4u * kDenL) {
                 const float4 b0 = ldo(f.bpv, j), b1 = ldo(f.bpv, j + kDenL), b2 = ldo(f.bpv, j + 2u * kDenL),

@@ -8,9 +8,10 @@ from pathlib import Path
 import numpy as np
 import pytest
 
-from sph_seepage_flows_amd import SFSystem, scenes
+from sph_seepage_flows_amd import Physics, SFSystem, scenes
 
 from _hip import runtime
+from _scene_util import make_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -37,6 +38,41 @@ def test_boundary_does_not_size_the_particle_arrays():
     assert took < 64 * n
     g.step(1e-6)
     assert g.sizes()[:2] == (sc.n, n)
+
+
+def test_more_than_2_29_column_ranges():
+    """Boundary particles three cells apart along z in every column of a 400^3
+    grid: each cell has nine columns that hold one, 5.7e8 ranges in all, past
+    what a 32-bit byte offset reaches.  (Along x they come in pairs 5/8 h apart,
+    which gives them their volumes.)  A water particle near the even one of a
+    pair has the same density and acceleration in every interior cell, those of
+    the same surroundings in a grid of 12^3: all positions are multiples of
+    2^-10, so the differences, and with them every sum, are the same bits."""
+    r = 0.0625
+    h = 4 * r
+    off = np.float32([0.05078125, 0.03125, 0.015625])
+
+    def handle(cells, at):
+        ph = Physics(hi=(cells * h,) * 3, r_water=r, r_sand=r)
+        pos = ((np.float32(at) + np.float32(0.5)) * np.float32(h) + off).astype(np.float32)
+        g = SFSystem.from_scene(make_scene(pos, np.zeros(len(pos), np.uint64), ph=ph))
+        c = (np.arange(cells, dtype=np.float32) + np.float32(0.5)) * np.float32(h)
+        z = c[1::3]
+        b = np.empty((cells, cells, len(z), 3), np.float32)
+        x = c - np.where(np.arange(cells) % 2 == 1, np.float32(0.09375), np.float32(0.0))
+        b[..., 0], b[..., 1], b[..., 2] = x[:, None, None], c[None, :, None], z
+        g.upload_boundary(b.reshape(-1, 3))
+        g.step(1e-6)
+        return g
+
+    small = handle(12, [(6, 6, 4)])
+    ref = {k: small.get(k)[0] for k in ("density", "pressure", "acc")}
+    assert 1e3 < ref["density"] < 1e5 and np.isfinite(ref["acc"]).all()
+    at = [(6, 6, 4), (100, 50, 199), (250, 300, 100), (374, 10, 394), (386, 200, 10), (394, 390, 304)]
+    big = handle(400, at)
+    print(f"{big.sizes()} density {ref['density']}", flush=True)
+    for k, v in ref.items():
+        np.testing.assert_array_equal(big.get(k), np.broadcast_to(v, (len(at),) + v.shape), err_msg=k)
 
 
 SHIM = """
