@@ -481,8 +481,9 @@ int sf_get_launch_config(sf_handle h, int pass, int* nb, int* cap);
 int sf_set_interface_lanes(sf_handle h, int lanes);
 /* Times every shape of every neighbour pass on the handle's current particles
  * (reps launches each, after one neighbour build) and keeps the fastest.
- * best_ms / default_ms (5 floats each, may be NULL) receive per pass the
- * chosen and the default (256, 16) shape's mean time. */
+ * best_ms / default_ms (5 floats each, may be NULL) receive per pass the mean
+ * time of the chosen shape and of the one launched while none is set.  The
+ * fields are left as one build and solve leave them. */
 int sf_autotune(sf_handle h, int reps, float* best_ms, float* default_ms);
 
 /* ---- differentiable window ----------------------------------------------

@@ -1559,12 +1559,14 @@ int sf_autotune(sf_handle h, int reps, float* best_ms, float* default_ms) {
     if (reps < 1 || reps > 1000) return set_error(SF_E_INVALID, "reps must be in [1, 1000]");
     // A neighbour build reorders the particles exactly as the next step's
     // first pass would; every neighbour pass is then idempotent (it rewrites
-    // the same outputs from unchanged inputs), so each is timed in place, in
-    // dependency order, without disturbing the trajectory.
+    // the same outputs from inputs that neither it nor a later pass changes),
+    // so each is timed in place, in dependency order, without disturbing the
+    // trajectory or the fields of the solve.
     if ((rc = build_neighbors(h))) return rc;
     if ((rc = solve(h))) return rc;
     for (int q = 0; q < 5; ++q) {
         const bool lists = q >= 3;
+        const int unset = q == 3 ? sand_momentum_nb((int)h->n) : q == 4 ? water_momentum_nb((int)h->n) : 256;
         float best = 0.f, dflt = 0.f;
         PassCfg pick{256, 16, h->cfg[q].lanes, true};
         for (int nb : kNbChoices)
@@ -1580,7 +1582,7 @@ int sf_autotune(sf_handle h, int reps, float* best_ms, float* default_ms) {
                 float ms = 0.f;
                 SF_HIP(hipEventElapsedTime(&ms, h->ev0, h->ev1));
                 ms /= (float)reps;
-                if (nb == 256 && cap == 16) dflt = ms;
+                if (nb == unset && cap == 16) dflt = ms;
                 if (best == 0.f || ms < best) {
                     best = ms;
                     pick = c;

@@ -324,6 +324,10 @@ void launch_interface(const SFConst& k, const Fields& f, int n, hipStream_t s);
 // last neighbour build.
 void launch_fill_empty(const SFConst& k, const Fields& f, int n, hipStream_t s);
 void launch_voidage_adhesion(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s);
+// The workgroup size the two momentum passes launch for n particles while their
+// shape is unset.
+int sand_momentum_nb(int n);
+int water_momentum_nb(int n);
 void launch_sand_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s);
 void launch_water_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s);
 // CFL reduction: partial maxima of |acc| -> finalize writes CflOut

@@ -1142,12 +1142,13 @@ __global__ __launch_bounds__(NB) void k_sand_momentum(SFConst k, Fields f, int n
         f.cs[i] = c;
     }
 }
+// one wave per workgroup: no wave's LDS and slot wait for the slowest of four
+// (15.1 -> 13.6 us at 24k, 71 -> 69 at 1M apart, 158 -> 150 interpenetrating,
+// 255 -> 255 at 4M)
+int sand_momentum_nb(int) { return 64; }
 void launch_sand_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
     if (n <= 0) return;
-    // one wave per workgroup unless the shape was set: no wave's LDS and slot
-    // wait for the slowest of four (15.1 -> 13.6 us at 24k, 71 -> 69 at 1M
-    // apart, 158 -> 150 interpenetrating, 255 -> 255 at 4M)
-    if (!c.chosen) c.nb = 64;
+    if (!c.chosen) c.nb = sand_momentum_nb(n);
     dispatch(f, c, [&](auto B, auto NB, auto CAP) {
         k_sand_momentum<decltype(B)::value, decltype(NB)::value, decltype(CAP)::value>
             <<<phase_grid(n * kSmL, NB), (int)NB, 0, s>>>(k, f, n);
@@ -1347,14 +1348,17 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     const v3 acc = mk3(k.gvx, k.gvy, k.gvz) + a - ad * (1.f / mi);
     f.acc[i] = f4(acc, 0.f);
 }
+// one wave per workgroup, as in the sand momentum pass, up to kWmOneWave
+// particles (24.7 -> 20.4 us at 24k, 134.5 -> 128 at 1M, 169 -> 168 at
+// 2M); above, neighbouring waves on one CU share more of its L1 than they
+// wait for each other (4M: 335 us with 256 threads, 354 with 64)
+int water_momentum_nb(int n) {
+    constexpr int kWmOneWave = 2 << 20;
+    return n <= kWmOneWave ? 64 : 256;
+}
 void launch_water_momentum(const SFConst& k, const Fields& f, int n, PassCfg c, hipStream_t s) {
     if (n <= 0) return;
-    // one wave per workgroup, as in the sand momentum pass, up to kWmOneWave
-    // particles (24.7 -> 20.4 us at 24k, 134.5 -> 128 at 1M, 169 -> 168 at
-    // 2M); above, neighbouring waves on one CU share more of its L1 than they
-    // wait for each other (4M: 335 us with 256 threads, 354 with 64)
-    constexpr int kWmOneWave = 2 << 20;
-    if (!c.chosen && n <= kWmOneWave) c.nb = 64;
+    if (!c.chosen) c.nb = water_momentum_nb(n);
     dispatch(f, c, [&](auto B, auto NB, auto CAP) {
         constexpr bool b = decltype(B)::value;
         constexpr int nb = decltype(NB)::value, cap = decltype(CAP)::value;

@@ -35,3 +35,19 @@ def test_fields_after_autotune_are_the_solve_s(kind):
     assert np.abs(b.get("avg_adhesion_force")).max() > 0 and np.abs(b.get("avg_drag_force")).max() > 0
     for name in FIELDS:
         np.testing.assert_array_equal(a.get(name), b.get(name), err_msg=f"{kind} {name}")
+
+
+@pytest.mark.parametrize("scene", ["block", "mixed"])
+def test_default_is_the_shape_an_untuned_handle_launches(scene):
+    """A pass that keeps the shape it launches anyway (64 threads in the momentum
+    passes at these sizes, 256 in the others) gains nothing: the two times are
+    one measurement."""
+    g = SFSystem.from_scene(scenes.small_block() if scene == "block" else scenes.mixed())
+    kept = 0
+    for _ in range(4):
+        for name, (nb, cap, best, dflt) in g.autotune(reps=20).items():
+            assert 0 < best <= dflt
+            if (nb, cap) == (64 if name.endswith("momentum") else 256, 16):
+                assert best == dflt, name
+                kept += 1
+    print(f"{kept} of 20 kept their shape", flush=True)
