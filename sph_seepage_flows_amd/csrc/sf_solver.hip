@@ -1278,12 +1278,11 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
     };
     auto water_range = [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, true, nw); };
     auto sand_range = [&](uint32_t b, uint32_t c0, uint32_t c1) { return phase_range(f.ct + b, c0, c1, false, nw); };
-    const bool listed = active && ldo(f.wl, t);  // grains in its 27 cells
     if constexpr (Nbr::fresh) {
         column_filter<kWmL, kStageWm>(k, f.rec0, stage, active, cb, cx, cy, cz, L, water_range, in_range, fetch, water);
         nl_flush2(L, fetch, water);
         bool over = false;
-        if (listed) {
+        if (active && ldo(f.wl, t)) {  // listed: grains in its 27 cells
             const uint32_t G = saved_lane((uint32_t)f.nl_lanes, false, nw, ldo(f.nlq, t));
             over = ldo(f.nlc, G) == kSavedOver;
             if (!over) saved_pairs<kWmL>(f, (uint32_t)f.nl_lanes, G, sub, L, fetch_sand, sand);
@@ -1314,6 +1313,7 @@ __global__ __launch_bounds__(NB) void k_water_momentum(SFConst k, Fields f, int 
         };
         column_filter<kWmL, kStageWm>(k, f.rec0, stage, active, cb, cx, cy, cz, L, water_range, in_range, fetch, was_water);
         nl_flush2(L, fetch, was_water);
+        const bool listed = active && ldo(f.wl, t);
         column_filter<kWmL, kStageWm>(k, f.rec0, stage, listed, cb, cx, cy, cz, L, sand_range, in_range, fetch_sand,
                                       was_sand);
         nl_flush2(L, fetch_sand, was_sand);
