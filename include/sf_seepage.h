@@ -456,14 +456,16 @@ int sf_step_graph(sf_handle h, float dt, int n_steps);
 #define SF_SORT_RADIX 0
 #define SF_SORT_INCREMENTAL 1
 int sf_set_sort_strategy(sf_handle h, int strategy);
-/* Largest number of 2048-slot tiles up to which the slot prefixes of the
- * incremental sort and of the water prefix sum the earlier tiles' counts
- * inside each prefix block; above it a one-block scan launch runs in between
- * (default 4096 tiles, about 8.4M slots).  Both branches give the same
- * prefixes; the switch lets a test run both on one input.  Process-wide (no
- * handle); graphs captured before keep the branch they were captured with.
- * tiles < 0 restores the default.  Returns the previous threshold.  No
- * counterpart in the reference. */
+/* Largest number of 2048-entry tiles up to which two prefixes sum the earlier
+ * tiles' counts inside each of their blocks: the water prefix over the slots
+ * after a radix sort, and the incremental sort's newcomer counts over the
+ * cells.  Above it a one-block scan launch runs in between (default 4096
+ * tiles, about 8.4M slots or cells).  Both branches give the same prefixes;
+ * the switch lets a test run both on one input.  (The incremental sort's
+ * prefix over slots goes by block totals, whatever the threshold.)
+ * Process-wide (no handle); graphs captured before keep the branch they were
+ * captured with.  tiles < 0 restores the default.  Returns the previous
+ * threshold.  No counterpart in the reference. */
 int sf_set_prefix_scan_threshold(int tiles);
 /* Launch shape of a neighbour pass (SF_PASS_DENSITY .. SF_PASS_WATER_MOMENTUM):
  * workgroup size nb in {64, 128, 256}; LDS candidate-list depth cap in {8, 16}

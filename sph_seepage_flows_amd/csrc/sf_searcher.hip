@@ -147,14 +147,9 @@ SF_DEV void scan_range(U* __restrict__ hist, int total, U* __restrict__ total_ou
     if (total_out && t == 0) *total_out = carry_s;
     __syncthreads();
 }
-__global__ __launch_bounds__(1024) void k_rs_scan(uint32_t* __restrict__ hist, int total) {
-    scan_range<uint32_t>(hist, total, nullptr);
-}
-// two independent scans, [0, n1) and [n1, n1 + n2), in one launch
 template <class U>
-__global__ __launch_bounds__(1024) void k_rs_scan2(U* __restrict__ part, int n1, int n2, U* __restrict__ total_out) {
-    scan_range<U>(part, n1, total_out);
-    scan_range<U>(part + n1, n2, nullptr);
+__global__ __launch_bounds__(1024) void k_rs_scan(U* __restrict__ hist, int total, U* __restrict__ total_out) {
+    scan_range<U>(hist, total, total_out);
 }
 
 // stable scatter: each wave ranks a contiguous chunk of 64*kRsItems keys
@@ -222,7 +217,7 @@ int radix_sort(const uint32_t* keys, int n, const RadixPlan& plan, const SortBuf
     for (int p = 0; p < plan.passes; ++p) {
         k_rs_upsweep<<<nblocks, kRsThreads, 0, s>>>(kin, n, plan.shift[p], plan.bits[p], b.hist);
         const int total = nblocks << plan.bits[p];
-        k_rs_scan<<<1, 1024, 0, s>>>(b.hist, total);
+        k_rs_scan<uint32_t><<<1, 1024, 0, s>>>(b.hist, total, nullptr);
         k_rs_downsweep<<<nblocks, kRsThreads, 0, s>>>(kin, vin, ko, vo, n, plan.shift[p], plan.bits[p], b.hist);
         *sorted_keys = ko;
         *perm = vo;
@@ -608,7 +603,7 @@ void launch_gather_wprefix(const GatherArgs& a, int n, uint32_t* wpart, uint32_t
     const int nb = wprefix_blocks(n + 1);
     k_gather<<<nb, kBlock, 0, s>>>(a, n, wpart);
     const int scanned = nb > g_direct_tiles ? 1 : 0;
-    if (scanned) k_rs_scan2<uint32_t><<<1, 1024, 0, s>>>(wpart, nb, 0, wpart + nb);
+    if (scanned) k_rs_scan<uint32_t><<<1, 1024, 0, s>>>(wpart, nb, wpart + nb);
     k_wprefix_plist<<<nb, kBlock, 0, s>>>(a.wflag, n, wpart, scanned, wpre, plist);
 }
 
@@ -710,7 +705,7 @@ void launch_incremental_sort(const PlaceArgs& a, const Newcomers& nc, int n, uin
     if (!flags_done) k_inc_flag<<<gn, kBlock, 0, s>>>(a.key, a.old_key, a.g.wflag, n, nc);
     const int nb1 = wprefix_blocks(gn + 1), nb2 = (int)a.parts;
     const int scanned = nb2 > g_direct_tiles ? 1 : 0;
-    if (scanned) k_rs_scan2<uint64_t><<<1, 1024, 0, s>>>(a.part, nb2, 0, nullptr);
+    if (scanned) k_rs_scan<uint64_t><<<1, 1024, 0, s>>>(a.part, nb2, nullptr);
     k_inc_prefix<<<nb1 + nb2, kBlock, 0, s>>>(nc.totals, gn, nb1, a.stay_base, a.in_count, (int)C, a.in_start, a.part,
                                               scanned);
     k_inc_place<<<gn + (int)((C + 1 + kBlock - 1) / kBlock), kBlock, 0, s>>>(a, n, C, gn);
