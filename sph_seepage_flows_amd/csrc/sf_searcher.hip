@@ -621,6 +621,13 @@ void launch_gather_wprefix(const GatherArgs& a, int n, uint32_t* wpart, uint32_t
 // newStart(c) = stayers in cells < c + newcomers in cells < c.
 // The result is the stable sort's, element for element.
 //
+// A chain is dependent loads, walked by every particle of its cell: some 0.27
+// us per newcomer of the fullest cell.  With every particle of 500k + 500k
+// moving by about a cell the build takes 149 us (163 with contiguous lists,
+// filled by a launch of their own); only where hundreds enter one cell at
+// once does the chain lose to them (500 of 101k: 193 against 111 us, the
+// solve of such a pile 300; 3000: 820 against 370, solve 1160).
+//
 // Every count carries the water's share in its upper half, so the same sums
 // give the number of water particles before a slot, that is the particle's
 // index within its phase, and the placement reorders everything at once:

@@ -215,14 +215,16 @@ SF_DEV void staged_walk(const SFConst& k, const Fields& f, float4* __restrict__ 
 // lane's list gets the same entries in the same order, so which way a column
 // goes does not change the sums.  Must be called by all lanes of the wave.
 // P2, P3 and P4's water walk stage the other phase's candidates (P2 216 ->
-// 200 us, P3 216 -> 203, P4 176 -> 155 at 500k + 500k interpenetrating; where
-// little is listed, the stage's LDS leaves fewer of the waves that find
+// 200 us, P3 216 -> 203, P4 176 -> 155 at 500k + 500k interpenetrating, all
+// with 256-thread workgroups and before P3 and P4 read P2's saved neighbours;
+// where little is listed, the stage's LDS leaves fewer of the waves that find
 // nothing resident: 2 x 4 us of 1.12 ms at 4M).
 constexpr uint32_t kStageList = 64;  // longest union range staged per wave: P2, P3, P4's water
 // P5's candidates are both phases': 16 water particles span 2-3 cells, so the
 // union is 4-5 cells of 8 water particles, or of 16 particles where the
-// phases interpenetrate (64-80).  96 instead of 64: P5 255 -> 227 us at 500k +
-// 500k interpenetrating, 137 -> 138 us where they are apart.
+// phases interpenetrate (64-80).  96 instead of 64, with 256-thread workgroups:
+// P5 255 -> 227 us at 500k + 500k interpenetrating, 137 -> 138 us where they
+// are apart.
 constexpr uint32_t kStageWm = 96;
 #define SF_STAGE(name, KS)                              \
     __shared__ float4 name##_lds[(NB / 64) * (KS)];     \
